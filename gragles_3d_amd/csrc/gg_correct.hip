@@ -20,17 +20,17 @@
 //   k_tri_scatter  every triangle record of the hull goes to its element's
 //                  range (the order inside an element does not matter: all its
 //                  barycenters carry the element's weights).
+//   k_slots        one workgroup per grain: per slot of the grain's hull-id table,
+//                  the barycenters that can be nearest to some voxel of the new
+//                  output box, as rows of the search's matrix product.
 // After each convolution:
-//   k_correct      one workgroup per (grain, z-layer) of the output box: the
-//                  band voxels (|phi_in| < delta) are queued with the slot of
+//   k_correct      one workgroup per (grain, run of z-layers) of the output box:
+//                  the band voxels (|phi_in| < delta) are queued with the slot of
 //                  their IDLocal id in the grain's hull-id table and grouped by
-//                  slot (counting sort in LDS), so a wavefront's 64 voxels
-//                  mostly border the same grain; each lane takes one, walks
-//                  the grain's elements in projection order (wave-uniform
-//                  loop that skips the elements no lane needs; the
-//                  barycenters are read with wave-uniform loads, four per
-//                  round) and keeps the first nearest barycenter (squared
-//                  distance, strict '<') among the elements that border its
+//                  slot (counting sort in LDS); a wavefront takes up to 128 of
+//                  one slot and finds, for each, the element of the first nearest
+//                  barycenter in projection order (squared distance, strict '<')
+//                  among the elements that border its
 //                  id; then phi_out = phi_in +
 //                  (phi_out - phi_in) * w_energy * w_mobility and, with stored
 //                  energies on, minus (SEE_self - SEE_id) * w_mobility * dt /
@@ -50,9 +50,7 @@ constexpr int kEW = 256;                           // threads of an element-buil
 constexpr int kRec = kJuncCap + kJuncCap / 2;      // lists + high-order junctions made by merging
 constexpr int kTopoCapBitsC = 6;
 static_assert((1 << kTopoCapBitsC) == kTopoCap, "grain topology table size");
-constexpr int kCorrGridPerCU = 512;  // workgroups per CU of a correction launch (512 against 128: stored-energy step 202.0 -> 199.5 ms, timed on one box)
-constexpr int kCellBits = 14;                      // a layer cell index (n^2 <= 9216) in a queue entry
-static_assert(kMaxN * kMaxN < (1 << kCellBits), "queue entry layout");
+constexpr int kCorrGridPerCU = 512;  // workgroups per CU of a correction launch: about one per tile
 
 enum { kClsGB = 0, kClsTL = 1, kClsQJ = 2, kClsHJ = 3 };
 
@@ -97,8 +95,6 @@ __global__ __launch_bounds__(kEW) void k_elements(SimParams sp, const int32_t* _
   __shared__ short s_elem[kRec];  // element index of a record that is an element
   __shared__ short s_hj[kRec], s_qj[kJuncCap];
   __shared__ short s_ord[kJuncCap];  // element -> record
-  __shared__ int s_efp[kJuncCap + 1];  // first barycenter of each element (whole chunks)
-  __shared__ int64_t s_tb;
   const int N = sp.N;
   const int tid = threadIdx.x;
   if (blockIdx.x == 0 && tid == 0) *cd.ready = 1;
@@ -265,15 +261,12 @@ __global__ __launch_bounds__(kEW) void k_elements(SimParams sp, const int32_t* _
       for (int e = 0; e < E; ++e) {
         s_elem[s_ord[e]] = (short)e;
         ef[e] = (int32_t)acc;
-        s_efp[e] = (int32_t)acc;
-        acc += (s_cnt[s_ord[e]] + kChunk - 1) / kChunk * kChunk;  // whole chunks
+        acc += s_cnt[s_ord[e]];
       }
       ef[E] = (int32_t)acc;
-      s_efp[E] = (int32_t)acc;
       const unsigned long long tb = atomicAdd(cd.tri_n, (unsigned long long)acc);
       if (tb + (unsigned long long)acc > (unsigned long long)cd.tri_cap) atomicOr(err, kErrTri);
       cd.tbase[g] = (int64_t)tb;
-      s_tb = (int64_t)tb;
       cd.ecount[g] = E;
       cd.eclass[4 * g] = nh;
       cd.eclass[4 * g + 1] = nq;
@@ -300,30 +293,20 @@ __global__ __launch_bounds__(kEW) void k_elements(SimParams sp, const int32_t* _
       while (s_red[rec] >= 0) rec = s_red[rec];
       cd.slot_elem[jb + s_ls[s_sorted[r]]] = s_elem[rec];
     }
-    // the padding points that complete each element's last chunk
-    for (int e = tid; e < E; e += kEW) {
-      const int64_t a = s_tb + s_efp[e] + s_cnt[s_ord[e]], b = s_tb + s_efp[e + 1];
-      for (int64_t q = a; q < b && q < cd.tri_cap; ++q) {
-        cd.tri[3 * q] = kFarPoint;
-        cd.tri[3 * q + 1] = kFarPoint;
-        cd.tri[3 * q + 2] = kFarPoint;
-      }
-    }
     __syncthreads();  // the LDS tables are refilled for the next grain
   }
 }
 
-// The barycenter pool's fill counter (a kernel, so that a captured step graph
+// The pools' fill counters (a kernel, so that a captured step graph
 // holds no memset node).
-__global__ void k_clear_counter(unsigned long long* c) {
-  if (threadIdx.x == 0) *c = 0ull;
+__global__ void k_clear_counters(unsigned long long* tri_n, int* row_n) {
+  if (threadIdx.x == 0) *tri_n = 0ull;
+  if (threadIdx.x == 1) *row_n = 0;
 }
 
 // Every triangle record of the last hull into its element's barycenter range.
 // The records of one hull tile are consecutive in the pool and in cell order;
-// a wavefront reserves one run per (grain, element) among its 64 records, so
-// an element's range is made of such runs in the hull's order and consecutive
-// barycenters lie close together (which keeps the chunk boxes small).
+// a wavefront reserves one run per (grain, element) among its 64 records.
 __global__ __launch_bounds__(256) void k_tri_scatter(TopoDev topo, CorrDev cd) {
   unsigned long long n = *topo.raw_n;
   if (n > (unsigned long long)topo.raw_cap) n = (unsigned long long)topo.raw_cap;
@@ -368,231 +351,598 @@ __global__ __launch_bounds__(256) void k_tri_scatter(TopoDev topo, CorrDev cd) {
   }
 }
 
-// Bounding box of every chunk of kChunk barycenters (padding points left
-// out), widened by 1e-3 voxel so the FP32 box holds its FP64 points.
-__global__ __launch_bounds__(256) void k_chunk_boxes(CorrDev cd) {
-  unsigned long long nt = *cd.tri_n;
-  if (nt > (unsigned long long)cd.tri_cap) nt = (unsigned long long)cd.tri_cap;
-  const int64_t nc = (int64_t)(nt / kChunk);
-  for (int64_t c = blockIdx.x * 256ll + threadIdx.x; c < nc; c += (int64_t)gridDim.x * 256ll) {
-    float lo[3] = {3e38f, 3e38f, 3e38f}, hi[3] = {-3e38f, -3e38f, -3e38f};
-    const double* q = cd.tri + 3 * c * kChunk;
-    for (int j = 0; j < kChunk; ++j) {
-      if (q[3 * j] >= 0.5 * kFarPoint) continue;
+// Nearest element of a band voxel p among the elements that border its id, as a
+// filter on the matrix cores with an FP64 decision.
+//
+// With q' = q - org, p' = p - (org.y, org.x, org.z) and D = org - (org.y,
+// org.x, org.z) (the point's row and column stand for x and y, as in the
+// reference), |q - p|^2 is W = R - 2 p'.q' plus terms that do not depend on q,
+// where R = |q'|^2 + 2 q'.D.  W of 32 barycenters against 32 voxels is one
+// v_mfma_f32_32x32x16_bf16: p' is a small integer (exact in BF16) and -2q' and
+// R are three BF16 pieces each (store_row), so a product of a piece and p' is
+// exact and the filter's error is the FP32 accumulation's.  The filter keeps,
+// per voxel, the smallest W, its element, and the smallest W of any other
+// element.  Where the two are closer than the error bound, and only there, the
+// wavefront searches the bordering elements' barycenters in FP64 for the first
+// nearest one in projection order, so the chosen element is always the
+// reference's (about 1.5 % of the searches of 64 voxels hold such a voxel).
+//
+// Bound: with rho >= |q'| over the grain's rows, the terms of W sum to at most
+// S = rho^2 + 2 rho (|D| + |p'|) in magnitude; 12 terms are added, each
+// addition rounds to at most 2^-24 S, and the pieces' remainders are 2^-26 of a
+// term, so 16 x 2^-24 S covers the error (measured on random rows and columns
+// of every box size: at most 2.2 x 2^-24 S).
+//
+// What bounds it: at 20000 grains (5.8e8 band voxels per step) the searches hold
+// 14 groups of 8 rows on average (75 before k_slots leaves out the ones that
+// cannot be nearest), and k_correct takes 24.5 ms per step and k_slots 5.0,
+// against 146 and, for chunk boxes, 3.4 of the FP64 search over boxed chunks
+// that it replaced; queueing and output are about 9 ms of it, the rest is the
+// minima (vector) behind the products, at four wavefronts per SIMD (128
+// registers; three: 28.9 ms).  128 voxels per search read each row once for
+// four products; 64 took 4 % longer.
+typedef __bf16 v8bf __attribute__((ext_vector_type(8)));
+typedef float v16f __attribute__((ext_vector_type(16)));
+constexpr float kFilterEps = 1.0f / 1048576.0f;  // 2^-20
+constexpr float kNone = 3e38f;                   // above every filter value
+constexpr int kManyExact = 12;  // voxels of 64 to decide from which on each lane searches for its own
+constexpr int kTake = 128;  // voxels of a wavefront's search: each row is read once for four products
+
+// A barycenter as a row of the filter: -2q' (three BF16 pieces per axis) and R
+// (three pieces), 16 values with 4 spare; the columns repeat p' and 1 to match.
+// Each piece is the nearest BF16 of what the pieces before it leave, so three
+// of them hold 24 bits.
+__device__ inline void store_row(uint16_t* __restrict__ row, double qx, double qy, double qz, double r) {
+  const double v[4] = {-2.0 * qx, -2.0 * qy, -2.0 * qz, r};
+  alignas(16) uint16_t w[kRowLen] = {};
 #pragma unroll
-      for (int a = 0; a < 3; ++a) {
-        const float v = (float)q[3 * j + a];
-        lo[a] = fminf(lo[a], v - 1e-3f);
-        hi[a] = fmaxf(hi[a], v + 1e-3f);
+  for (int a = 0; a < 4; ++a) {
+    double rest = v[a];
+#pragma unroll
+    for (int k = 0; k < 3; ++k) {
+      const __bf16 piece = (__bf16)(float)rest;
+      rest -= (double)(float)piece;
+      w[3 * a + k] = __builtin_bit_cast(uint16_t, piece);
+    }
+  }
+  const uint4* s = (const uint4*)w;
+  ((uint4*)row)[0] = s[0];
+  ((uint4*)row)[1] = s[1];
+}
+
+// The filter's rows of every alive grain: per hull-id slot, element by element,
+// the barycenters that can be nearest to some voxel of the grain's output box
+// (the box the next convolution corrects).  Against the slot's nearest one to
+// the box centre, q0, a barycenter q is left out when W(q) - W(q0) =
+// R - R0 - 2 p'.(q' - q0') is positive for every p' of the box, |p'_a| <= half:
+// because the point's row and column are swapped, most grains see their
+// barycenters from far off the domain's diagonal plane x = y, and few remain.
+// One workgroup per grain, one wavefront per slot.
+__global__ __launch_bounds__(256) void k_slots(SimParams sp, const int32_t* __restrict__ state, DescDev dout,
+                                               TopoDev topo, CorrDev cd) {
+  __shared__ int s_key[kTopoCap];
+  __shared__ unsigned long long s_em[kElemCap];
+  __shared__ int s_ef[kElemCap + 1];
+  __shared__ int s_rho;
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int wv = __builtin_amdgcn_readfirstlane(tid >> 6);
+  for (int g = 1 + blockIdx.x; g <= sp.N; g += gridDim.x) {
+    if (state[g] != kAlive) continue;
+    const int64_t tb = cd.tbase[g];
+    int E = cd.ecount[g];
+    if (tb + cd.efirst[(int64_t)g * (kElemCap + 1) + E] > cd.tri_cap) E = 0;  // (the device error is set)
+    for (int i = tid; i < kTopoCap; i += 256) s_key[i] = topo.key[(int64_t)g * kTopoCap + i];
+    for (int e = tid; e < E; e += 256) s_em[e] = cd.emask[(int64_t)g * kElemCap + e];
+    for (int e = tid; e <= E; e += 256) s_ef[e] = cd.efirst[(int64_t)g * (kElemCap + 1) + e];
+    if (tid == 0) s_rho = 0;
+    __syncthreads();
+    const int32_t* b = dout.bounds + 6 * g;
+    const int n = b[3] - b[0];
+    const int ox = b[0] + n / 2, oy = b[1] + n / 2, oz = b[2] + n / 2;
+    const double dd2 = 2.0 * (double)(ox - oy), half2 = 2.0 * (double)(n / 2);
+    const double* __restrict__ tri = cd.tri + 3 * tb;
+    float rho2 = 0.f;
+    for (int slot = wv; slot < kTopoCap; slot += 4) {
+      int2* out = cd.slist + (int64_t)g * kTopoCap + slot;
+      if (s_key[slot] == -1 || s_key[slot] == g) {
+        if (lane == 0) *out = make_int2(0, 0);
+        continue;
       }
-    }
-    float* bx = cd.cbox + 6 * c;
+      // f(e, r, valid): barycenter r (relative to the grain's first) of
+      // element e, 64 per call; after(e): past the element's last call
+      auto over = [&](auto f, auto after) {
+        for (int e0 = 0; e0 < E; e0 += 64) {
+          const int el = e0 + lane;
+          unsigned long long m = __ballot(el < E && ((s_em[el < E ? el : 0] >> slot) & 1ull));
+          for (; m; m &= m - 1) {
+            const int e = e0 + (int)__builtin_ctzll(m);
+            const int r0 = s_ef[e], r1 = s_ef[e + 1];
+            for (int r = r0; r < r1; r += 64) f(e, r + lane, r + lane < r1);
+            after(e);
+          }
+        }
+      };
+      auto load = [&](int r, double& qx, double& qy, double& qz) {
+        const double* q = tri + 3 * (int64_t)r;
+        qx = q[0] - ox;
+        qy = q[1] - oy;
+        qz = q[2] - oz;
+        return qx * qx + qy * qy + qz * qz + dd2 * (qx - qy);
+      };
+      double R0 = 1e300, x0 = 0, y0 = 0, z0 = 0;
+      over(
+          [&](int, int r, bool valid) {
+            if (!valid) return;
+            double qx, qy, qz;
+            const double R = load(r, qx, qy, qz);
+            if (R < R0) {
+              R0 = R;
+              x0 = qx;
+              y0 = qy;
+              z0 = qz;
+            }
+          },
+          [](int) {});
+      double best = R0;
 #pragma unroll
-    for (int a = 0; a < 3; ++a) {
-      bx[a] = lo[a];
-      bx[3 + a] = hi[a];
+      for (int o = 1; o < 64; o <<= 1) best = fmin(best, __shfl_xor(best, o));
+      const int src = (int)__builtin_ctzll(__ballot(R0 == best));
+      R0 = best;
+      x0 = __shfl(x0, src);
+      y0 = __shfl(y0, src);
+      z0 = __shfl(z0, src);
+      // 1e-3: far above the rounding of either side (and of the FP64 search)
+      auto keep = [&](double R, double qx, double qy, double qz) {
+        return (R - R0) - half2 * (fabs(qx - x0) + fabs(qy - y0) + fabs(qz - z0)) <= 1e-3;
+      };
+      int groups = 0, cnt = 0;
+      over(
+          [&](int, int r, bool valid) {
+            double qx, qy, qz;
+            const double R = load(valid ? r : 0, qx, qy, qz);
+            cnt += __popcll(__ballot(valid && keep(R, qx, qy, qz)));
+          },
+          [&](int) {
+            groups += (cnt + kChunk - 1) / kChunk;
+            cnt = 0;
+          });
+      int first = 0;
+      if (lane == 0 && groups > 0) first = atomicAdd(cd.row_n, groups);
+      first = __builtin_amdgcn_readfirstlane(first);
+      if (first > cd.row_groups - groups) {
+        if (lane == 0) *out = make_int2(0, -1);  // no room: the slot is searched without a list
+        continue;
+      }
+      int cur = first;
+      over(
+          [&](int, int r, bool valid) {
+            double qx, qy, qz;
+            const double R = load(valid ? r : 0, qx, qy, qz);
+            const bool k = valid && keep(R, qx, qy, qz);
+            const unsigned long long m = __ballot(k);
+            if (k) {
+              const int pos = cnt + __popcll(m & ((1ull << lane) - 1ull));
+              const int64_t row = (int64_t)cur * kChunk + pos;
+              store_row(cd.rows + kRowLen * row, qx, qy, qz, R);
+              cd.rsrc[row] = r;
+              rho2 = fmaxf(rho2, (float)(qx * qx + qy * qy + qz * qz));
+            }
+            cnt += __popcll(m);
+          },
+          [&](int e) {
+            const int ng = (cnt + kChunk - 1) / kChunk;
+            if (cnt + lane < ng * kChunk) {
+              const int64_t row = (int64_t)cur * kChunk + cnt + lane;
+              store_row(cd.rows + kRowLen * row, 0.0, 0.0, 0.0, kFarPoint);
+              cd.rsrc[row] = -1;
+            }
+            for (int t = lane; t < ng; t += 64) cd.tags[cur + t] = (uint16_t)(e | (t == ng - 1 ? kTagEnd : 0));
+            cur += ng;
+            cnt = 0;
+          });
+      if (lane == 0) *out = make_int2(first, groups);
     }
+#pragma unroll
+    for (int o = 1; o < 64; o <<= 1) rho2 = fmaxf(rho2, __shfl_xor(rho2, o));
+    if (lane == 0) atomicMax(&s_rho, __float_as_int(1.0001f * sqrtf(rho2)));  // non-negative: ordered as integers
+    __syncthreads();
+    if (tid == 0) {
+      cd.org[g] = make_int4(ox, oy, oz, s_rho);
+      cd.sbox[g] = make_int4(b[0], b[1], b[2], n);
+    }
+    __syncthreads();  // the tables are refilled for the next grain
   }
 }
 
-// Queue entry of a band voxel: its layer cell, and its IDLocal id's slot in the
-// grain's hull-id table + 1 (0: not there).  Bucket of the slot grouping: the
-// slot, or kTopoCap for an id the hull does not name.
-__device__ inline int bucket_of(uint32_t qv) {
-  const int f = (int)(qv >> kCellBits);
-  return f == 0 ? kTopoCap : f - 1;
+// The filter's values are finite, so its minima need no handling of NaN (which
+// would be an extra instruction per operand).
+#pragma float_control(precise, off, push)
+__device__ inline float min4(const v16f& d, int u, float run) {
+  return fminf(fminf(fminf(fminf(run, d[4 * u]), d[4 * u + 1]), d[4 * u + 2]), d[4 * u + 3]);
+}
+__device__ inline float min16(const v16f& d, float run) {
+  float m = run;
+#pragma unroll
+  for (int i = 0; i < 16; i += 2) m = fminf(fminf(m, d[i]), d[i + 1]);
+  return m;
 }
 
-template <class T, int NMAX>
-__global__ __launch_bounds__(256) void k_correct(SimParams sp, PlanDev P, int cls, const int32_t* __restrict__ state,
+// Two smallest filter values over different elements: m1 of element e1, m2 of
+// any other.
+struct Near {
+  float m1, m2;
+  int e1;
+  __device__ void add(float m, int e) {  // element e's smallest value; elements come one by one
+    m2 = fminf(m2, fmaxf(m1, m));
+    e1 = m < m1 ? e : e1;
+    m1 = fminf(m1, m);
+  }
+  __device__ void merge_halves() {  // the lane pair (l, l ^ 32) holds one voxel's two halves of the rows
+    const float o1 = __shfl_xor(m1, 32), o2 = __shfl_xor(m2, 32);
+    const int oe = __shfl_xor(e1, 32);
+    const float other = fminf(m2, o2);
+    m2 = oe == e1 ? other : fminf(other, fmaxf(m1, o1));
+    e1 = o1 < m1 ? oe : e1;
+    m1 = fminf(m1, o1);
+  }
+};
+#pragma float_control(pop)
+
+// One workgroup per (grain, run of ZT z-layers) of the output box: its band
+// voxels are queued in LDS grouped by the slot of their IDLocal id in the
+// grain's hull-id table, and a wavefront takes up to kTake of one slot at a
+// time, whichever are left.
+template <class T, int NMAX, int ZT>
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4))) void k_correct(SimParams sp, PlanDev P, int cls, const int32_t* __restrict__ state,
                                                  DescDev din, DescDev dout, IdlDev il, TopoDev topo, CorrDev cd) {
   if (*cd.ready == 0) return;  // no hull yet (run_sim's first step)
   constexpr int kBuckets = kTopoCap + 1;  // a slot, or the last bucket: an id the hull does not name
-  static_assert(kTopoCap == 64, "one wavefront scans the slot buckets");
+  static_assert(kTopoCap == 64, "one lane per slot");
+  constexpr int VPT = (ZT * NMAX * NMAX + 255) / 256;  // voxels per thread
+  static_assert(ZT * NMAX * NMAX <= 0xFFFF, "cell indexes are 16-bit");
   __shared__ int s_key[kTopoCap];
-  __shared__ unsigned long long s_em[kElemCap];
-  __shared__ double s_en[kElemCap], s_mo[kElemCap];
-  __shared__ int s_ef[kElemCap + 1];
-  __shared__ uint32_t s_raw[NMAX * NMAX];  // band voxels in layer order
-  __shared__ uint32_t s_q[NMAX * NMAX];    // the same, grouped by slot
-  __shared__ int s_cnt[kBuckets], s_at[kBuckets];
-  __shared__ int s_nq;
+  __shared__ uint16_t s_q[ZT * NMAX * NMAX];  // band voxels grouped by slot
+  __shared__ int s_cnt[kBuckets];
+  __shared__ int s_next;
   const int total = P.totals[kQLayers * kClasses + cls];
-  const int tid = threadIdx.x, lane = tid & 63, wv = tid >> 6;
+  const int tid = threadIdx.x, lane = tid & 63;
   const T* __restrict__ ain = (const T*)din.arena;
   T* __restrict__ aout = (T*)dout.arena;
   const double delta = sp.delta;
-  // consecutive tiles (the layers of one grain) on one XCD: the layer two
-  // tiles share, and the grain's tables, come from that XCD's L2
+  // consecutive tiles (the layers of one grain) on one XCD: the grain's
+  // rows and tables come from that XCD's L2
   const TileRange tr = xcd_tiles(total);
   for (int tile = tr.first; tile < tr.end; tile += tr.step) {
     int g, kl;
     plan_tile(P, cls, kQLayers, tile, g, kl);
+    if (kl % ZT) continue;  // the plan's tiles are single layers; the first of a run takes the run
     const int32_t* b = dout.bounds + 6 * g;
     const int x0 = b[0], y0 = b[1], z0 = b[2], n = b[3] - b[0], nn2 = n * n;
+    const int nv = min(ZT, n - kl) * nn2;  // voxels of the run
     // a grain whose barycenters did not fit the pool (the device error is set)
     // is corrected with the default weights
     const int64_t tb = cd.tbase[g];
     int E = cd.ecount[g];
     if (tb + cd.efirst[(int64_t)g * (kElemCap + 1) + E] > cd.tri_cap) E = 0;
+    const int4 sb = cd.sbox[g];
+    const bool lists = sb.x == x0 && sb.y == y0 && sb.z == z0 && sb.w == n;  // they hold for this box
     for (int i = tid; i < kTopoCap; i += 256) s_key[i] = topo.key[(int64_t)g * kTopoCap + i];
-    for (int e = tid; e < E; e += 256) {
-      s_em[e] = cd.emask[(int64_t)g * kElemCap + e];
-      s_en[e] = cd.energy[(int64_t)g * kElemCap + e];
-      s_mo[e] = cd.mobility[(int64_t)g * kElemCap + e];
-    }
-    for (int e = tid; e <= E; e += 256) s_ef[e] = cd.efirst[(int64_t)g * (kElemCap + 1) + e];
     if (tid < kBuckets) s_cnt[tid] = 0;
-    if (tid == 0) s_nq = 0;
+    if (tid == 0) s_next = 0;
     __syncthreads();
     // IDLocal as the resize to the output bounds leaves it: the old content at
     // the same linear index, 0 past its old size
     const int32_t* ob = il.bounds + 6 * g;
     const int64_t oldsize = (int64_t)(ob[3] - ob[0]) * (ob[4] - ob[1]) * (ob[5] - ob[2]);
-    const uint32_t* __restrict__ idl = il.arena + il.off[g];
-    const T* __restrict__ in = ain + din.off[g];
-    T* __restrict__ out = aout + dout.off[g];
     const int64_t lbase = (int64_t)kl * nn2;
-    for (int c = tid; c < nn2; c += 256) {
-      const double val = (double)in[lbase + c];
-      if (fabs(val) < delta) {
-        const int64_t li = lbase + c;
-        const uint32_t id = li < oldsize ? idl[li] : 0u;
-        int slot = -1;
-        uint32_t hsl = (id * 2654435761u) >> (32 - kTopoCapBitsC);
-        for (int pr = 0; pr < kTopoCap; ++pr) {
-          const int k = s_key[hsl];
-          if (k == (int)id) {
-            slot = (int)hsl;
-            break;
-          }
-          if (k == -1) break;
-          hsl = (hsl + 1) & (kTopoCap - 1);
-        }
-        const uint32_t qv = (uint32_t)c | (uint32_t)(slot + 1) << kCellBits;
-        atomicAdd(&s_cnt[bucket_of(qv)], 1);
-        s_raw[atomicAdd(&s_nq, 1)] = qv;
-      }
-    }
-    __syncthreads();
-    // group the queue by slot (counting sort), so that a wavefront's voxels
-    // mostly border one grain and it walks only that grain's elements
-    if (wv == 0) {
-      const int v = s_cnt[lane];
-      int incl = v;
+    const uint32_t* __restrict__ idl = il.arena + il.off[g] + lbase;
+    const int oldn = (int)min((int64_t)nv, oldsize - lbase);  // cells below it have an old id
+    const T* __restrict__ in = ain + din.off[g] + lbase;
+    T* __restrict__ out = aout + dout.off[g] + lbase;
+    // counting sort of the band voxels by slot: each lane keeps its voxels'
+    // bucket and rank in registers, so one LDS queue is enough
+    int pk[VPT];  // bucket << 16 | rank in the bucket, -1: not in the band
 #pragma unroll
-      for (int d = 1; d < 64; d <<= 1) {
-        const int u = __shfl_up(incl, d, 64);
-        if (lane >= d) incl += u;
+    for (int u0 = 0; u0 < VPT; u0 += 4) {
+      T v[4];
+      uint32_t id[4];
+#pragma unroll
+      for (int u = 0; u < 4; ++u) {
+        const int c = (u0 + u) * 256 + tid;
+        if (u0 + u < VPT && c < nv) v[u] = in[c];
       }
-      s_at[lane] = incl - v;
-      if (lane == 63) s_at[kTopoCap] = incl;
+#pragma unroll
+      for (int u = 0; u < 4; ++u) {
+        const int c = (u0 + u) * 256 + tid;
+        const bool band = u0 + u < VPT && c < nv && fabs((double)v[u]) < delta;
+        if (u0 + u < VPT) pk[u0 + u] = band ? 0 : -1;
+        id[u] = band && c < oldn ? idl[c] : 0u;
+      }
+#pragma unroll
+      for (int u = 0; u < 4; ++u) {
+        if (u0 + u < VPT && pk[u0 + u] == 0) {
+          int bucket = kTopoCap;
+          uint32_t hsl = (id[u] * 2654435761u) >> (32 - kTopoCapBitsC);
+          for (int pr = 0; pr < kTopoCap; ++pr) {
+            const int k = s_key[hsl];
+            if (k == (int)id[u]) {
+              bucket = (int)hsl;
+              break;
+            }
+            if (k == -1) break;
+            hsl = (hsl + 1) & (kTopoCap - 1);
+          }
+          pk[u0 + u] = bucket << 16 | atomicAdd(&s_cnt[bucket], 1);
+        }
+      }
     }
     __syncthreads();
-    const int nq = s_nq;
-    for (int w = tid; w < nq; w += 256) {
-      const uint32_t qv = s_raw[w];
-      s_q[atomicAdd(&s_at[bucket_of(qv)], 1)] = qv;
+    // lane s: slot s's count, first queue entry and first chunk of kTake entries
+    const int cnt = s_cnt[lane], cnt_none = s_cnt[kTopoCap];
+    const int both = cnt | ((cnt + kTake - 1) / kTake) << 16;
+    int incl = both;
+#pragma unroll
+    for (int d = 1; d < 64; d <<= 1) {
+      const int u = __shfl_up(incl, d, 64);
+      if (lane >= d) incl += u;
+    }
+    const int start = (incl - both) & 0xFFFF, chunk0 = (incl - both) >> 16;
+    const int all = __builtin_amdgcn_readlane(incl, 63);
+    const int named = all & 0xFFFF, nch = all >> 16;  // entries with a slot, and their chunks
+#pragma unroll
+    for (int u = 0; u < VPT; ++u) {
+      const int bucket = pk[u] >> 16;
+      const int at = __shfl(start, bucket & 63, 64);
+      if (pk[u] >= 0) s_q[(bucket < kTopoCap ? at : named) + (pk[u] & 0xFFFF)] = (uint16_t)(u * 256 + tid);
     }
     __syncthreads();
     const double* __restrict__ tri = cd.tri + 3 * tb;
+    const int4 o4 = cd.org[g];
     const double see_g = cd.see_on ? cd.see[g] : 0.0;
-    for (int w0 = wv * 64; w0 < nq; w0 += 256) {
-      const int w = w0 + lane;  // a wavefront takes 64 consecutive queue entries
-      const bool act = w < nq;
-      const uint32_t qv = act ? s_q[w] : 0u;
-      const int c = (int)(qv & ((1u << kCellBits) - 1u));
-      const int slot = (int)(qv >> kCellBits) - 1;
-      const int yl = c / n, xl = c - yl * n;
-      // Vector3d(i, j, k): row, column, depth, against barycenters (x, y, z)
-      const double px = (double)(y0 + yl), py = (double)(x0 + xl), pz = (double)(z0 + kl);
-      // the first nearest barycenter in the projection order is the smallest
-      // (squared distance, element) pair, found here in any order: elements
-      // from boundaries back to junctions, skipping every chunk whose box no
-      // lane can reach below its bound or its current pair
-      double dmin = 10000000.0;
-      int emin = -1;
-      const unsigned long long bit = (act && slot >= 0) ? 1ull << slot : 0ull;
-      const float* __restrict__ cbx = cd.cbox + 6 * (tb / kChunk);
-      // A chunk whose FP32 box lies beyond the lane's current pair cannot hold
-      // the answer.  Box distances only decide which chunks to skip, so each is
-      // taken with a margin that covers its rounding (about 3 ulp): the skip is
-      // conservative, and every barycenter that can win is compared in FP64.
-      // (A first pass that bounded the search by the nearest box's farthest
-      // corner cost more than it saved.)
-      const float fpx = (float)px, fpy = (float)py, fpz = (float)pz;  // integers: exact
-      for (int e = E - 1; e >= 0; --e) {
-        const bool need = (s_em[e] & bit) != 0ull;
-        if (__ballot(need) == 0ull) continue;
-        const int ch1 = __builtin_amdgcn_readfirstlane(s_ef[e + 1]) / kChunk;
-        for (int ch = __builtin_amdgcn_readfirstlane(s_ef[e]) / kChunk; ch < ch1; ++ch) {
-          const float* bx = cbx + 6 * ch;
-          const float ex = fmaxf(fmaxf(bx[0] - fpx, fpx - bx[3]), 0.0f);
-          const float ey = fmaxf(fmaxf(bx[1] - fpy, fpy - bx[4]), 0.0f);
-          const float ez = fmaxf(fmaxf(bx[2] - fpz, fpz - bx[5]), 0.0f);
-          const float lb = (ex * ex + ey * ey + ez * ez) * (1.0f - 1e-6f) - 1e-6f;  // below the true one
-          const bool want = need && (double)lb <= dmin;
-          if (__ballot(want) == 0ull) continue;
-          const double* q = tri + 3 * kChunk * ch;
+    const float fn = 1.0f / (float)n, fnn = 1.0f / (float)nn2;
+    // coordinates of cell c of the run: its layer, row and column
+    auto cell_at = [&](int c, int& zl, int& yl, int& xl) {
+      zl = (int)((float)c * fnn);
+      int r = c - zl * nn2;
+      if (r < 0) { --zl; r += nn2; }
+      if (r >= nn2) { ++zl; r -= nn2; }
+      yl = (int)((float)r * fn);
+      xl = r - yl * n;
+      if (xl < 0) { --yl; xl += n; }
+      if (xl >= n) { ++yl; xl -= n; }
+    };
+    const int nchunks = nch + (cnt_none + kTake - 1) / kTake;
+    for (;;) {
+      int j = 0;
+      if (lane == 0) j = atomicAdd(&s_next, 1);
+      j = __builtin_amdgcn_readfirstlane(j);
+      if (j >= nchunks) break;
+      int slot = -1, base, count;
+      if (j < nch) {
+        slot = 63 - (int)__builtin_clzll(__ballot(chunk0 <= j));
+        const int off = (j - __builtin_amdgcn_readlane(chunk0, slot)) * kTake;
+        base = __builtin_amdgcn_readlane(start, slot) + off;
+        count = min(kTake, __builtin_amdgcn_readlane(cnt, slot) - off);
+      } else {
+        const int off = (j - nch) * kTake;
+        base = named + off;
+        count = min(kTake, cnt_none - off);
+      }
+      Near nr[4] = {{kNone, kNone, -1}, {kNone, kNone, -1}, {kNone, kNone, -1}, {kNone, kNone, -1}};
+      bool listed = false;
+      int first = 0, npos = 0;
+      if (slot >= 0 && E > 0) {
+        const int2 sl = cd.slist[(int64_t)g * kTopoCap + slot];
+        first = __builtin_amdgcn_readfirstlane(sl.x);
+        npos = __builtin_amdgcn_readfirstlane(sl.y);
+        listed = lists && npos >= 0;
+        if (listed && npos > 0) {
+          // the voxels of queue entries base + 32 f + lane % 32 as columns
+          v8bf col[4];
 #pragma unroll
-          for (int u0 = 0; u0 < kChunk; u0 += 4) {
-            double d[4];
+          for (int f = 0; f < 4; ++f) {
+            const int fc = s_q[base + min(f * 32 + (lane & 31), count - 1)];
+            int fz, fy, fx;
+            cell_at(fc, fz, fy, fx);
+            const __bf16 bx = (__bf16)(float)(y0 + fy - o4.y), by = (__bf16)(float)(x0 + fx - o4.x),
+                         bz = (__bf16)(float)(z0 + kl + fz - o4.z), one = (__bf16)1.0f, nul = (__bf16)0.0f;
+            if (lane < 32) col[f] = v8bf{bx, bx, bx, by, by, by, bz, bz};
+            else col[f] = v8bf{bz, one, one, one, nul, nul, nul, nul};
+          }
+          float run[4] = {kNone, kNone, kNone, kNone};  // the running minimum of the current element
+          // lane's row of the four groups of a product, and its half of the row
+          const uint16_t* __restrict__ mine =
+              cd.rows + (int64_t)first * (kChunk * kRowLen) + (lane & 31) * kRowLen + (lane >> 5) * 8;
+          for (int t0 = 0; t0 < npos; t0 += 64) {
+            const int np = min(64, npos - t0);
+            const int tag = lane < np ? (int)cd.tags[first + t0 + lane] : 0;  // lane t: group t0 + t's
+            const unsigned long long ends = __ballot(tag & kTagEnd);
+            auto fetch = [&](int i) {  // groups t0 + i .. + 3 (up to kRowSpare past the list: not used)
+              return *(const v8bf*)(mine + (int64_t)(t0 + i) * (kChunk * kRowLen));
+            };
+            auto product = [&](const v8bf& a, int i) {
+              const int nib = (int)(ends >> i) & 15;
+              const bool whole = (nib & 7) == 0 && i + 4 <= np;  // the four groups are one element's
 #pragma unroll
-            for (int u = 0; u < 4; ++u) {
-              const double dx = px - q[3 * (u0 + u)], dy = py - q[3 * (u0 + u) + 1], dz = pz - q[3 * (u0 + u) + 2];
-              d[u] = dx * dx + dy * dy + dz * dz;
+              for (int f = 0; f < 4; f += 2) {
+                if (f * 32 >= count) break;
+                const v16f d0 = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a, col[f], v16f{}, 0, 0, 0);
+                const v16f d1 = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a, col[f + 1], v16f{}, 0, 0, 0);
+                if (whole) {
+                  run[f] = min16(d0, run[f]);
+                  run[f + 1] = min16(d1, run[f + 1]);
+                  if (nib) {
+                    const int e = __builtin_amdgcn_readlane(tag, i + 3) & (kTagEnd - 1);
+                    nr[f].add(run[f], e);
+                    nr[f + 1].add(run[f + 1], e);
+                    run[f] = run[f + 1] = kNone;
+                  }
+                } else {
+#pragma unroll
+                  for (int u = 0; u < 4; ++u) {
+                    if (i + u < np) {
+                      run[f] = min4(d0, u, run[f]);
+                      run[f + 1] = min4(d1, u, run[f + 1]);
+                      if ((nib >> u) & 1) {
+                        const int e = __builtin_amdgcn_readlane(tag, i + u) & (kTagEnd - 1);
+                        nr[f].add(run[f], e);
+                        nr[f + 1].add(run[f + 1], e);
+                        run[f] = run[f + 1] = kNone;
+                      }
+                    }
+                  }
+                }
+              }
+            };
+            v8bf a0 = fetch(0), a1 = fetch(4);
+            for (int i = 0; i < np; i += 8) {
+              const v8bf b0 = fetch(i + 8), b1 = fetch(i + 12);
+              product(a0, i);
+              if (i + 4 < np) product(a1, i + 4);
+              a0 = b0;
+              a1 = b1;
+            }
+          }
+#pragma unroll
+          for (int f = 0; f < 4; ++f) nr[f].merge_halves();
+        }
+      }
+#pragma unroll
+      for (int h = 0; h < kTake / 64; ++h) {  // 64 of the voxels, one per lane
+        if (h * 64 >= count) break;
+        const bool act = h * 64 + lane < count;
+        const int c = s_q[base + (act ? h * 64 + lane : 0)];
+        int zl, yl, xl;
+        cell_at(c, zl, yl, xl);
+        // Vector3d(i, j, k): row, column, depth, against barycenters (x, y, z)
+        const int px = y0 + yl, py = x0 + xl, pz = z0 + kl + zl;
+        const Near me = lane < 32 ? nr[2 * h] : nr[2 * h + 1];
+        int emin = me.e1;
+        if (slot >= 0 && E > 0) {
+          bool exact = act;
+          if (listed) {
+            const float qx = (float)(px - o4.y), qy = (float)(py - o4.x), qz = (float)(pz - o4.z);
+            const float rho = __int_as_float(o4.w);
+            const float dd = 1.4143f * fabsf((float)(o4.x - o4.y)), pp = sqrtf(qx * qx + qy * qy + qz * qz);
+            const float S = rho * rho + 2.0f * rho * (dd + pp);
+            // a squared distance of 1e7 or more is no neighbour (the reference's
+            // initial minimum): the FP64 search decides where one could be that far
+            const float reach = dd + pp + rho;
+            exact = act && emin >= 0 && (me.m2 - me.m1 <= 2.0f * kFilterEps * S || reach * reach > 9.9e6f);
+          }
+          unsigned long long todo = __ballot(exact);
+          if (listed && __popcll(todo) > kManyExact) {
+            // every lane searches for its own voxel, the rows' barycenters uniform
+            double dmin = 10000000.0;
+            int em = -1;
+            for (int t = 0; t < npos; ++t) {
+              const int e = cd.tags[first + t] & (kTagEnd - 1);
+#pragma unroll
+              for (int r = 0; r < kChunk; ++r) {
+                const int src = cd.rsrc[((int64_t)first + t) * kChunk + r];
+                const double* q = tri + 3 * (int64_t)max(src, 0);
+                const double dx = px - q[0], dy = py - q[1], dz = pz - q[2];
+                const double d = dx * dx + dy * dy + dz * dz;
+                if (src >= 0 && (d < dmin || (d == dmin && e < em))) {
+                  dmin = d;
+                  em = e;
+                }
+              }
+            }
+            if (exact) emin = em;
+            todo = 0;
+          }
+          for (; todo; todo &= todo - 1) {
+            const int who = (int)__builtin_ctzll(todo);
+            const double dpx = (double)__builtin_amdgcn_readlane(px, who),
+                         dpy = (double)__builtin_amdgcn_readlane(py, who),
+                         dpz = (double)__builtin_amdgcn_readlane(pz, who);
+            double dmin = 10000000.0;
+            int em = -1;
+            auto attempt = [&](int r, int e) {
+              const double* q = tri + 3 * (int64_t)r;
+              const double dx = dpx - q[0], dy = dpy - q[1], dz = dpz - q[2];
+              const double d = dx * dx + dy * dy + dz * dz;
+              if (d < dmin || (d == dmin && e < em)) {
+                dmin = d;
+                em = e;
+              }
+            };
+            if (listed) {
+              for (int r = lane; r < npos * kChunk; r += 64) {
+                const int src = cd.rsrc[(int64_t)first * kChunk + r];
+                if (src >= 0) attempt(src, cd.tags[first + r / kChunk] & (kTagEnd - 1));
+              }
+            } else {
+              for (int e0 = 0; e0 < E; e0 += 64) {
+                const int el = e0 + lane;
+                const bool has = el < E && ((cd.emask[(int64_t)g * kElemCap + (el < E ? el : 0)] >> slot) & 1ull);
+                for (unsigned long long m = __ballot(has); m; m &= m - 1) {
+                  const int e = e0 + (int)__builtin_ctzll(m);
+                  const int32_t* ef = cd.efirst + (int64_t)g * (kElemCap + 1) + e;
+                  const int r1 = ef[1];
+                  for (int r = ef[0] + lane; r < r1; r += 64) attempt(r, e);
+                }
+              }
             }
 #pragma unroll
-            for (int u = 0; u < 4; ++u)
-              if (want && (d[u] < dmin || (d[u] == dmin && e < emin))) {
-                dmin = d[u];
-                emin = e;
+            for (int o = 1; o < 64; o <<= 1) {  // the smallest (distance, element) pair
+              const double od = __shfl_xor(dmin, o);
+              const int oe = __shfl_xor(em, o);
+              if (od < dmin || (od == dmin && (unsigned)oe < (unsigned)em)) {
+                dmin = od;
+                em = oe;
               }
+            }
+            if (lane == who) emin = em;
           }
         }
-      }
-      const double w_energy = emin >= 0 ? s_mo[emin] : 1.0, w_mobility = emin >= 0 ? s_en[emin] : 1.0;
-      if (act) {
-        const int64_t li = lbase + c;
-        const double val = (double)in[li];
-        double o = (double)out[li];
-        o = val + (o - val) * w_energy * w_mobility;
-        if (cd.see_on) {
-          const uint32_t id = li < oldsize ? idl[li] : 0u;
-          const bool nb = id == 0u || (id <= (uint32_t)sp.N && state[id] != kDeleted);
-          double f = 0;
-          if (nb) f = (see_g - cd.see[id]) * w_mobility * cd.dt / cd.tsq;
-          o = o - f;
+        double w_energy = 1.0, w_mobility = 1.0;
+        if (emin >= 0) {
+          w_energy = cd.mobility[(int64_t)g * kElemCap + emin];
+          w_mobility = cd.energy[(int64_t)g * kElemCap + emin];
         }
-        out[li] = (T)o;
+        if (act) {
+          const double val = (double)in[c];
+          double o = (double)out[c];
+          o = val + (o - val) * w_energy * w_mobility;
+          if (cd.see_on) {
+            const uint32_t id = c < oldn ? idl[c] : 0u;
+            const bool nb = id == 0u || (id <= (uint32_t)sp.N && state[id] != kDeleted);
+            double f = 0;
+            if (nb) f = (see_g - cd.see[id]) * w_mobility * cd.dt / cd.tsq;
+            o = o - f;
+          }
+          out[c] = (T)o;
+        }
       }
     }
-    __syncthreads();  // the queues and the element tables are refilled for the next tile
+    __syncthreads();  // the queue is refilled for the next tile
   }
 }
 
 template <class T>
 void correct_classes(const Launch& L, const SimParams& sp, const PlanDev& P, const int32_t* state, const DescDev& din,
                      const DescDev& dout, const IdlDev& il, const TopoDev& topo, const CorrDev& cd) {
-  hipLaunchKernelGGL((k_correct<T, 32>), dim3(tile_grid(L, kCorrGridPerCU, 0)), dim3(256), 0, L.stream, sp, P, 0,
+  hipLaunchKernelGGL((k_correct<T, 32, 4>), dim3(tile_grid(L, kCorrGridPerCU, 0)), dim3(256), 0, L.stream, sp, P, 0,
                      state, din, dout, il, topo, cd);
-  hipLaunchKernelGGL((k_correct<T, 48>), dim3(tile_grid(L, kCorrGridPerCU, 1)), dim3(256), 0, L.stream, sp, P, 1,
+  hipLaunchKernelGGL((k_correct<T, 48, 4>), dim3(tile_grid(L, kCorrGridPerCU, 1)), dim3(256), 0, L.stream, sp, P, 1,
                      state, din, dout, il, topo, cd);
-  hipLaunchKernelGGL((k_correct<T, 64>), dim3(tile_grid(L, kCorrGridPerCU, 2)), dim3(256), 0, L.stream, sp, P, 2,
+  hipLaunchKernelGGL((k_correct<T, 64, 2>), dim3(tile_grid(L, kCorrGridPerCU, 2)), dim3(256), 0, L.stream, sp, P, 2,
                      state, din, dout, il, topo, cd);
-  hipLaunchKernelGGL((k_correct<T, 96>), dim3(tile_grid(L, kCorrGridPerCU, 3)), dim3(256), 0, L.stream, sp, P, 3,
+  hipLaunchKernelGGL((k_correct<T, 96, 1>), dim3(tile_grid(L, kCorrGridPerCU, 3)), dim3(256), 0, L.stream, sp, P, 3,
                      state, din, dout, il, topo, cd);
 }
 
 }  // namespace
 
-void launch_elements(const Launch& L, const SimParams& sp, const int32_t* state, const TopoDev& topo,
-                     const CorrDev& cd, int32_t* err) {
-  hipLaunchKernelGGL(k_clear_counter, dim3(1), dim3(64), 0, L.stream, cd.tri_n);
+void launch_elements(const Launch& L, const SimParams& sp, const int32_t* state, const DescDev& dout,
+                     const TopoDev& topo, const CorrDev& cd, int32_t* err) {
+  hipLaunchKernelGGL(k_clear_counters, dim3(1), dim3(64), 0, L.stream, cd.tri_n, cd.row_n);
   const int blocks = sp.N < L.grid ? sp.N : L.grid;
   hipLaunchKernelGGL(k_elements, dim3(blocks > 0 ? blocks : 1), dim3(kEW), 0, L.stream, sp, state, topo, cd, err);
   hipLaunchKernelGGL(k_tri_scatter, dim3(L.grid), dim3(256), 0, L.stream, topo, cd);
-  hipLaunchKernelGGL(k_chunk_boxes, dim3(L.grid), dim3(256), 0, L.stream, cd);
+  hipLaunchKernelGGL(k_slots, dim3(sp.N > 0 ? sp.N : 1), dim3(256), 0, L.stream, sp, state, dout, topo, cd);
 }
 
 void launch_correction(const Launch& L, const SimParams& sp, const PlanDev& P, const int32_t* state,

@@ -93,8 +93,11 @@ struct TopoDev {
 // junctions, triple lines, boundaries.  An element's neighbour set is a mask
 // over the grain's hull-id table slots (TopoDev::key).
 constexpr int kElemCap = kJuncCap;
-constexpr int kChunk = 16;         // barycenters per bounding box of the nearest-element search
-constexpr double kFarPoint = 1e30;  // coordinate of a chunk's padding points
+constexpr int kChunk = 8;          // rows of one element come in groups of kChunk
+constexpr double kFarPoint = 1e30;  // squared distance that a group's padding rows stand for
+constexpr int kRowLen = 16;        // BF16 values of a barycenter's row in the nearest-element filter
+constexpr int kRowSpare = 64;      // groups past the pool's end, read ahead and never used
+constexpr int kTagEnd = 0x8000;
 struct CorrDev {
   int32_t* ready;              // set by the element build: a hull with elements exists (run_sim's loop != 0)
   int see_on;                  // Settings::UseStoredElasticEnergy
@@ -115,9 +118,18 @@ struct CorrDev {
   int32_t* ecur;               // [(N+1) * kElemCap] fill cursors
   int32_t* slot_elem;          // [(N+1) * kJuncCap] element of each junction slot
   int64_t* tbase;              // [N+1] the grain's first barycenter in tri
-  double* tri;                 // [3 * tri_cap] barycenters grouped by element, each element padded
-                               // to whole chunks of kChunk with far-away points
-  float* cbox;                 // [6 * (tri_cap / kChunk)] bounding box of each chunk (lo xyz, hi xyz)
+  double* tri;                 // [3 * tri_cap] barycenters grouped by element
+  // Per hull-id slot of each grain, the barycenters that can be the nearest of
+  // its elements to some voxel of the grain's box (k_slots in gg_correct.hip).
+  int2* slist;                 // [(N+1) * kTopoCap] first group and groups of the slot's list (-1: no list)
+  int4* sbox;                  // [N+1] the box the lists hold for: x0, y0, z0, side
+  int4* org;                   // [N+1] grid point the rows are relative to (x, y, z), and the largest distance of
+                               // a listed barycenter from it (the bits of a float)
+  uint16_t* rows;              // [kRowLen * kChunk * (row_groups + kRowSpare)] rows of the filter's matrix
+  int32_t* rsrc;               // [kChunk * row_groups] the row's barycenter, relative to tbase (-1: padding)
+  uint16_t* tags;              // [row_groups + kRowSpare] element of each group, kTagEnd on its last one
+  int* row_n;                  // groups placed (may exceed row_groups: then slots have no list)
+  int row_groups;
   unsigned long long* tri_n;   // barycenters placed
   int64_t tri_cap;
 };
@@ -419,8 +431,8 @@ void upload_mc_tables();
 // Convolution correction (gg_correct.hip): the elements of every alive grain
 // from its last hull (after launch_hull with topo.corr), their barycenters
 // grouped by element, and the correction of the convolved output buffer.
-void launch_elements(const Launch& L, const SimParams& sp, const int32_t* state, const TopoDev& topo,
-                     const CorrDev& cd, int32_t* err);
+void launch_elements(const Launch& L, const SimParams& sp, const int32_t* state, const DescDev& dout,
+                     const TopoDev& topo, const CorrDev& cd, int32_t* err);
 void launch_correction(const Launch& L, const SimParams& sp, const PlanDev& P, const int32_t* state,
                        const DescDev& din, const DescDev& dout, const IdlDev& il_stale, const TopoDev& topo,
                        const CorrDev& cd, bool fp32);
