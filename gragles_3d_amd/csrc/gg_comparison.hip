@@ -9,6 +9,8 @@
 // reference's neighbour-outer loop; then the wall distance, IDLocal (new id,
 // or the previous step's id at the same linear index when nothing covers the
 // voxel), 0.5*(in - max) inside 0.7*delta, and the bounding box of phi >= 0.
+#include <algorithm>
+
 #include "gg_internal.h"
 
 namespace gg {
@@ -492,11 +494,12 @@ void space_launch(const Launch& L, const SimParams& sp, const PlanDev& P, const 
     hipLaunchKernelGGL(k_space_bin<true>, dim3(gb), dim3(256), 0, L.stream, sp, P, din, W, ZL, err);
   }
   if (part == kSpaceBuild) return;
+  const int grid = (int)std::min<int64_t>((int64_t)L.cus * kColGridPerCUSpace, ((int64_t)W.cap / 4 + kXcds) / kXcds * kXcds);
   if (sp.N < 0xFFFF)
-    hipLaunchKernelGGL((k_cmp_space<T, ZL, QB, true>), dim3(L.cus * kColGridPerCUSpace), dim3(256), 0, L.stream, sp,
+    hipLaunchKernelGGL((k_cmp_space<T, ZL, QB, true>), dim3(grid), dim3(256), 0, L.stream, sp,
                        W, din, dout, ld, ilo, iln, newb);
   else
-    hipLaunchKernelGGL((k_cmp_space<T, ZL, QB, false>), dim3(L.cus * kColGridPerCUSpace), dim3(256), 0, L.stream, sp,
+    hipLaunchKernelGGL((k_cmp_space<T, ZL, QB, false>), dim3(grid), dim3(256), 0, L.stream, sp,
                        W, din, dout, ld, ilo, iln, newb);
 }
 
@@ -528,7 +531,7 @@ void cmp_launch(const Launch& L, int cls, const SimParams& sp, const PlanDev& P,
                 const DescDev& dout, const ListDev& ld, const IdlDev& ilo, const IdlDev& iln, int32_t* newb) {
   constexpr int ZL = kCmpShapes[V][0], QB = kCmpShapes[V][1];
   constexpr bool ZMAJ = kCmpShapes[V][2] != 0;
-  hipLaunchKernelGGL((k_cmp_cols<T, NMAX, ZL, QB, ZMAJ>), dim3(tile_grid(L, kColGridPerCU, cls)), dim3(256), 0,
+  hipLaunchKernelGGL((k_cmp_cols<T, NMAX, ZL, QB, ZMAJ>), dim3(tile_grid(L, kColGridPerCU, cls, sp.N, (cols_of(cls) * ((NMAX + ZL - 1) / ZL) + 3) / 4)), dim3(256), 0,
                      L.stream, sp, P, cls, din, dout, ld, ilo, iln, newb);
 }
 

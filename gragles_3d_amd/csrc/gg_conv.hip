@@ -699,24 +699,25 @@ __global__ __launch_bounds__(kT) void k_circ_z_bf16(PlanDev P, int cls, DescDev 
 
 // part 0: (x,y) forward / x-then-y circulant; part 1: z; part 2: (y,x) inverse (FP64 only)
 template <int NMAX>
-void conv_class(const Launch& L, int part, const PlanDev& P, int cls, const DescDev& din, const DescDev& dout,
+void conv_class(const Launch& L, int part, const SimParams& sp, const PlanDev& P, int cls, const DescDev& din, const DescDev& dout,
                 const TablesDev& tb, const int64_t* spec_off, void* spec, int mode) {
-  const int grid = tile_grid(L, kGridPerCU, cls);
+  const int layers = tile_grid(L, kGridPerCU, cls, sp.N, layers_of(cls));
+  const int cols = tile_grid(L, kGridPerCU, cls, sp.N, mode == kConvFFT64 ? spec_cols_of(cls) : cols_of(cls));
   if (mode == kConvCirculantF32) {
-    if (part == 0) hipLaunchKernelGGL(k_circ_xy<NMAX>, dim3(grid), dim3(kT), 0, L.stream, P, cls, din, dout, tb);
-    if (part == 1) hipLaunchKernelGGL(k_circ_z<NMAX>, dim3(grid), dim3(kT), 0, L.stream, P, cls, dout, tb);
+    if (part == 0) hipLaunchKernelGGL(k_circ_xy<NMAX>, dim3(layers), dim3(kT), 0, L.stream, P, cls, din, dout, tb);
+    if (part == 1) hipLaunchKernelGGL(k_circ_z<NMAX>, dim3(cols), dim3(kT), 0, L.stream, P, cls, dout, tb);
   } else if (mode == kConvSplitBF16) {
-    if (part == 0) hipLaunchKernelGGL(k_circ_xy_bf16<NMAX>, dim3(grid), dim3(kT), 0, L.stream, P, cls, din, dout, tb);
-    if (part == 1) hipLaunchKernelGGL(k_circ_z_bf16<NMAX>, dim3(grid), dim3(kT), 0, L.stream, P, cls, dout, tb);
+    if (part == 0) hipLaunchKernelGGL(k_circ_xy_bf16<NMAX>, dim3(layers), dim3(kT), 0, L.stream, P, cls, din, dout, tb);
+    if (part == 1) hipLaunchKernelGGL(k_circ_z_bf16<NMAX>, dim3(cols), dim3(kT), 0, L.stream, P, cls, dout, tb);
   } else {
     if (part == 0)
-      hipLaunchKernelGGL(k_fft_xy_fwd<NMAX>, dim3(tile_grid(L, kGridPerCU, cls)), dim3(kT), 0, L.stream, P, cls, din, tb, spec_off,
+      hipLaunchKernelGGL(k_fft_xy_fwd<NMAX>, dim3(layers), dim3(kT), 0, L.stream, P, cls, din, tb, spec_off,
                          (double2*)spec);
     if (part == 1)
-      hipLaunchKernelGGL(k_fft_z<NMAX>, dim3(tile_grid(L, kGridPerCU, cls)), dim3(kT), 0, L.stream, P, cls, dout, tb, spec_off,
+      hipLaunchKernelGGL(k_fft_z<NMAX>, dim3(cols), dim3(kT), 0, L.stream, P, cls, dout, tb, spec_off,
                          (double2*)spec);
     if (part == 2)
-      hipLaunchKernelGGL(k_fft_xy_inv<NMAX>, dim3(tile_grid(L, kGridPerCU, cls)), dim3(kT), 0, L.stream, P, cls, dout, tb, spec_off,
+      hipLaunchKernelGGL(k_fft_xy_inv<NMAX>, dim3(layers), dim3(kT), 0, L.stream, P, cls, dout, tb, spec_off,
                          (const double2*)spec);
   }
 }
@@ -725,11 +726,10 @@ void conv_class(const Launch& L, int part, const PlanDev& P, int cls, const Desc
 
 void launch_conv(const Launch& L, int part, const SimParams& sp, const PlanDev& P, const DescDev& din,
                  const DescDev& dout, const TablesDev& tb, const int64_t* spec_off, void* spec, int mode) {
-  (void)sp;
-  conv_class<32>(L, part, P, 0, din, dout, tb, spec_off, spec, mode);
-  conv_class<48>(L, part, P, 1, din, dout, tb, spec_off, spec, mode);
-  conv_class<64>(L, part, P, 2, din, dout, tb, spec_off, spec, mode);
-  conv_class<96>(L, part, P, 3, din, dout, tb, spec_off, spec, mode);
+  conv_class<32>(L, part, sp, P, 0, din, dout, tb, spec_off, spec, mode);
+  conv_class<48>(L, part, sp, P, 1, din, dout, tb, spec_off, spec, mode);
+  conv_class<64>(L, part, sp, P, 2, din, dout, tb, spec_off, spec, mode);
+  conv_class<96>(L, part, sp, P, 3, din, dout, tb, spec_off, spec, mode);
 }
 
 }  // namespace gg

@@ -924,13 +924,13 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4))) void k
 template <class T>
 void correct_classes(const Launch& L, const SimParams& sp, const PlanDev& P, const int32_t* state, const DescDev& din,
                      const DescDev& dout, const IdlDev& il, const TopoDev& topo, const CorrDev& cd) {
-  hipLaunchKernelGGL((k_correct<T, 32, 4>), dim3(tile_grid(L, kCorrGridPerCU, 0)), dim3(256), 0, L.stream, sp, P, 0,
+  hipLaunchKernelGGL((k_correct<T, 32, 4>), dim3(tile_grid(L, kCorrGridPerCU, 0, sp.N, layers_of(0))), dim3(256), 0, L.stream, sp, P, 0,
                      state, din, dout, il, topo, cd);
-  hipLaunchKernelGGL((k_correct<T, 48, 4>), dim3(tile_grid(L, kCorrGridPerCU, 1)), dim3(256), 0, L.stream, sp, P, 1,
+  hipLaunchKernelGGL((k_correct<T, 48, 4>), dim3(tile_grid(L, kCorrGridPerCU, 1, sp.N, layers_of(1))), dim3(256), 0, L.stream, sp, P, 1,
                      state, din, dout, il, topo, cd);
-  hipLaunchKernelGGL((k_correct<T, 64, 2>), dim3(tile_grid(L, kCorrGridPerCU, 2)), dim3(256), 0, L.stream, sp, P, 2,
+  hipLaunchKernelGGL((k_correct<T, 64, 2>), dim3(tile_grid(L, kCorrGridPerCU, 2, sp.N, layers_of(2))), dim3(256), 0, L.stream, sp, P, 2,
                      state, din, dout, il, topo, cd);
-  hipLaunchKernelGGL((k_correct<T, 96, 1>), dim3(tile_grid(L, kCorrGridPerCU, 3)), dim3(256), 0, L.stream, sp, P, 3,
+  hipLaunchKernelGGL((k_correct<T, 96, 1>), dim3(tile_grid(L, kCorrGridPerCU, 3, sp.N, layers_of(3))), dim3(256), 0, L.stream, sp, P, 3,
                      state, din, dout, il, topo, cd);
 }
 

@@ -673,16 +673,16 @@ template <class T, bool TOPO>
 void hull_classes(const Launch& L, const SimParams& sp, const PlanDev& P, const DescDev& din, int32_t* exflag,
                   double* partials, const IdlDev& il, const TopoDev& topo, int32_t* err, int c0, int c1) {
   if (c0 <= 0 && 0 < c1)
-    hipLaunchKernelGGL((k_hull<T, 32, TOPO>), dim3(tile_grid(L, kGridPerCU, 0)), dim3(kHT), 0, L.stream, sp, P, 0,
+    hipLaunchKernelGGL((k_hull<T, 32, TOPO>), dim3(tile_grid(L, kGridPerCU, 0, sp.N, layers_of(0))), dim3(kHT), 0, L.stream, sp, P, 0,
                        din, exflag, partials, il, topo, err);
   if (c0 <= 1 && 1 < c1)
-    hipLaunchKernelGGL((k_hull<T, 48, TOPO>), dim3(tile_grid(L, kGridPerCU, 1)), dim3(kHT), 0, L.stream, sp, P, 1,
+    hipLaunchKernelGGL((k_hull<T, 48, TOPO>), dim3(tile_grid(L, kGridPerCU, 1, sp.N, layers_of(1))), dim3(kHT), 0, L.stream, sp, P, 1,
                        din, exflag, partials, il, topo, err);
   if (c0 <= 2 && 2 < c1)
-    hipLaunchKernelGGL((k_hull<T, 64, TOPO>), dim3(tile_grid(L, kGridPerCU, 2)), dim3(kHT), 0, L.stream, sp, P, 2,
+    hipLaunchKernelGGL((k_hull<T, 64, TOPO>), dim3(tile_grid(L, kGridPerCU, 2, sp.N, layers_of(2))), dim3(kHT), 0, L.stream, sp, P, 2,
                        din, exflag, partials, il, topo, err);
   if (c0 <= 3 && 3 < c1)
-    hipLaunchKernelGGL((k_hull<T, 96, TOPO>), dim3(tile_grid(L, kGridPerCU, 3)), dim3(kHT), 0, L.stream, sp, P, 3,
+    hipLaunchKernelGGL((k_hull<T, 96, TOPO>), dim3(tile_grid(L, kGridPerCU, 3, sp.N, layers_of(3))), dim3(kHT), 0, L.stream, sp, P, 3,
                        din, exflag, partials, il, topo, err);
 }
 

@@ -355,9 +355,20 @@ struct Launch {
 // Classes 2 and 3 (boxes of side 49..96) hold few grains in the workloads
 // measured here; their launches get 1/16 of that (at least 8 per CU), so a
 // nearly empty class does not pay for dispatching a full-size grid.
-inline int tile_grid(const Launch& L, int per_cu, int cls) {
-  return L.cus * (cls >= 2 ? (per_cu / 16 > 8 ? per_cu / 16 : 8) : per_cu);
+// Few grains cannot fill that: the launch never has more workgroups than
+// per_grain (what one grain's largest box of the class takes) times the grains,
+// as dispatching empty ones costs about 0.4 us per 1000 (64 to 131072 of them
+// per launch were up to 50 us, most of a step at 27 grains).  The count stays a
+// multiple of 8 (xcd_tiles).
+inline int tile_grid(const Launch& L, int per_cu, int cls, int grains, int per_grain) {
+  const int full = L.cus * (cls >= 2 ? (per_cu / 16 > 8 ? per_cu / 16 : 8) : per_cu);
+  const int64_t need = ((int64_t)grains * per_grain + kXcds - 1) / kXcds * kXcds;
+  return need < full ? (int)need : full;
 }
+// tiles of the largest box of a class
+inline int layers_of(int cls) { return class_max(cls); }
+inline int cols_of(int cls) { return (class_max(cls) * class_max(cls) + kColBlock - 1) / kColBlock; }
+inline int spec_cols_of(int cls) { return (class_max(cls) * (class_max(cls) / 2 + 1) + kSpecBlock - 1) / kSpecBlock; }
 
 void launch_plan(const Launch& L, const SimParams& sp, const int32_t* state, const int32_t* bounds,
                  int64_t* off_out, int64_t* spec_off, const PlanDev& P, int64_t arena_cap,

@@ -525,7 +525,7 @@ void k_redist_z_reg(SimParams sp, PlanDev P, int cls, DescDev din, DescDev dout)
 template <class T, int NMAX>
 void xy_class(const Launch& L, const SimParams& sp, const PlanDev& P, int cls, const DescDev& din,
               const DescDev& dout, int32_t* err) {
-  hipLaunchKernelGGL((k_redist_xy<T, NMAX>), dim3(tile_grid(L, kGridPerCU, cls)), dim3(128), 0, L.stream, sp, P, cls, din, dout, err);
+  hipLaunchKernelGGL((k_redist_xy<T, NMAX>), dim3(tile_grid(L, kGridPerCU, cls, sp.N, layers_of(cls))), dim3(128), 0, L.stream, sp, P, cls, din, dout, err);
 }
 
 // part 0: x/y sweeps per layer (one launch per size class); part 1: z sweeps + clamp
@@ -537,11 +537,11 @@ void redist_all(const Launch& L, int part, const SimParams& sp, const PlanDev& P
   auto in = [&](int c) { return c0 <= c && c < c1; };
   if (part == 0) {
     if (in(0))
-      hipLaunchKernelGGL((k_redist_xy_reg<T, 32>), dim3(tile_grid(L, kGridPerCU, 0)), dim3(64), 0, L.stream, sp, P, 0,
+      hipLaunchKernelGGL((k_redist_xy_reg<T, 32>), dim3(tile_grid(L, kGridPerCU, 0, sp.N, layers_of(0) / 2)), dim3(64), 0, L.stream, sp, P, 0,
                          din, dout, err);
     if (in(1)) {
       if constexpr (reg48)
-        hipLaunchKernelGGL((k_redist_xy_reg<T, 48>), dim3(tile_grid(L, kGridPerCU, 1)), dim3(64), 0, L.stream, sp, P,
+        hipLaunchKernelGGL((k_redist_xy_reg<T, 48>), dim3(tile_grid(L, kGridPerCU, 1, sp.N, layers_of(1))), dim3(64), 0, L.stream, sp, P,
                            1, din, dout, err);
       else
         xy_class<T, 48>(L, sp, P, 1, din, dout, err);
@@ -550,21 +550,21 @@ void redist_all(const Launch& L, int part, const SimParams& sp, const PlanDev& P
     if (in(3)) xy_class<T, 96>(L, sp, P, 3, din, dout, err);
   } else {
     if (in(0))
-      hipLaunchKernelGGL((k_redist_z_reg<T, 32>), dim3(tile_grid(L, kGridPerCU, 0)), dim3(64), 0, L.stream, sp, P, 0,
+      hipLaunchKernelGGL((k_redist_z_reg<T, 32>), dim3(tile_grid(L, kGridPerCU, 0, sp.N, cols_of(0))), dim3(64), 0, L.stream, sp, P, 0,
                          din, dout);
     if (in(1)) {
       if constexpr (reg48)
-        hipLaunchKernelGGL((k_redist_z_reg<T, 48>), dim3(tile_grid(L, kGridPerCU, 1)), dim3(64), 0, L.stream, sp, P, 1,
+        hipLaunchKernelGGL((k_redist_z_reg<T, 48>), dim3(tile_grid(L, kGridPerCU, 1, sp.N, cols_of(1))), dim3(64), 0, L.stream, sp, P, 1,
                            din, dout);
       else
-        hipLaunchKernelGGL((k_redist_z<T, 48>), dim3(tile_grid(L, kGridPerCU, 1)), dim3(64), 0, L.stream, sp, P, 1,
+        hipLaunchKernelGGL((k_redist_z<T, 48>), dim3(tile_grid(L, kGridPerCU, 1, sp.N, cols_of(1))), dim3(64), 0, L.stream, sp, P, 1,
                            din, dout);
     }
     if (in(2))
-      hipLaunchKernelGGL((k_redist_z<T, 64>), dim3(tile_grid(L, kGridPerCU, 2)), dim3(64), 0, L.stream, sp, P, 2, din,
+      hipLaunchKernelGGL((k_redist_z<T, 64>), dim3(tile_grid(L, kGridPerCU, 2, sp.N, cols_of(2))), dim3(64), 0, L.stream, sp, P, 2, din,
                          dout);
     if (in(3))
-      hipLaunchKernelGGL((k_redist_z<T, 96>), dim3(tile_grid(L, kGridPerCU, 3)), dim3(64), 0, L.stream, sp, P, 3, din,
+      hipLaunchKernelGGL((k_redist_z<T, 96>), dim3(tile_grid(L, kGridPerCU, 3, sp.N, cols_of(3))), dim3(64), 0, L.stream, sp, P, 3, din,
                          dout);
   }
 }
