@@ -26,6 +26,10 @@ constexpr int kScratchDevices = 64;
 static std::mutex g_scratch_mu[kScratchDevices];          // one call at a time per GPU
 static int32_t* g_scratch_ptr[kScratchDevices] = {};      // device address of scratch, per GPU
 
+constexpr int kSides = 3;  // with the main stream, the four hardware queues a process gets
+// bytes of a distance arena (twice the first boxes') between which every size class gets a branch
+constexpr int64_t kBranchMin = 100000000, kBranchMax = 400000000;
+
 struct gg_ctx {
   gg_params p{};
   SimParams sp{};
@@ -92,9 +96,9 @@ struct gg_ctx {
   const int32_t* graph_plan = nullptr;  // c->P.grains when the graph was captured
   // stage timing
   bool timing = false;
-  // second stream for the list build, which runs beside the convolution
-  hipStream_t side = nullptr;
-  hipEvent_t ev_fork = nullptr, ev_join = nullptr;
+  // streams beside the main one: size classes touch disjoint grains and run side by side
+  hipStream_t side[kSides] = {};
+  hipEvent_t ev_fork = nullptr, ev_join[kSides] = {};
   hipEvent_t ev[12] = {};
   double seg_ms[GG_NUM_SEGMENTS] = {};
   int64_t seg_n[GG_NUM_SEGMENTS] = {};
@@ -347,22 +351,93 @@ int conv_mode(const gg_ctx* c) {
 }
 
 // ---- stages (each enqueues its kernels on the context stream) -------------
-void stage_convolution(gg_ctx* c) {
-  Launch L = launch_of(c);
-  { SegTimer t(c, kSegConvA); launch_conv(L, 0, c->sp, c->P, din(c), dout(c), c->TB, c->d_spec_off, c->d_spec, conv_mode(c)); }
-  { SegTimer t(c, kSegConvB); launch_conv(L, 1, c->sp, c->P, din(c), dout(c), c->TB, c->d_spec_off, c->d_spec, conv_mode(c)); }
-  if (!c->fp32) {
-    SegTimer t(c, kSegConvC);
-    launch_conv(L, 2, c->sp, c->P, din(c), dout(c), c->TB, c->d_spec_off, c->d_spec, conv_mode(c));
+// Work beside the main stream: side streams start after what is enqueued on
+// the main stream so far, and the main stream goes on after all of them
+// (parallel branches of a captured step graph).
+//
+// A branch per size class where that pays: below a full GPU's worth of voxels a
+// launch leaves much of the chip idle, and a launch of a class without grains
+// still takes about 4 us, so the classes run side by side; the correction has
+// long tails at any size.  Per step, classes one after another and as branches:
+// 77 grains of side 45 to 80, FP64: 1.95 and 1.72 ms; 343 grains, FP64,
+// correction: 2.52 and 2.24; 512 grains, FP64: 0.98 and 0.88; 4000 grains, FP32,
+// correction: 14.8 and 14.1.  Elsewhere only the list build, the n <= 32
+// comparison and the hull leave the main stream: more voxels fill the GPU launch
+// by launch (8000 grains, FP32: 8.11 and 8.24), and where a step is short the
+// forks cost more than they overlap, on the device and, eager, on the host (27
+// grains: 0.35 and 0.38; 2000 grains, FP32, eager: 4 % slower).
+int sides_of(const gg_ctx* c) {
+  const int64_t bytes = c->arena_cap * (int64_t)c->esz;
+  const bool many = bytes >= kBranchMin && (c->corr_on || (!c->fp32 && bytes <= kBranchMax));
+  return many ? kSides : 1;
+}
+void fork_sides(gg_ctx* c) {
+  hipEventRecord(c->ev_fork, c->stream);
+  for (int i = 0; i < sides_of(c); ++i) hipStreamWaitEvent(c->side[i], c->ev_fork, 0);
+}
+void join_sides(gg_ctx* c) {
+  for (int i = 0; i < sides_of(c); ++i) {
+    hipEventRecord(c->ev_join[i], c->side[i]);
+    hipStreamWaitEvent(c->stream, c->ev_join[i], 0);
   }
-  { SegTimer t(c, kSegIdl); launch_idl_resize(L, c->sp, c->d_state, dout(c), c->IL[c->il_cur ^ 1]); }
+}
+// Branch b (0: the main stream; 1..3: side streams, all the first where there
+// is one only).
+Launch branch(gg_ctx* c, int b) {
+  Launch L = launch_of(c);
+  if (b > 0) L.stream = c->side[sides_of(c) == 1 ? 0 : b - 1];
+  return L;
+}
+// The branch of a size class in the convolution and the redistancing: the
+// n <= 48 class, usually the longest, stays on the main stream.
+Launch launch_of_class(gg_ctx* c, int cls) {
+  static const int b[kClasses] = {1, 0, 2, 3};
+  return branch(c, sides_of(c) == 1 ? 0 : b[cls]);
+}
+
+// The convolution of classes [c0, c1): its passes, then the correction.
+void enqueue_convolution(gg_ctx* c, const Launch& L, int c0, int c1) {
+  const int parts = c->fp32 ? 2 : 3;
+  for (int part = 0; part < parts; ++part) {
+    SegTimer t(c, kSegConvA + part);
+    launch_conv(L, part, c->sp, c->P, din(c), dout(c), c->TB, c->d_spec_off, c->d_spec, conv_mode(c), c0, c1);
+  }
   if (c->corr_on) {
     // IL[il_cur] holds the last comparison's IDLocal, read as its resize to
     // the output bounds leaves it
     SegTimer t(c, kSegCorrect);
-    launch_correction(L, c->sp, c->P, c->d_state, din(c), dout(c), c->IL[c->il_cur], c->topo, corr_args(c),
-                      c->fp32);
+    launch_correction(L, c->sp, c->P, c->d_state, din(c), dout(c), c->IL[c->il_cur], c->topo, corr_args(c), c->fp32,
+                      c0, c1);
   }
+}
+
+// lists: the list build and the comparison's neighbour table (in spatial order
+// its work list too) run beside the convolution, as in a timestep.  The list
+// build reads the state, the box bounds and the current lists and writes the
+// other list buffer and the set-comparison start bounds; the convolution reads
+// and writes distance values only.  The work list needs the plan and the input
+// bounds, which the convolution leaves alone.
+void stage_convolution(gg_ctx* c, bool lists = false) {
+  if (c->timing) {
+    enqueue_convolution(c, launch_of(c), 0, kClasses);
+    SegTimer t(c, kSegIdl);
+    launch_idl_resize(launch_of(c), c->sp, c->d_state, dout(c), c->IL[c->il_cur ^ 1]);
+    return;
+  }
+  fork_sides(c);
+  const Launch S = branch(c, 3);
+  if (lists) {
+    // the roles after the switch that follows the convolution
+    launch_lists(S, c->sp, c->d_state, dout(c), din(c), c->LD, c->d_newb, c->d_err);
+    launch_comparison_table(S, c->sp, c->d_state, dout(c), c->LD);
+    if (c->cmp_order == GG_CMP_ORDER_SPACE)
+      launch_comparison_space(S, c->cmp_space_shape, c->sp, c->P, dout(c), din(c), c->LD, c->IL[c->il_cur],
+                              c->IL[c->il_cur ^ 1], c->d_newb, c->W, c->d_err, c->fp32, kSpaceBuild);
+    c->cmp_prebuilt = true;
+  }
+  for (int cls = kClasses - 1; cls >= 0; --cls) enqueue_convolution(c, launch_of_class(c, cls), cls, cls + 1);
+  launch_idl_resize(branch(c, 2), c->sp, c->d_state, dout(c), c->IL[c->il_cur ^ 1]);
+  join_sides(c);
 }
 
 void stage_lists(gg_ctx* c) {
@@ -372,59 +447,48 @@ void stage_lists(gg_ctx* c) {
 
 void stage_comparison(gg_ctx* c) {
   static const int seg[kClasses] = {kSegCompare, kSegCompare48, kSegCompare64, kSegCompare96};
+  auto one_class = [&](const Launch& L, int cls) {
+    launch_comparison(L, cls, c->cmp_variant[cls], c->sp, c->P, din(c), dout(c), c->LD, c->IL[c->il_cur],
+                      c->IL[c->il_cur ^ 1], c->d_newb, c->fp32);
+  };
   if (c->cmp_order == GG_CMP_ORDER_SPACE) {
     SegTimer t(c, kSegCompare);
     if (!c->cmp_prebuilt) launch_comparison_table(launch_of(c), c->sp, c->d_state, din(c), c->LD);
     launch_comparison_space(launch_of(c), c->cmp_space_shape, c->sp, c->P, din(c), dout(c), c->LD,
                             c->IL[c->il_cur], c->IL[c->il_cur ^ 1], c->d_newb, c->W, c->d_err, c->fp32,
                             c->cmp_prebuilt ? kSpaceRun : kSpaceAll);
-    c->cmp_prebuilt = false;
   } else if (c->timing) {
     for (int cls = 0; cls < kClasses; ++cls) {
       SegTimer t(c, seg[cls]);
       // the first class's segment includes building the neighbour table
       if (cls == 0) launch_comparison_table(launch_of(c), c->sp, c->d_state, din(c), c->LD);
-      launch_comparison(launch_of(c), cls, c->cmp_variant[cls], c->sp, c->P, din(c), dout(c), c->LD, c->IL[c->il_cur],
-                        c->IL[c->il_cur ^ 1], c->d_newb, c->fp32);
+      one_class(launch_of(c), cls);
     }
   } else {
     // The size classes touch disjoint grains (their bounding-box atomics and
-    // IDLocal rows included), so the n <= 32 class runs on the side stream
-    // beside the others; each launch's tail then overlaps the other's work.
-    launch_comparison_table(launch_of(c), c->sp, c->d_state, din(c), c->LD);
-    hipEventRecord(c->ev_fork, c->stream);
-    hipStreamWaitEvent(c->side, c->ev_fork, 0);
-    Launch S = launch_of(c);
-    S.stream = c->side;
-    launch_comparison(S, 0, c->cmp_variant[0], c->sp, c->P, din(c), dout(c), c->LD, c->IL[c->il_cur], c->IL[c->il_cur ^ 1], c->d_newb,
-                      c->fp32);
-    hipEventRecord(c->ev_join, c->side);
-    for (int cls = 1; cls < kClasses; ++cls)
-      launch_comparison(launch_of(c), cls, c->cmp_variant[cls], c->sp, c->P, din(c), dout(c), c->LD, c->IL[c->il_cur],
-                        c->IL[c->il_cur ^ 1], c->d_newb, c->fp32);
-    hipStreamWaitEvent(c->stream, c->ev_join, 0);
+    // IDLocal rows included).
+    if (!c->cmp_prebuilt) launch_comparison_table(launch_of(c), c->sp, c->d_state, din(c), c->LD);
+    fork_sides(c);
+    one_class(branch(c, 1), 0);
+    one_class(branch(c, 0), 1);
+    one_class(branch(c, sides_of(c) == 1 ? 0 : 2), 2);
+    one_class(branch(c, sides_of(c) == 1 ? 0 : 3), 3);
+    join_sides(c);
   }
+  c->cmp_prebuilt = false;
   c->il_cur ^= 1;
 }
 
-// Runs launch(L, c0, c1) over the size classes: outside stage timing the
-// n <= 32 class goes on the side stream beside the others (classes touch
-// disjoint grains), forked from and joined back to the main stream.
+// Runs launch(L, c0, c1) over the size classes, outside stage timing as branches.
 template <class F>
 void over_classes(gg_ctx* c, F launch) {
-  Launch L = launch_of(c);
   if (c->timing) {
-    launch(L, 0, kClasses);
+    launch(launch_of(c), 0, kClasses);
     return;
   }
-  hipEventRecord(c->ev_fork, c->stream);
-  hipStreamWaitEvent(c->side, c->ev_fork, 0);
-  Launch S = L;
-  S.stream = c->side;
-  launch(S, 0, 1);
-  hipEventRecord(c->ev_join, c->side);
-  launch(L, 1, kClasses);
-  hipStreamWaitEvent(c->stream, c->ev_join, 0);
+  fork_sides(c);
+  for (int cls = kClasses - 1; cls >= 0; --cls) launch(launch_of_class(c, cls), cls, cls + 1);
+  join_sides(c);
 }
 
 // Level set, first part: the output boxes (they follow from the
@@ -466,12 +530,17 @@ void stage_level_set(gg_ctx* c) {
 }
 
 void redist_parts(gg_ctx* c) {
-  for (int part = 0; part < 2; ++part) {
-    SegTimer t(c, part == 0 ? kSegRedistXY : kSegRedistZ);
-    over_classes(c, [&](const Launch& LL, int c0, int c1) {
-      launch_redist(LL, part, c->sp, c->P2, din(c), dout(c), c->d_err, c->fp32, c0, c1);
-    });
+  if (c->timing) {
+    for (int part = 0; part < 2; ++part) {
+      SegTimer t(c, part == 0 ? kSegRedistXY : kSegRedistZ);
+      launch_redist(launch_of(c), part, c->sp, c->P2, din(c), dout(c), c->d_err, c->fp32);
+    }
+    return;
   }
+  over_classes(c, [&](const Launch& L, int c0, int c1) {
+    for (int part = 0; part < 2; ++part)
+      launch_redist(L, part, c->sp, c->P2, din(c), dout(c), c->d_err, c->fp32, c0, c1);
+  });
 }
 
 // The redistancing over the output plan, then the input role takes the output
@@ -483,11 +552,12 @@ void stage_redistancing(gg_ctx* c) {
   c->p2_valid = false;
 }
 
-// Level set and redistancing of one timestep with the hull on the side stream
-// beside the redistancing: the hull reads the input role and IDLocal, the
-// redistancing reads the input role and writes the output role, and the
-// existence, volume and area finish after both.  The post-redistancing resize
-// follows the deletion marks, as in the stage-by-stage order.
+// Level set and redistancing of one timestep, the hull beside the
+// redistancing: the hull reads the input role and IDLocal, the redistancing
+// reads the input role and writes the output role, and the existence, volume
+// and area finish after both.  The post-redistancing resize follows the
+// deletion marks, as in the stage-by-stage order.  The hull's classes go on
+// the branches whose redistancing is usually short.
 void stage_level_set_and_redistancing(gg_ctx* c) {
   if (c->timing) {
     stage_level_set(c);
@@ -497,14 +567,28 @@ void stage_level_set_and_redistancing(gg_ctx* c) {
   Launch L = launch_of(c);
   stage_output_plan(c);
   if (c->topo.on) launch_topo_clear(L, c->sp, c->topo);
-  hipEventRecord(c->ev_fork, c->stream);
-  hipStreamWaitEvent(c->side, c->ev_fork, 0);
-  Launch S = L;
-  S.stream = c->side;
-  launch_hull(S, c->sp, c->P, din(c), c->d_exflag, c->d_partials, c->IL[c->il_cur], c->topo, c->d_err, c->fp32);
-  hipEventRecord(c->ev_join, c->side);
-  for (int part = 0; part < 2; ++part) launch_redist(L, part, c->sp, c->P2, din(c), dout(c), c->d_err, c->fp32);
-  hipStreamWaitEvent(c->stream, c->ev_join, 0);
+  fork_sides(c);
+  auto hull = [&](int b, int cls) {
+    launch_hull(branch(c, b), c->sp, c->P, din(c), c->d_exflag, c->d_partials, c->IL[c->il_cur], c->topo, c->d_err,
+                c->fp32, cls, cls + 1);
+  };
+  auto redist = [&](int cls) {
+    for (int part = 0; part < 2; ++part)
+      launch_redist(launch_of_class(c, cls), part, c->sp, c->P2, din(c), dout(c), c->d_err, c->fp32, cls, cls + 1);
+  };
+  // The long launches start first on their branches: side 1 redistances the
+  // n <= 32 class and both do the n <= 96 class, side 2 redistances the n <= 64
+  // class before the hull of n <= 48, side 3 has the other hulls.
+  if (sides_of(c) > 1) redist(2);
+  hull(3, 2);
+  hull(3, 0);
+  hull(2, 1);
+  redist(0);
+  redist(1);
+  if (sides_of(c) == 1) redist(2);
+  hull(1, 3);
+  redist(3);
+  join_sides(c);
   stage_finalize_state(c);
   stage_elements(c);
   launch_post_redist(L, c->sp, c->d_state, din(c), dout(c));
@@ -525,28 +609,8 @@ void enqueue_step(gg_ctx* c) {
     c->sel ^= 1;
     stage_lists(c);
   } else {
-    // The list build reads the state, the box bounds and the current lists and
-    // writes the other list buffer and the set-comparison start bounds; the
-    // convolution reads and writes distance values and IDLocal bounds only. So
-    // the lists go on the side stream, forked from and joined back to the main
-    // stream (inside a captured graph too), beside the convolution.  In spatial
-    // order the comparison's neighbour table (from the new lists) and its work
-    // list (from the plan and the input bounds, which the convolution leaves
-    // alone) follow them there.
-    hipEventRecord(c->ev_fork, c->stream);
-    hipStreamWaitEvent(c->side, c->ev_fork, 0);
-    const Launch S{c->side, c->grid, c->grid / 8};
-    launch_lists(S, c->sp, c->d_state, dout(c), din(c), c->LD, c->d_newb, c->d_err);  // the roles after the switch below
-    if (c->cmp_order == GG_CMP_ORDER_SPACE) {
-      launch_comparison_table(S, c->sp, c->d_state, dout(c), c->LD);
-      launch_comparison_space(S, c->cmp_space_shape, c->sp, c->P, dout(c), din(c), c->LD, c->IL[c->il_cur],
-                              c->IL[c->il_cur ^ 1], c->d_newb, c->W, c->d_err, c->fp32, kSpaceBuild);
-      c->cmp_prebuilt = true;
-    }
-    hipEventRecord(c->ev_join, c->side);
-    stage_convolution(c);
+    stage_convolution(c, true);
     c->sel ^= 1;
-    hipStreamWaitEvent(c->stream, c->ev_join, 0);
   }
   stage_comparison(c);
   c->sel ^= 1;
@@ -582,9 +646,11 @@ int gg_create(const gg_params* params, gg_ctx** out) {
     delete c;
     return GG_ERR_HIP;
   }
-  if (hipStreamCreateWithFlags(&c->side, hipStreamNonBlocking) != hipSuccess ||
-      hipEventCreateWithFlags(&c->ev_fork, hipEventDisableTiming) != hipSuccess ||
-      hipEventCreateWithFlags(&c->ev_join, hipEventDisableTiming) != hipSuccess) {
+  bool made = hipEventCreateWithFlags(&c->ev_fork, hipEventDisableTiming) == hipSuccess;
+  for (int i = 0; i < kSides; ++i)
+    made = made && hipStreamCreateWithFlags(&c->side[i], hipStreamNonBlocking) == hipSuccess &&
+           hipEventCreateWithFlags(&c->ev_join[i], hipEventDisableTiming) == hipSuccess;
+  if (!made) {
     gg_destroy(c);
     return GG_ERR_HIP;
   }
@@ -691,8 +757,10 @@ int gg_destroy(gg_ctx* c) {
   for (auto e : c->evpool) hipEventDestroy(e);
   for (void* p : c->allocs) hipFree(p);
   if (c->ev_fork) hipEventDestroy(c->ev_fork);
-  if (c->ev_join) hipEventDestroy(c->ev_join);
-  if (c->side) hipStreamDestroy(c->side);
+  for (int i = 0; i < kSides; ++i) {
+    if (c->ev_join[i]) hipEventDestroy(c->ev_join[i]);
+    if (c->side[i]) hipStreamDestroy(c->side[i]);
+  }
   if (c->stream) hipStreamDestroy(c->stream);
   delete c;
   return GG_OK;
@@ -958,7 +1026,7 @@ int gg_coarsen_grid(gg_ctx* c, int32_t new_size, double new_dt) {
   // once the work queued before this call is done); a captured step graph
   // holds the old grid in its kernel arguments
   HIPCHK(c, hipStreamSynchronize(c->stream));
-  HIPCHK(c, hipStreamSynchronize(c->side));
+  for (int i = 0; i < kSides; ++i) HIPCHK(c, hipStreamSynchronize(c->side[i]));
   const TablesDev old_tb = c->TB;
   if ((rc = build_tables(c))) return rc;
   for (const void* q : {(const void*)old_tb.tw_off, (const void*)old_tb.twc, (const void*)old_tb.tws,
@@ -1383,7 +1451,7 @@ int gg_set_physics(gg_ctx* c, const gg_physics* ph, const double* quat, const do
   if (rc) return rc;
   hipSetDevice(c->p.device);
   HIPCHK(c, hipStreamSynchronize(c->stream));
-  HIPCHK(c, hipStreamSynchronize(c->side));
+  for (int i = 0; i < kSides; ++i) HIPCHK(c, hipStreamSynchronize(c->side[i]));
   drop_graph(c);  // kernel arguments change
   const int N = c->p.n_grains;
   if (!ph->correction) {

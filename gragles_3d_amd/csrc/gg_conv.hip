@@ -725,11 +725,12 @@ void conv_class(const Launch& L, int part, const SimParams& sp, const PlanDev& P
 }  // namespace
 
 void launch_conv(const Launch& L, int part, const SimParams& sp, const PlanDev& P, const DescDev& din,
-                 const DescDev& dout, const TablesDev& tb, const int64_t* spec_off, void* spec, int mode) {
-  conv_class<32>(L, part, sp, P, 0, din, dout, tb, spec_off, spec, mode);
-  conv_class<48>(L, part, sp, P, 1, din, dout, tb, spec_off, spec, mode);
-  conv_class<64>(L, part, sp, P, 2, din, dout, tb, spec_off, spec, mode);
-  conv_class<96>(L, part, sp, P, 3, din, dout, tb, spec_off, spec, mode);
+                 const DescDev& dout, const TablesDev& tb, const int64_t* spec_off, void* spec, int mode, int c0,
+                 int c1) {
+  if (c0 <= 0 && 0 < c1) conv_class<32>(L, part, sp, P, 0, din, dout, tb, spec_off, spec, mode);
+  if (c0 <= 1 && 1 < c1) conv_class<48>(L, part, sp, P, 1, din, dout, tb, spec_off, spec, mode);
+  if (c0 <= 2 && 2 < c1) conv_class<64>(L, part, sp, P, 2, din, dout, tb, spec_off, spec, mode);
+  if (c0 <= 3 && 3 < c1) conv_class<96>(L, part, sp, P, 3, din, dout, tb, spec_off, spec, mode);
 }
 
 }  // namespace gg

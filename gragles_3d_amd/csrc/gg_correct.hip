@@ -923,14 +923,18 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4))) void k
 
 template <class T>
 void correct_classes(const Launch& L, const SimParams& sp, const PlanDev& P, const int32_t* state, const DescDev& din,
-                     const DescDev& dout, const IdlDev& il, const TopoDev& topo, const CorrDev& cd) {
-  hipLaunchKernelGGL((k_correct<T, 32, 4>), dim3(tile_grid(L, kCorrGridPerCU, 0, sp.N, layers_of(0))), dim3(256), 0, L.stream, sp, P, 0,
+                     const DescDev& dout, const IdlDev& il, const TopoDev& topo, const CorrDev& cd, int c0, int c1) {
+  if (c0 <= 0 && 0 < c1)
+    hipLaunchKernelGGL((k_correct<T, 32, 4>), dim3(tile_grid(L, kCorrGridPerCU, 0, sp.N, layers_of(0))), dim3(256), 0, L.stream, sp, P, 0,
                      state, din, dout, il, topo, cd);
-  hipLaunchKernelGGL((k_correct<T, 48, 4>), dim3(tile_grid(L, kCorrGridPerCU, 1, sp.N, layers_of(1))), dim3(256), 0, L.stream, sp, P, 1,
+  if (c0 <= 1 && 1 < c1)
+    hipLaunchKernelGGL((k_correct<T, 48, 4>), dim3(tile_grid(L, kCorrGridPerCU, 1, sp.N, layers_of(1))), dim3(256), 0, L.stream, sp, P, 1,
                      state, din, dout, il, topo, cd);
-  hipLaunchKernelGGL((k_correct<T, 64, 2>), dim3(tile_grid(L, kCorrGridPerCU, 2, sp.N, layers_of(2))), dim3(256), 0, L.stream, sp, P, 2,
+  if (c0 <= 2 && 2 < c1)
+    hipLaunchKernelGGL((k_correct<T, 64, 2>), dim3(tile_grid(L, kCorrGridPerCU, 2, sp.N, layers_of(2))), dim3(256), 0, L.stream, sp, P, 2,
                      state, din, dout, il, topo, cd);
-  hipLaunchKernelGGL((k_correct<T, 96, 1>), dim3(tile_grid(L, kCorrGridPerCU, 3, sp.N, layers_of(3))), dim3(256), 0, L.stream, sp, P, 3,
+  if (c0 <= 3 && 3 < c1)
+    hipLaunchKernelGGL((k_correct<T, 96, 1>), dim3(tile_grid(L, kCorrGridPerCU, 3, sp.N, layers_of(3))), dim3(256), 0, L.stream, sp, P, 3,
                      state, din, dout, il, topo, cd);
 }
 
@@ -947,9 +951,9 @@ void launch_elements(const Launch& L, const SimParams& sp, const int32_t* state,
 
 void launch_correction(const Launch& L, const SimParams& sp, const PlanDev& P, const int32_t* state,
                        const DescDev& din, const DescDev& dout, const IdlDev& il_stale, const TopoDev& topo,
-                       const CorrDev& cd, bool fp32) {
-  if (fp32) correct_classes<float>(L, sp, P, state, din, dout, il_stale, topo, cd);
-  else correct_classes<double>(L, sp, P, state, din, dout, il_stale, topo, cd);
+                       const CorrDev& cd, bool fp32, int c0, int c1) {
+  if (fp32) correct_classes<float>(L, sp, P, state, din, dout, il_stale, topo, cd, c0, c1);
+  else correct_classes<double>(L, sp, P, state, din, dout, il_stale, topo, cd, c0, c1);
 }
 
 }  // namespace gg

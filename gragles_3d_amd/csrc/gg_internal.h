@@ -380,7 +380,8 @@ void launch_init_phi(const Launch& L, const SimParams& sp, const PlanDev& P, con
 // convolution forms: the FP64 FFT, the FP32 circulant, the split-BF16 circulant
 enum { kConvFFT64 = 0, kConvCirculantF32 = 1, kConvSplitBF16 = 2 };
 void launch_conv(const Launch& L, int part, const SimParams& sp, const PlanDev& P, const DescDev& din,
-                 const DescDev& dout, const TablesDev& tb, const int64_t* spec_off, void* spec, int mode);
+                 const DescDev& dout, const TablesDev& tb, const int64_t* spec_off, void* spec, int mode, int c0 = 0,
+                 int c1 = kClasses);
 void launch_idl_resize(const Launch& L, const SimParams& sp, const int32_t* state, const DescDev& dout,
                        const IdlDev& il);
 void launch_init_lists(const Launch& L, const SimParams& sp, const int32_t* state, const DescDev& d,
@@ -446,5 +447,5 @@ void launch_elements(const Launch& L, const SimParams& sp, const int32_t* state,
                      const TopoDev& topo, const CorrDev& cd, int32_t* err);
 void launch_correction(const Launch& L, const SimParams& sp, const PlanDev& P, const int32_t* state,
                        const DescDev& din, const DescDev& dout, const IdlDev& il_stale, const TopoDev& topo,
-                       const CorrDev& cd, bool fp32);
+                       const CorrDev& cd, bool fp32, int c0 = 0, int c1 = kClasses);
 }  // namespace gg
