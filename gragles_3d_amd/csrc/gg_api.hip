@@ -508,11 +508,9 @@ void stage_output_plan(gg_ctx* c) {
 
 void stage_hull(gg_ctx* c) {
   SegTimer t(c, kSegHull);
-  if (c->topo.on) launch_topo_clear(launch_of(c), c->sp, c->topo);
-  over_classes(c, [&](const Launch& LL, int c0, int c1) {
-    launch_hull(LL, c->sp, c->P, din(c), c->d_exflag, c->d_partials, c->IL[c->il_cur], c->topo, c->d_err, c->fp32,
-                c0, c1);
-  });
+  if (c->topo.on) launch_topo_clear(launch_of(c), c->sp, c->P, c->topo);
+  launch_hull(launch_of(c), c->sp, c->P, din(c), c->d_exflag, c->d_partials, c->IL[c->il_cur], c->topo, c->d_err,
+              c->fp32);
 }
 
 // Level set, last part: deletion, list flip, existence, volume and area.
@@ -556,8 +554,7 @@ void stage_redistancing(gg_ctx* c) {
 // redistancing: the hull reads the input role and IDLocal, the redistancing
 // reads the input role and writes the output role, and the existence, volume
 // and area finish after both.  The post-redistancing resize follows the
-// deletion marks, as in the stage-by-stage order.  The hull's classes go on
-// the branches whose redistancing is usually short.
+// deletion marks, as in the stage-by-stage order. 
 void stage_level_set_and_redistancing(gg_ctx* c) {
   if (c->timing) {
     stage_level_set(c);
@@ -566,28 +563,14 @@ void stage_level_set_and_redistancing(gg_ctx* c) {
   }
   Launch L = launch_of(c);
   stage_output_plan(c);
-  if (c->topo.on) launch_topo_clear(L, c->sp, c->topo);
+  if (c->topo.on) launch_topo_clear(L, c->sp, c->P, c->topo);
   fork_sides(c);
-  auto hull = [&](int b, int cls) {
-    launch_hull(branch(c, b), c->sp, c->P, din(c), c->d_exflag, c->d_partials, c->IL[c->il_cur], c->topo, c->d_err,
-                c->fp32, cls, cls + 1);
-  };
-  auto redist = [&](int cls) {
+  launch_hull(branch(c, 3), c->sp, c->P, din(c), c->d_exflag, c->d_partials, c->IL[c->il_cur], c->topo, c->d_err,
+              c->fp32);
+  for (int cls : {2, 0, 1, 3})
     for (int part = 0; part < 2; ++part)
-      launch_redist(launch_of_class(c, cls), part, c->sp, c->P2, din(c), dout(c), c->d_err, c->fp32, cls, cls + 1);
-  };
-  // The long launches start first on their branches: side 1 redistances the
-  // n <= 32 class and both do the n <= 96 class, side 2 redistances the n <= 64
-  // class before the hull of n <= 48, side 3 has the other hulls.
-  if (sides_of(c) > 1) redist(2);
-  hull(3, 2);
-  hull(3, 0);
-  hull(2, 1);
-  redist(0);
-  redist(1);
-  if (sides_of(c) == 1) redist(2);
-  hull(1, 3);
-  redist(3);
+      launch_redist(branch(c, sides_of(c) == 1 ? 0 : cls == 3 ? 1 : cls == 1 ? 0 : cls == 0 ? 1 : 2), part, c->sp,
+                    c->P2, din(c), dout(c), c->d_err, c->fp32, cls, cls + 1);
   join_sides(c);
   stage_finalize_state(c);
   stage_elements(c);
@@ -1055,7 +1038,7 @@ int gg_coarsen_grid(gg_ctx* c, int32_t new_size, double new_dt) {
                       c->d_newb, c->fp32);
   c->il_cur ^= 1;
   // extractContour on the resampled input buffer
-  if (c->topo.on) launch_topo_clear(L, c->sp, c->topo);
+  if (c->topo.on) launch_topo_clear(L, c->sp, c->P, c->topo);
   launch_hull(L, c->sp, c->P, din(c), c->d_exflag, c->d_partials, c->IL[c->il_cur], c->topo, c->d_err, c->fp32);
   launch_finalize(L, c->sp, c->P, c->d_state, c->LD, c->d_exflag, c->d_partials, c->d_cnb, din(c), dout(c),
                   c->d_volume, c->d_area, kFinBounds | kFinState | kFinCoarsen);

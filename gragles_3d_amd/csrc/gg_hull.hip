@@ -3,22 +3,22 @@
 // the box resize (grainhdl::level_set, src/grainhdl.cpp:669-684 ->
 // LSbox::extractContour, src/box.cpp:1144-1161).
 //
-// k_hull walks the cells of one z-layer of a grain's input box exactly as
+// The hull kernels walk the cells of a grain's input box as
 // MarchingCubesAlgorithm::generateHull (src/marchingCubes.cpp:364-478): case
 // index from the eight corners (inside = phi >= 0), VertexInterp
 // (:484-499) on the cut edges, triangles from the case table, then the
 // signed-tetrahedron volume term (src/grainHull.cpp:40-56, including its
 // float(1/6) factor) and the triangle area (:120-131).  A grain exists iff
-// some cell is cut.  Each tile keeps Neumaier-compensated FP64 sums and writes
-// them to its own slot; k_finalize adds a grain's slots in layer order, so the
-// result does not depend on scheduling.
+// some cell is cut.  Neumaier-compensated FP64 sums go to fixed slots of the
+// grain's layers, and k_finalize adds them in layer order, so the result does
+// not depend on scheduling.
 #include <algorithm>
 
 #include "gg_internal.h"
 
 namespace gg {
 namespace {
-constexpr int kGridPerCU = 64;  // workgroups per CU of a hull launch (each loads the triangle table once)
+constexpr int kGridPerCU = 64;  // most workgroups per CU of a hull launch (each loads the triangle table once)
 #include "mc_cases.inc"
 
 // Triangle table row of each case: edge indices in nibbles, first triangle in
@@ -49,529 +49,651 @@ struct Acc {
   }
 };
 
-constexpr int kHT = 256;
-constexpr int kTopoLdsBits = 7, kTopoLds = 1 << kTopoLdsBits;  // per-tile topology table
 constexpr int kTopoCapBits = 6;
 static_assert((1 << kTopoCapBits) == kTopoCap, "grain topology table size");
 static_assert(kTopoCap <= 64, "a junction list is a 64-bit mask over the grain table's slots");
-constexpr int kJuncLdsBits = 8, kJuncLds = 1 << kJuncLdsBits;  // per-tile junction table
 constexpr int kJuncCapBits = 9;
 static_assert((1 << kJuncCapBits) == kJuncCap, "grain junction table size");
-constexpr int kCPT = 4;              // cells classified per lane and pass (a 4 KiB queue: six workgroups per CU)
-constexpr int kChunk = kCPT * kHT;  // cells classified per pass
 
-// Offset of corner q of the cell (xl, yl) in the two staged layers L[0..2*NMAX^2).
-template <int NMAX>
-__device__ inline int corner_off(int q, int xl, int yl, int n) {
-  return (int)((kCornerZ >> q) & 1u) * (NMAX * NMAX) + (yl + (int)((kCornerY >> q) & 1u)) * n + xl +
-         (int)((kCornerX >> q) & 1u);
+// Cells are found from sign bits.  A wavefront loads a run of layers (one
+// contiguous stretch of the box) in pieces of 64 voxels and keeps the ballot of
+// phi >= 0 of each as one 64-bit word in LDS; a lane takes a row of cells (rows
+// of more than 63 in two parts), shifts out the bits of its four corner rows and
+// gets the row's cut cells (some corners inside, some outside) as one mask.  Most
+// rows have none, and no corner value is read for a cell that is not cut.  Cut
+// cells are queued and worked on 64 at a time, their corner values read again
+// from the layers (cached).
+constexpr int kHullAhead = 8;  // loads in flight
+
+// An entry of a cell queue: x | y << 7 | layer << 14 (| case << 21).
+__device__ inline uint32_t cell_entry(int x, int y, int k) {
+  return (uint32_t)x | (uint32_t)y << 7 | (uint32_t)k << 14;
 }
 
-// VertexInterp (src/marchingCubes.cpp:484-499) at iso level 0 on cube edge e of
-// the cell with lower corner (x,y,z); the corner values come from LDS.
-template <class T, int NMAX>
-__device__ inline void edge_vertex(int e, const T* L, int xl, int yl, int n, int x, int y, int z, double& px,
-                                   double& py, double& pz) {
-  const int a = (int)((kEdgeA >> (4 * e)) & 15u), b = (int)((kEdgeB >> (4 * e)) & 15u);
-  const double v1 = (double)L[corner_off<NMAX>(a, xl, yl, n)];
-  const double v2 = (double)L[corner_off<NMAX>(b, xl, yl, n)];
-  const double p1x = x + (int)((kCornerX >> a) & 1u), p1y = y + (int)((kCornerY >> a) & 1u),
-               p1z = z + (int)((kCornerZ >> a) & 1u);
-  const double p2x = x + (int)((kCornerX >> b) & 1u), p2y = y + (int)((kCornerY >> b) & 1u),
-               p2z = z + (int)((kCornerZ >> b) & 1u);
-  if (fabs(v1) < 0.00001) {
-    px = p1x; py = p1y; pz = p1z;
-  } else if (fabs(v2) < 0.00001) {
-    px = p2x; py = p2y; pz = p2z;
-  } else if (fabs(v1 - v2) < 0.00001) {
-    px = p1x; py = p1y; pz = p1z;
-  } else {
-    // An edge runs along one axis, so p2 - p1 is a unit step and only mu is
-    // rounded. The FP32 path takes mu in FP32 (reciprocal, ~2 ulp): the values
-    // it interpolates are FP32 already; the FP64 path divides in FP64.
-    double mu;
-    if constexpr (sizeof(T) == 4) {
-      const float f1 = (float)v1, f2 = (float)v2;
-      mu = (double)(f1 * __builtin_amdgcn_rcpf(f1 - f2));
-    } else {
-      mu = v1 / (v1 - v2);
+// The sign words of count voxels from src on; returns whether any is inside.
+template <class T>
+__device__ inline bool load_words(unsigned long long* w, const T* __restrict__ src, int count, int lane) {
+  const int nw = (count + 63) >> 6;
+  unsigned long long any = 0ull;
+  for (int k0 = 0; k0 < nw; k0 += kHullAhead) {
+    T v[kHullAhead];
+#pragma unroll
+    for (int u = 0; u < kHullAhead; ++u) {
+      const int c = (k0 + u) * 64 + lane;
+      v[u] = c < count ? src[c] : T(-1);
     }
-    px = p1x + mu * (p2x - p1x);
-    py = p1y + mu * (p2y - p1y);
-    pz = p1z + mu * (p2z - p1z);
+    unsigned lo = 0, hi = 0;  // lane u: word k0 + u
+#pragma unroll
+    for (int u = 0; u < kHullAhead; ++u) {
+      const unsigned long long m = __ballot(v[u] >= T(0));
+      any |= m;
+      lo = lane == u ? (unsigned)m : lo;
+      hi = lane == u ? (unsigned)(m >> 32) : hi;
+    }
+    if (lane < kHullAhead && k0 + lane <= nw) w[k0 + lane] = (unsigned long long)hi << 32 | lo;
+  }
+  if (lane == 0 && (nw & (kHullAhead - 1)) == 0) w[nw] = 0ull;  // read past the end by word_bits
+  return any != 0ull;
+}
+
+// 64 bits of the words from bit o on.
+__device__ inline unsigned long long word_bits(const unsigned long long* w, int o) {
+  const int i = o >> 6, sh = o & 63;
+  const unsigned long long lo = w[i] >> sh;
+  return sh ? lo | w[i + 1] << (64 - sh) : lo;
+}
+
+// LDS writes of a wavefront are seen by its later reads in order; this keeps
+// the compiler from moving one past the other.
+__device__ inline void wave_fence() {
+  __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+  __builtin_amdgcn_wave_barrier();
+}
+
+// Queues the cut cells of layers k0 .. k0 + nl - 1 (words of layers k0 .. k0 +
+// nl in w), one per row and round.  push(entry, has) is called by the whole
+// wavefront; CASE: entries with the cell's case index.
+template <bool CASE, class F>
+__device__ inline void cut_cells(const unsigned long long* w, int n, int k0, int nl, int lane, F push) {
+  const int m1 = n - 1;
+  const bool split = m1 > 63;  // rows of more than 63 cells in two parts
+  const int rows = nl * m1, items = split ? 2 * rows : rows;
+  const uint32_t inv = ((1u << 24) + (uint32_t)m1 - 1u) / (uint32_t)m1;  // r / m1 = r * inv >> 24 for r < 96^2
+  for (int i0 = 0; i0 < items; i0 += 64) {
+    const int it = i0 + lane;
+    const bool live = it < items;
+    const int r = live ? (split ? it >> 1 : it) : 0, xs = split && (it & 1) ? 63 : 0;
+    const int kl = (int)(((uint64_t)(uint32_t)r * inv) >> 24), y = r - kl * m1;
+    const int o = (kl * n + y) * n + xs;
+    const unsigned long long m00 = word_bits(w, o), m10 = word_bits(w, o + n), m01 = word_bits(w, o + n * n),
+                             m11 = word_bits(w, o + n * n + n);
+    const unsigned long long any = m00 | m10 | m01 | m11, all = m00 & m10 & m01 & m11;
+    const int width = min(63, m1 - xs);
+    unsigned long long cut = live ? ((any | any >> 1) & ~(all & all >> 1)) & ((1ull << width) - 1ull) : 0ull;
+    const uint32_t base = cell_entry(xs, y, k0 + kl);
+    while (__ballot(cut != 0ull)) {
+      const bool has = cut != 0ull;
+      const int x = has ? (int)__builtin_ctzll(cut) : 0;
+      cut &= cut - 1ull;
+      uint32_t e = base + (uint32_t)x;
+      if constexpr (CASE) {
+        const unsigned a = (unsigned)(m01 >> x) & 3u, b = (unsigned)(m00 >> x) & 3u, c = (unsigned)(m11 >> x) & 3u,
+                       d = (unsigned)(m10 >> x) & 3u;
+        e |= (a | b >> 1 << 2 | (b & 1u) << 3 | c << 4 | d >> 1 << 6 | (d & 1u) << 7) << 21;
+      }
+      push(e, has);
+    }
   }
 }
 
-// One (grain, z-layer) tile: layers kl and kl+1 are staged in LDS; each lane
-// classifies kCPT cells, the triangles of the cut ones (some corners inside,
-// some outside) are listed in a fixed order by one workgroup scan, and then
-// every lane works on one triangle at a time, so the triangle work is neither
-// left to a few lanes of each wavefront nor held up by cells with many
-// triangles.  The triangle table sits in LDS; corner and edge tables are bit
-// masks, so no lookup goes to memory with a lane-dependent address.
-// FP32: six waves per SIMD asked of the compiler, which the LDS of both
-// classes then allows.
+// Corner values of the lane's cell into cv[corner * 64 + lane]; returns its case
+// index (inside: phi >= 0).
+template <class T>
+__device__ inline unsigned stage_corners(T* cv, const T* __restrict__ p, int n, int nn2, int lane) {
+  const T* q = p + nn2;
+  const T v[8] = {q[0], q[1], p[1], p[0], q[n], q[n + 1], p[n + 1], p[n]};
+  unsigned ci = 0;
+#pragma unroll
+  for (int c = 0; c < 8; ++c) {
+    cv[c * 64 + lane] = v[c];
+    ci |= v[c] >= T(0) ? 1u << c : 0u;
+  }
+  return ci;
+}
+
+// Cube edge e as a word: corner a, corner b << 3, the offset of a (x, y, z bits
+// 6..8), the edge's axis as bits 9..11 and bit 12 if b lies below a on it.
+constexpr uint32_t edge_word(int e) {
+  const unsigned a = (unsigned)(kEdgeA >> (4 * e)) & 15u, b = (unsigned)(kEdgeB >> (4 * e)) & 15u;
+  const unsigned ax = (kCornerX >> a) & 1u, ay = (kCornerY >> a) & 1u, az = (kCornerZ >> a) & 1u;
+  const unsigned bx = (kCornerX >> b) & 1u, by = (kCornerY >> b) & 1u, bz = (kCornerZ >> b) & 1u;
+  const unsigned down = (ax & ~bx & 1u) | (ay & ~by & 1u) | (az & ~bz & 1u);
+  return a | b << 3 | ax << 6 | ay << 7 | az << 8 | (ax ^ bx) << 9 | (ay ^ by) << 10 | (az ^ bz) << 11 | down << 12;
+}
+
+// VertexInterp (src/marchingCubes.cpp:484-499) at iso level 0 on the edge of
+// word ew, in the cell with lower corner (x,y,z); the corner values from
+// stage_corners.  An edge runs along one axis, so the vertex is the edge's first
+// corner plus t along it: 0 where the first value is below 1e-5, +-1 where the
+// second is, else +-mu.  (The reference also takes the first corner where the
+// values are within 1e-5 of each other: one is inside and the other outside, so
+// then one of them is below 1e-5.)
+template <class T>
+__device__ inline void edge_vertex(uint32_t ew, const T* cv, int slot, int x, int y, int z, double& px, double& py,
+                                   double& pz) {
+  const T v1 = cv[(ew & 7u) * 64 + slot], v2 = cv[((ew >> 3) & 7u) * 64 + slot];
+  double t;
+  if constexpr (sizeof(T) == 4) {
+    // mu in FP32 (reciprocal, ~2 ulp): the values it interpolates are FP32
+    // already.  |v| <= 1e-5f is |v| < 1e-5 (the float lies just below it).
+    float mu = v1 * __builtin_amdgcn_rcpf(v1 - v2);
+    mu = fabsf(v2) <= 1e-5f ? 1.0f : mu;
+    mu = fabsf(v1) <= 1e-5f ? 0.0f : mu;
+    t = (double)((ew >> 12) & 1u ? -mu : mu);
+  } else {
+    double mu = v1 / (v1 - v2);
+    mu = fabs(v2) < 0.00001 ? 1.0 : mu;
+    mu = fabs(v1) < 0.00001 ? 0.0 : mu;
+    t = (ew >> 12) & 1u ? -mu : mu;
+  }
+  px = (double)(x + (int)((ew >> 6) & 1u)) + ((ew >> 9) & 1u ? t : 0.0);
+  py = (double)(y + (int)((ew >> 7) & 1u)) + ((ew >> 10) & 1u ? t : 0.0);
+  pz = (double)(z + (int)((ew >> 8) & 1u)) + ((ew >> 11) & 1u ? t : 0.0);
+}
+
+struct Tri {
+  double p0x, p0y, p0z, p1x, p1y, p1z, p2x, p2y, p2z;
+  __device__ double volume() const {  // src/grainHull.cpp:40-56
+    const double v321 = p2x * p1y * p0z;
+    const double v231 = p1x * p2y * p0z;
+    const double v312 = p2x * p0y * p1z;
+    const double v132 = p0x * p2y * p1z;
+    const double v213 = p1x * p0y * p2z;
+    const double v123 = p0x * p1y * p2z;
+    return (double)(1.0f / 6.0f) * (-v321 + v231 + v312 - v132 - v213 + v123);
+  }
+  __device__ double area() const {  // src/grainHull.cpp:120-131, src/InterfacialElement.cpp:81-92
+    const double abx = p0x - p1x, aby = p0y - p1y, abz = p0z - p1z;
+    const double acx = p0x - p2x, acy = p0y - p2y, acz = p0z - p2z;
+    const double cx = aby * acz - abz * acy;
+    const double cy = abz * acx - abx * acz;
+    const double cz = abx * acy - aby * acx;
+    return sqrt(cx * cx + cy * cy + cz * cz) / 2.0;
+  }
+};
+// The triangle of the table row's low three nibbles in the cell at (x, y, z).
+template <class T>
+__device__ inline Tri cell_triangle(uint32_t row, const uint32_t* s_edge, const T* cv, int slot, int x, int y, int z) {
+  Tri t;
+  edge_vertex<T>(s_edge[row & 15u], cv, slot, x, y, z, t.p0x, t.p0y, t.p0z);
+  edge_vertex<T>(s_edge[(row >> 4) & 15u], cv, slot, x, y, z, t.p1x, t.p1y, t.p1z);
+  edge_vertex<T>(s_edge[(row >> 8) & 15u], cv, slot, x, y, z, t.p2x, t.p2y, t.p2z);
+  return t;
+}
+
+struct TriTable {
+  uint64_t row[256];
+  uint8_t count[256];  // triangles of each case
+  uint32_t edge[16];
+};
+__device__ inline void load_tri_table(TriTable& s) {
+  for (int i = threadIdx.x; i < 256; i += blockDim.x) {
+    uint64_t row = c_tri[i];
+    s.row[i] = row;
+    int cnt = 0;
+    for (; (row & 15u) != 15u; row >>= 12) ++cnt;
+    s.count[i] = (uint8_t)cnt;
+    if (i < 16) s.edge[i] = i < 12 ? edge_word(i) : 0u;
+  }
+}
+
+// Compensated sums over the wavefront, the same on every run.
+__device__ inline void wave_reduce(Acc& vol, Acc& area) {
+  for (int off = 32; off > 0; off >>= 1) {
+    const double s2 = __shfl_down(vol.s, off), c2 = __shfl_down(vol.c, off);
+    const double a2 = __shfl_down(area.s, off), d2 = __shfl_down(area.c, off);
+    vol.merge(s2, c2);
+    area.merge(a2, d2);
+  }
+}
+
+constexpr int kHullWords = 304;  // sign words in LDS: two layers of the largest box, or more of smaller ones
+template <class T>
+struct HullWave {
+  unsigned long long w[kHullWords];
+  uint32_t cells[128];
+  uint16_t tq[5 * 64];  // triangles of the 64 cells at work: lane | triangle << 6
+  uint8_t ci[64];       // their cases
+  T cv[8 * 64];
+};
+
+// Existence, volume and area without topology: a wavefront takes kHullRun
+// consecutive layer tiles of the plan (all classes, so the pieces of a run
+// belong to one or two grains), carries a grain's pending cells and sums over
+// its layers, and reuses the upper layer's words as the next lower ones.  Each
+// lane of a batch of 64 cells then works on one triangle at a time.  A piece's
+// sums go to the slot of its first layer, zeros to the others.
 //
-// TOPO: each cut cell also names its grains (the grain itself at inside
-// corners, the IDLocal id at the others), a per-tile LDS table keeps the first
-// appearance of each id, and the tile adds it to the grain's table.  A
-// separate instantiation, so the registers it needs cost nothing when off.
+// What bounds it: latency (loads of a run, then the corner gathers and the
+// chain of triangle arithmetic of a batch) at the six (FP32) and four (FP64)
+// wavefronts per SIMD its registers allow; of the vector instructions about half
+// are triangle arithmetic.  Before, two layers of values were staged in LDS per
+// workgroup, every lane read eight corners of four cells to classify them, and
+// each class had a launch whose XCDs took contiguous ranges, so that the
+// largest boxes all went to one XCD.  Hull of one step, alone: 8000 grains FP32
+// 1.46 -> 0.94 ms, FP64 2.35 -> 1.21; 20000 bimodal grains FP32 2.16 -> 1.12.  With
+// contiguous ranges over all classes the last would be 2.25, with 16 loads in
+// flight 2.31, at five wavefronts 2.37; runs of 8 layers leave 512 grains 60 %
+// slower.
+constexpr int kHullRun = 4;
+template <class T>
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(6))) void k_hull(PlanDev P, DescDev din,
+                                                                                      int32_t* exflag,
+                                                                                      double* partials) {
+  __shared__ HullWave<T> s_wave[4];
+  __shared__ TriTable s_tri;
+  load_tri_table(s_tri);
+  __syncthreads();
+  const int lane = threadIdx.x & 63, wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  HullWave<T>& s = s_wave[wv];
+  const unsigned long long below = (1ull << lane) - 1ull;
+  // The classes with the largest boxes first (the longest pieces of work), each
+  // class spread over the XCDs; workgroups take 4 consecutive runs.
+  int skip = 0;  // workgroups of this XCD served by the classes before
+  for (int cls = kClasses - 1; cls >= 0; --cls) {
+    const int total = P.totals[kQLayers * kClasses + cls];
+    const uint32_t* __restrict__ tmap = P.tmap[kQLayers] + P.tile_base[kQLayers * kClasses + cls];
+    const int64_t slots = P.layer_base[cls];
+    const TileRange tr = xcd_tiles((total + 4 * kHullRun - 1) / (4 * kHullRun), skip);
+    skip = tr.skip;
+    for (int bt = tr.first; bt < tr.end; bt += tr.step) {
+      const int t1 = min(total, (bt * 4 + wv + 1) * kHullRun);
+      for (int t = (bt * 4 + wv) * kHullRun; t < t1;) {  // pieces of one grain
+        const uint32_t tile = tmap[t];
+        const int g = (int)(tile >> 8), ka = (int)(tile & 0xFFu);
+        const int32_t* b = din.bounds + 6 * g;
+        const int x0 = b[0], y0 = b[1], z0 = b[2], n = b[3] - b[0], nn2 = n * n;
+        const int kb = min(n, ka + t1 - t);  // its layers in this run: [ka, kb)
+        const T* __restrict__ box = (const T*)din.arena + din.off[g];
+        Acc vol{0.0, 0.0}, area{0.0, 0.0};
+        int pend = 0;
+        bool cut = false;
+        auto batch = [&](int base, int cnt) {  // cells base .. base + cnt - 1 of the queue
+          const uint32_t e = s.cells[base + min(lane, cnt - 1)];
+          const int xl = e & 127u, yl = (e >> 7) & 127u, kl = (e >> 14) & 127u;
+          const unsigned ci = stage_corners<T>(s.cv, box + ((int64_t)kl * n + yl) * n + xl, n, nn2, lane);
+          s.ci[lane] = (uint8_t)ci;
+          const int nt = lane < cnt ? s_tri.count[ci] : 0;
+          int incl = nt;
+  #pragma unroll
+          for (int o = 1; o < 64; o <<= 1) {
+            const int u = __shfl_up(incl, o);
+            if (lane >= o) incl += u;
+          }
+          const int nq = __builtin_amdgcn_readlane(incl, 63);
+          for (int j = 0; j < nt; ++j) s.tq[incl - nt + j] = (uint16_t)(lane | j << 6);
+          wave_fence();
+          for (int q = lane; q < nq; q += 64) {
+            const int v = s.tq[q], slot = v & 63;
+            const uint32_t ce = s.cells[base + slot];
+            const Tri tri = cell_triangle<T>((uint32_t)(s_tri.row[s.ci[slot]] >> (12 * (v >> 6))), s_tri.edge, s.cv, slot,
+                                             x0 + (int)(ce & 127u), y0 + (int)((ce >> 7) & 127u),
+                                             z0 + (int)((ce >> 14) & 127u));
+            vol.add(tri.volume());
+            area.add(tri.area());
+          }
+          wave_fence();  // the queue and the corners are refilled
+        };
+        for (int k = ka; k < min(kb, n - 1);) {
+          // as many layers as the words hold
+          const int nl = min(min(kb, n - 1) - k, (kHullWords * 64 - 64) / nn2 - 1);
+          if (load_words<T>(s.w, box + (int64_t)k * nn2, (nl + 1) * nn2, lane)) {
+            wave_fence();
+            cut_cells<false>(s.w, n, k, nl, lane, [&](uint32_t e, bool has) {
+              const unsigned long long m = __ballot(has);
+              if (has) s.cells[pend + __popcll(m & below)] = e;
+              pend += __popcll(m);
+              cut = true;
+              if (pend >= 64) {
+                wave_fence();
+                pend -= 64;
+                batch(pend, 64);
+              }
+            });
+            wave_fence();
+          }
+          k += nl;
+        }
+        if (pend > 0) batch(0, pend);
+        wave_reduce(vol, area);
+        if (lane == 0) {
+          double* pp = partials + 4 * (slots + t);
+          pp[0] = vol.s;
+          pp[1] = vol.c;
+          pp[2] = area.s;
+          pp[3] = area.c;
+          if (cut) atomicOr(&exflag[g], 1);
+        }
+        if (lane < 4)
+          for (int u = 1; u < kb - ka; ++u) partials[4 * (slots + t + u) + lane] = 0.0;
+        t += kb - ka;
+      }
+    }
+  }
+}
+
 // A cell's barycenter sum (non-negative grid coordinates) in fixed point:
 // integer adds make a list's position sum independent of the order in which
-// tiles and lanes add to it (exact to 2^-33 grid units per cell).
+// cells add to it (exact to 2^-33 grid units per cell).
 __device__ inline unsigned long long fixpos(double v) {
   return (unsigned long long)__double2ll_rn(v * kPosScale);
 }
 
-template <class T, int NMAX, bool TOPO>
-__global__ __launch_bounds__(kHT) __attribute__((amdgpu_waves_per_eu(sizeof(T) == 4 ? 6 : 1)))
-void k_hull(SimParams sp, PlanDev P, int cls, DescDev din, int32_t* exflag, double* partials, IdlDev il,
-            TopoDev topo, int32_t* err) {
-  __shared__ T L[2 * NMAX * NMAX];
-  __shared__ uint32_t q[kChunk];
-  __shared__ uint64_t s_tri[256];
-  __shared__ uint8_t s_ntri[256];  // triangles of each case
-  __shared__ int s_wave[kHT / 64];
-  __shared__ double s_red[4][kHT / 64];
-  __shared__ int s_any[kHT / 64];
-  __shared__ int s_tk[kTopoLds], s_to[kTopoLds];  // per-tile topology table (id, first appearance)
-  __shared__ unsigned long long s_jm[kJuncLds];    // per-tile junction lists (slot masks)
-  __shared__ int s_jg[TOPO ? kJuncLds : 1];        // the grain-table slot each per-tile list went to
-  // Element sums per tile list in LDS, added to the grain's table once per tile
-  // and list; the FP64 n <= 96 class has no LDS left for them and adds each
-  // cell's sums to the grain's table directly.
-  constexpr bool kElemLds = TOPO && !(sizeof(T) == 8 && NMAX == 96);
-  __shared__ unsigned long long s_jp[kElemLds ? 3 * kJuncLds : 1];  // fixed point, kPosScale per grid unit
-  __shared__ double s_ja[kElemLds ? kJuncLds : 1];  // summed triangle areas
-  __shared__ int s_jc[kElemLds ? kJuncLds : 1];
-  __shared__ int s_gk[kTopoCap];                   // copy of the grain's id table
-  const int total = P.totals[kQLayers * kClasses + cls];
-  const T* arena = (const T*)din.arena;
-  const int tid = threadIdx.x, lane = tid & 63, wv = tid >> 6;
-  for (int i = tid; i < 256; i += kHT) {
-    uint64_t row = c_tri[i];
-    s_tri[i] = row;
-    int cnt = 0;
-    for (; (row & 15u) != 15u; row >>= 12) ++cnt;
-    s_ntri[i] = (uint8_t)cnt;
-  }
-  if constexpr (TOPO) {
-    for (int i = tid; i < kTopoLds; i += kHT) {
-      s_tk[i] = -1;
-      s_to[i] = INT_MAX;
-    }
-    for (int i = tid; i < kJuncLds; i += kHT) {
-      s_jm[i] = 0ull;
-      if constexpr (kElemLds) {
-        s_jc[i] = 0;
-        s_ja[i] = 0.0;
-        s_jp[3 * i] = s_jp[3 * i + 1] = s_jp[3 * i + 2] = 0ull;
-      }
-    }
-  }
-  // consecutive tiles (the layers of one grain) on one XCD: the layer two
-  // tiles share, and the grain's tables, come from that XCD's L2
-  const TileRange tr = xcd_tiles(total);
-  for (int tile = tr.first; tile < tr.end; tile += tr.step) {
-    int g, kl;
-    plan_tile(P, cls, kQLayers, tile, g, kl);
-    const int64_t slot = P.layer_base[cls] + tile;
+template <class T, int NMAX>
+struct TopoWave {
+  static constexpr int kWords = NMAX <= 48 ? 192 : 304;  // at least two layers
+  static constexpr int kCells = 384;
+  unsigned long long w[kWords];
+  uint32_t cells[kCells + 64];
+  T cv[8 * 64];
+};
+// The grain's tables while its hull is walked (layout of TopoDev's rows).
+struct TopoLds {
+  int key[kTopoCap], ord[kTopoCap];
+  unsigned long long jm[kJuncCap], jp[3 * kJuncCap];
+  double ja[kJuncCap];
+  int jc[kJuncCap], jo[kJuncCap];
+};
+
+// The hull with topology: one workgroup per grain, so the grain's tables live in
+// LDS and go out once, each wavefront with a share of the layers.  First every
+// wavefront queues its cut cells and counts their triangles, and the grain's
+// triangle records are reserved with one add; then the cells are worked on 64 at
+// a time, one per lane: the ids at its corners (the grain itself inside, the
+// IDLocal id outside, none outside the IDLocal box) into the id table with
+// their first appearance, the mask of their slots into the junction table, and
+// then its triangles, each made once for the volume, the area, the element sums
+// and the record.  A wavefront whose queue fills up works it off at once and
+// reserves those records by itself.
+//
+// What bounds it: latency, as without topology, and per cell the id and list
+// look-ups and the chain of one cell's triangles (one lane per cell, because
+// an element's sums add a cell's triangles in order).  128 registers (FP32; 26
+// spilled outside the loops) let two workgroups share a CU: 6.3 ms per step at
+// 20000 grains with records, against 10.4 at 185 registers.  A workgroup per
+// (grain, layer) with tables in LDS merged into global ones, and each triangle
+// made three times (volume, sums, record), took 26.5 ms; 2000 grains without
+// records 1.7 -> 0.55 ms.
+constexpr int kTopoWaves = 8;
+template <class T, int NMAX>
+__global__ __launch_bounds__(64 * kTopoWaves) __attribute__((amdgpu_waves_per_eu(4))) void k_hull_topo(PlanDev P, int c0, int c1, DescDev din, int32_t* exflag,
+                                                               double* partials, IdlDev il, TopoDev topo,
+                                                               int32_t* err) {
+  __shared__ TopoWave<T, NMAX> s_wave[kTopoWaves];
+  __shared__ TopoLds s_t;
+  __shared__ TriTable s_tri;
+  __shared__ int s_cnt[kTopoWaves];
+  __shared__ unsigned long long s_raw;
+  __shared__ double s_red[kTopoWaves][4];
+  __shared__ int s_cut;
+  load_tri_table(s_tri);
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int wv = __builtin_amdgcn_readfirstlane(tid >> 6);
+  TopoWave<T, NMAX>& s = s_wave[wv];
+  const unsigned long long below = (1ull << lane) - 1ull;
+  int ng = 0;  // grains of the classes (none of a plan that did not fit its arena)
+  for (int c = c0; c < c1; ++c) ng += P.cls_count[c];
+  for (int i = blockIdx.x; i < ng; i += gridDim.x) {
+    const int p = P.cls_start[c0] + ng - 1 - i;  // the class with the larger boxes first
+    const int g = P.grains[p];
     const int32_t* b = din.bounds + 6 * g;
-    const int x0 = b[0], y0 = b[1], z0 = b[2];
-    const int n = b[3] - b[0], nn2 = n * n, m1 = n - 1;
-    const int z = z0 + kl;
-    // c / m1 = c * m1_inv >> 24 for every cell index c < m1^2 (m1 < 96)
-    const uint32_t m1_inv = m1 > 0 ? ((1u << 24) + (uint32_t)m1 - 1u) / (uint32_t)m1 : 0u;
+    const int x0 = b[0], y0 = b[1], z0 = b[2], n = b[3] - b[0], m1 = n - 1, nn2 = n * n;
+    const T* __restrict__ box = (const T*)din.arena + din.off[g];
+    const int32_t* ib = il.bounds + 6 * g;
+    const int ix0 = ib[0], iy0 = ib[1], iz0 = ib[2], inx = ib[3] - ib[0], iny = ib[4] - ib[1], inz = ib[5] - ib[2];
+    const bool same = ix0 == x0 && iy0 == y0 && iz0 == z0 && inx == n && iny == n && inz == n;
+    const uint32_t* __restrict__ idl = il.arena + il.off[g];
+    for (int i = tid; i < kJuncCap; i += 64 * kTopoWaves) {
+      s_t.jm[i] = 0ull;
+      s_t.jp[3 * i] = s_t.jp[3 * i + 1] = s_t.jp[3 * i + 2] = 0ull;
+      s_t.ja[i] = 0.0;
+      s_t.jc[i] = 0;
+      s_t.jo[i] = INT_MAX;
+    }
+    if (tid < kTopoCap) {
+      s_t.key[tid] = -1;
+      s_t.ord[tid] = INT_MAX;
+    }
+    if (tid == 0) s_cut = 0;
+    __syncthreads();
     Acc vol{0.0, 0.0}, area{0.0, 0.0};
-    int any = 0;
-    if (kl < m1) {
-      const T* box = arena + din.off[g] + (int64_t)kl * nn2;
-      stage_to_lds(L, box, nn2, tid, kHT);
-      stage_to_lds(L + NMAX * NMAX, box + nn2, nn2, tid, kHT);
-      __syncthreads();
-      for (int c0 = 0; c0 < m1 * m1; c0 += kChunk) {
-        uint32_t code[kCPT];
-        int mine = 0;  // triangles of this lane's cut cells
+    // cells base .. base + cnt - 1 of the queue; their records go from raw[rec] on
+    auto batch = [&](int base, int cnt, int64_t rec, bool records) -> int {
+      const bool act = lane < cnt;
+      const uint32_t e = s.cells[base + min(lane, cnt - 1)];
+      const int xl = e & 127u, yl = (e >> 7) & 127u, kl = (e >> 14) & 127u;
+      const int64_t at = ((int64_t)kl * n + yl) * n + xl;
+      const unsigned ci = stage_corners<T>(s.cv, box + at, n, nn2, lane);
+      uint32_t ids[8];
+      if (same) {
+        const uint32_t* i0 = idl + at;
+        const uint32_t* i1 = i0 + nn2;
+        ids[3] = i0[0];
+        ids[2] = i0[1];
+        ids[7] = i0[n];
+        ids[6] = i0[n + 1];
+        ids[0] = i1[0];
+        ids[1] = i1[1];
+        ids[4] = i1[n];
+        ids[5] = i1[n + 1];
+      } else {
 #pragma unroll
-        for (int r = 0; r < kCPT; ++r) {
-          const int c = c0 + r * kHT + tid;
-          code[r] = 0u;
-          if (c < m1 * m1) {
-            const int yl = (int)(((uint32_t)c * m1_inv) >> 24), xl = c - yl * m1;
-            unsigned ci = 0;
-#pragma unroll
-            for (int qq = 0; qq < 8; ++qq)
-              if (L[corner_off<NMAX>(qq, xl, yl, n)] >= T(0)) ci |= 1u << qq;
-            if (ci != 0u && ci != 255u) {
-              code[r] = ci | ((uint32_t)yl << 8) | ((uint32_t)xl << 16);
-              mine += s_ntri[ci];
-            }
-          }
+        for (int q = 0; q < 8; ++q) {
+          const int cx = x0 + xl + (int)((kCornerX >> q) & 1u) - ix0;
+          const int cy = y0 + yl + (int)((kCornerY >> q) & 1u) - iy0;
+          const int cz = z0 + kl + (int)((kCornerZ >> q) & 1u) - iz0;
+          ids[q] = ((unsigned)cx < (unsigned)inx && (unsigned)cy < (unsigned)iny && (unsigned)cz < (unsigned)inz)
+                       ? idl[((int64_t)cz * iny + cy) * inx + cx]
+                       : 0xFFFFFFFFu;
         }
-        if constexpr (TOPO) {
-          const int32_t* ib = il.bounds + 6 * g;
-          const int ix0 = ib[0], iy0 = ib[1], iz0 = ib[2], inx = ib[3] - ib[0], iny = ib[4] - ib[1],
-                    inz = ib[5] - ib[2];
-          const uint32_t* idl = il.arena + il.off[g];
-          // the ids a cut cell names (own id inside, IDLocal id outside, none
-          // outside the IDLocal box) and which of them are first occurrences
-          auto cell_ids = [&](uint32_t cd, uint32_t (&ids)[8], bool (&first)[8]) {
-            const unsigned ci = cd & 0xFFu;
-            const int yl = (cd >> 8) & 0xFF, xl = cd >> 16;
+      }
 #pragma unroll
-            for (int qq = 0; qq < 8; ++qq) {
-              uint32_t id = (uint32_t)g;
-              if (!((ci >> qq) & 1u)) {
-                const int cx = x0 + xl + (int)((kCornerX >> qq) & 1u) - ix0;
-                const int cy = y0 + yl + (int)((kCornerY >> qq) & 1u) - iy0;
-                const int cz = z + (int)((kCornerZ >> qq) & 1u) - iz0;
-                id = ((unsigned)cx < (unsigned)inx && (unsigned)cy < (unsigned)iny && (unsigned)cz < (unsigned)inz)
-                         ? idl[((int64_t)cz * iny + cy) * inx + cx]
-                         : 0xFFFFFFFFu;
-              }
-              ids[qq] = id;
-            }
+      for (int q = 0; q < 8; ++q)
+        if ((ci >> q) & 1u) ids[q] = (uint32_t)g;
+      const int cell = (kl * m1 + yl) * m1 + xl;
+      // 1. grains: each distinct id with its first-appearance key (cell in the
+      //    (z, y, x) loop * 8 + rank among the cell's ascending ids); the slots
+      //    of the cell's ids make its list's mask
+      uint64_t mask = 0;
 #pragma unroll
-            for (int qq = 0; qq < 8; ++qq) {
-              first[qq] = true;
+      for (int q = 0; q < 8; ++q) {
+        bool first = act && ids[q] != 0xFFFFFFFFu;
+        int rank = 0;
 #pragma unroll
-              for (int q2 = 0; q2 < qq; ++q2) first[qq] &= ids[q2] != ids[qq];
-            }
-          };
-          // the barycenter sums (src/triangle.h:12-18) and number of a cut
-          // cell's triangles, vertices as the hull's
-          auto cell_elems = [&](uint32_t cd, double& sx, double& sy, double& sz, double& sa) -> int {
-            const unsigned ci = cd & 0xFFu;
-            const int cyl = (cd >> 8) & 0xFF, cxl = (cd >> 16) & 0xFF;
-            const int nt = s_ntri[ci];
-            uint64_t row = s_tri[ci];
-            sx = sy = sz = sa = 0.0;
-            for (int j = 0; j < nt; ++j, row >>= 12) {
-              double p0x, p0y, p0z, p1x, p1y, p1z, p2x, p2y, p2z;
-              edge_vertex<T, NMAX>((int)(row & 15u), L, cxl, cyl, n, x0 + cxl, y0 + cyl, z, p0x, p0y, p0z);
-              edge_vertex<T, NMAX>((int)((row >> 4) & 15u), L, cxl, cyl, n, x0 + cxl, y0 + cyl, z, p1x, p1y, p1z);
-              edge_vertex<T, NMAX>((int)((row >> 8) & 15u), L, cxl, cyl, n, x0 + cxl, y0 + cyl, z, p2x, p2y, p2z);
-              sx += (p0x + p1x + p2x) / 3;
-              sy += (p0y + p1y + p2y) / 3;
-              sz += (p0z + p1z + p2z) / 3;
-              // GrainBoundary::computeArea (src/InterfacialElement.cpp:81-92)
-              const double abx = p0x - p1x, aby = p0y - p1y, abz = p0z - p1z;
-              const double acx = p0x - p2x, acy = p0y - p2y, acz = p0z - p2z;
-              const double cx = aby * acz - abz * acy, cy = abz * acx - abx * acz, cz = abx * acy - aby * acx;
-              sa += sqrt(cx * cx + cy * cy + cz * cz) / 2.0;
-            }
-            return nt;
-          };
-          // 1. grains: each distinct id with its first-appearance key (cell in the
-          //    (z, y, x) loop * 8 + rank among the cell's ascending ids), per tile
-          //    in LDS, then into the grain's table
+        for (int q2 = 0; q2 < q; ++q2) first &= ids[q2] != ids[q];
+        if (!first) continue;
 #pragma unroll
-          for (int r = 0; r < kCPT; ++r) {
-            if (code[r] == 0u) continue;
-            uint32_t ids[8];
-            bool first[8];
-            cell_ids(code[r], ids, first);
-            const int cell = (kl * m1 + (int)((code[r] >> 8) & 0xFF)) * m1 + (int)(code[r] >> 16);
+        for (int q2 = 0; q2 < 8; ++q2) {
+          bool lower = ids[q2] < ids[q];
 #pragma unroll
-            for (int qq = 0; qq < 8; ++qq) {
-              if (!first[qq] || ids[qq] == 0xFFFFFFFFu) continue;
-              int rank = 0;
-#pragma unroll
-              for (int q2 = 0; q2 < 8; ++q2) rank += (first[q2] & (ids[q2] < ids[qq])) ? 1 : 0;
-              const int key = (int)ids[qq], o = cell * 8 + rank;
-              uint32_t hsl = ((uint32_t)key * 2654435761u) >> (32 - kTopoLdsBits);
-              bool done = false;
-              for (int pr = 0; pr < kTopoLds && !done; ++pr) {
-                const int old = atomicCAS(&s_tk[hsl], -1, key);
-                if (old == -1 || old == key) {
-                  atomicMin(&s_to[hsl], o);
-                  done = true;
-                }
-                hsl = (hsl + 1) & (kTopoLds - 1);
-              }
-              if (!done) atomicOr(err, kErrTopo);
-            }
-          }
-          __syncthreads();
-          int32_t* gk = topo.key + (int64_t)g * kTopoCap;
-          int32_t* go = topo.ord + (int64_t)g * kTopoCap;
-          for (int i = tid; i < kTopoLds; i += kHT) {
-            const int key = s_tk[i];
-            if (key != -1) {
-              uint32_t hsl = ((uint32_t)key * 2654435761u) >> (32 - kTopoCapBits);
-              bool done = false;
-              for (int pr = 0; pr < kTopoCap && !done; ++pr) {
-                const int old = atomicCAS(&gk[hsl], -1, key);
-                if (old == -1 || old == key) {
-                  atomicMin(&go[hsl], s_to[i]);
-                  done = true;
-                }
-                hsl = (hsl + 1) & (kTopoCap - 1);
-              }
-              if (!done) atomicOr(err, kErrTopo);
-            }
-            s_tk[i] = -1;
-            s_to[i] = INT_MAX;
-          }
-          __syncthreads();
-          // the grain's id table as it stands now (this chunk's ids are in it), read
-          // past the L1 once, for the slot lookups below
-          for (int i = tid; i < kTopoCap; i += kHT)
-            s_gk[i] = __hip_atomic_load(&gk[i], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-          __syncthreads();
-          // 2. junctions: a cell's list of distinct ids as a mask over the slots
-          //    its ids hold in the grain's table (a slot never changes once
-          //    taken, so equal lists give equal masks); distinct masks per tile in
-          //    LDS, then into the grain's junction table
-          uint64_t cmask[kCPT];
-          int cjsl[kCPT];  // the per-tile list of each cut cell
-#pragma unroll
-          for (int r = 0; r < kCPT; ++r) {
-            cmask[r] = 0;
-            cjsl[r] = -1;
-            if (code[r] == 0u) continue;
-            uint32_t ids[8];
-            bool first[8];
-            cell_ids(code[r], ids, first);
-            uint64_t mask = 0;
-#pragma unroll
-            for (int qq = 0; qq < 8; ++qq) {
-              if (!first[qq] || ids[qq] == 0xFFFFFFFFu) continue;
-              uint32_t hsl = (ids[qq] * 2654435761u) >> (32 - kTopoCapBits);
-              for (int pr = 0; pr < kTopoCap; ++pr) {
-                const int k = s_gk[hsl];
-                if (k == (int)ids[qq]) {
-                  mask |= 1ull << hsl;
-                  break;
-                }
-                if (k == -1) break;  // not in the table (it was full: reported above)
-                hsl = (hsl + 1) & (kTopoCap - 1);
-              }
-            }
-            cmask[r] = mask;
-            if (mask == 0) continue;
-            uint32_t hsl = (uint32_t)((mask * 0x9E3779B97F4A7C15ull) >> (64 - kJuncLdsBits));
-            int jsl = -1;
-            for (int pr = 0; pr < kJuncLds && jsl < 0; ++pr) {
-              const unsigned long long old = atomicCAS(&s_jm[hsl], 0ull, (unsigned long long)mask);
-              if (old == 0ull || old == mask) jsl = (int)hsl;
-              hsl = (hsl + 1) & (kJuncLds - 1);
-            }
-            if (jsl < 0) {
-              atomicOr(err, kErrTopo);
-              continue;
-            }
-            cjsl[r] = jsl;
-            if constexpr (kElemLds) {
-              // 3. interfacial elements (src/grainHull.cpp:227-270), per tile list
-              double sx, sy, sz, sa;
-              const int nt = cell_elems(code[r], sx, sy, sz, sa);
-              atomicAdd(&s_jp[3 * jsl], fixpos(sx));
-              atomicAdd(&s_jp[3 * jsl + 1], fixpos(sy));
-              atomicAdd(&s_jp[3 * jsl + 2], fixpos(sz));
-              atomicAdd(&s_ja[jsl], sa);
-              atomicAdd(&s_jc[jsl], nt);
-            }
-          }
-          __syncthreads();
-          unsigned long long* gj = topo.jkey + (int64_t)g * kJuncCap;
-          unsigned long long* gp = topo.jpos + (int64_t)g * kJuncCap * 3;
-          int32_t* gc = topo.jcnt + (int64_t)g * kJuncCap;
-          double* ga = topo.jarea + (int64_t)g * kJuncCap;
-          for (int i = tid; i < kJuncLds; i += kHT) {
-            const unsigned long long m = s_jm[i];
-            if (m != 0ull) {
-              uint32_t hsl = (uint32_t)((m * 0x9E3779B97F4A7C15ull) >> (64 - kJuncCapBits));
-              int gsl = -1;
-              for (int pr = 0; pr < kJuncCap && gsl < 0; ++pr) {
-                const unsigned long long old = atomicCAS(&gj[hsl], 0ull, m);
-                if (old == 0ull || old == m) gsl = (int)hsl;
-                hsl = (hsl + 1) & (kJuncCap - 1);
-              }
-              s_jg[i] = gsl;
-              if (gsl < 0) {
-                atomicOr(err, kErrTopo);
-              } else if constexpr (kElemLds) {
-                atomicAdd(&gp[3 * gsl], s_jp[3 * i]);
-                atomicAdd(&gp[3 * gsl + 1], s_jp[3 * i + 1]);
-                atomicAdd(&gp[3 * gsl + 2], s_jp[3 * i + 2]);
-                atomicAdd(&ga[gsl], s_ja[i]);
-                atomicAdd(&gc[gsl], s_jc[i]);
-              }
-            }
-            else {
-              s_jg[i] = -1;
-            }
-            s_jm[i] = 0ull;
-            if constexpr (kElemLds) {
-              s_jc[i] = 0;
-              s_ja[i] = 0.0;
-              s_jp[3 * i] = s_jp[3 * i + 1] = s_jp[3 * i + 2] = 0ull;
-            }
-          }
-          __syncthreads();
-          // 4. with the convolution correction on: per cut cell the grain-table
-          //    slot of its list and that list's first appearance; then every
-          //    triangle's barycenter as a record (grain, slot), appended to the
-          //    pool (one reservation per workgroup and pass)
-          if (topo.corr) {
-            int rslot[kCPT];
-            int cnt = 0;
-#pragma unroll
-            for (int r = 0; r < kCPT; ++r) {
-              // the grain-table slot of the cell's list, as the merge above left it
-              rslot[r] = cjsl[r] >= 0 ? s_jg[cjsl[r]] : -1;
-              if (rslot[r] < 0) continue;
-              const int cell = (kl * m1 + (int)((code[r] >> 8) & 0xFF)) * m1 + (int)(code[r] >> 16);
-              atomicMin(&topo.jord[(int64_t)g * kJuncCap + rslot[r]], cell);
-              cnt += s_ntri[code[r] & 0xFFu];
-            }
-            int sc = cnt;  // inclusive scan over the wavefront
-            for (int off = 1; off < 64; off <<= 1) {
-              const int y = __shfl_up(sc, off);
-              if (lane >= off) sc += y;
-            }
-            if (lane == 63) s_wave[wv] = sc;
-            __syncthreads();
-            int pos = sc - cnt, tot = 0;
-            for (int w = 0; w < kHT / 64; ++w) {
-              if (w < wv) pos += s_wave[w];
-              tot += s_wave[w];
-            }
-            __shared__ unsigned long long s_rbase;
-            if (tid == 0) s_rbase = tot ? atomicAdd(topo.raw_n, (unsigned long long)tot) : 0ull;
-            __syncthreads();
-            const unsigned long long rb = s_rbase;
-            if (tot && rb + (unsigned long long)tot > (unsigned long long)topo.raw_cap) {
-              if (tid == 0) atomicOr(err, kErrTri);
-            } else if (tot) {
-#pragma unroll
-              for (int r = 0; r < kCPT; ++r) {
-                if (rslot[r] < 0) continue;
-                const unsigned ci = code[r] & 0xFFu;
-                const int cyl = (code[r] >> 8) & 0xFF, cxl = (code[r] >> 16) & 0xFF;
-                const int nt = s_ntri[ci];
-                uint64_t row = s_tri[ci];
-                for (int j = 0; j < nt; ++j, row >>= 12) {
-                  double p0x, p0y, p0z, p1x, p1y, p1z, p2x, p2y, p2z;
-                  edge_vertex<T, NMAX>((int)(row & 15u), L, cxl, cyl, n, x0 + cxl, y0 + cyl, z, p0x, p0y, p0z);
-                  edge_vertex<T, NMAX>((int)((row >> 4) & 15u), L, cxl, cyl, n, x0 + cxl, y0 + cyl, z, p1x, p1y, p1z);
-                  edge_vertex<T, NMAX>((int)((row >> 8) & 15u), L, cxl, cyl, n, x0 + cxl, y0 + cyl, z, p2x, p2y, p2z);
-                  TriRec t;
-                  t.x = (p0x + p1x + p2x) / 3;
-                  t.y = (p0y + p1y + p2y) / 3;
-                  t.z = (p0z + p1z + p2z) / 3;
-                  t.g = g;
-                  t.slot = rslot[r];
-                  topo.raw[rb + pos++] = t;
-                }
-              }
-            }
-            __syncthreads();  // s_wave and s_rbase are reused
-          }
-          // 3. interfacial elements (src/grainHull.cpp:227-270) of the class
-          //    without LDS for them: each cut cell adds its sums to its list's
-          //    slot in the grain's junction table
-#pragma unroll
-          for (int r = 0; r < kCPT; ++r) {
-            if constexpr (kElemLds) break;
-            const int slot = cjsl[r] >= 0 ? s_jg[cjsl[r]] : -1;
-            if (slot < 0) continue;
-            double sx, sy, sz, sa;
-            const int nt = cell_elems(code[r], sx, sy, sz, sa);
-            atomicAdd(&gp[3 * slot], fixpos(sx));
-            atomicAdd(&gp[3 * slot + 1], fixpos(sy));
-            atomicAdd(&gp[3 * slot + 2], fixpos(sz));
-            atomicAdd(&ga[slot], sa);
-            atomicAdd(&gc[slot], nt);
-          }
+          for (int q3 = 0; q3 < q2; ++q3) lower &= ids[q3] != ids[q2];
+          rank += lower ? 1 : 0;
         }
-        // exclusive scan of the per-lane triangle counts: wavefront, then workgroup
-        int sc = mine;
-        for (int off = 1; off < 64; off <<= 1) {
-          const int y = __shfl_up(sc, off);
-          if (lane >= off) sc += y;
+        const int key = (int)ids[q], o = cell * 8 + rank;
+        uint32_t hsl = ((uint32_t)key * 2654435761u) >> (32 - kTopoCapBits);
+        bool done = false;
+        for (int pr = 0; pr < kTopoCap && !done; ++pr) {
+          int old = s_t.key[hsl];
+          if (old == -1) old = atomicCAS(&s_t.key[hsl], -1, key);
+          if (old == -1 || old == key) {
+            if (o < s_t.ord[hsl]) atomicMin(&s_t.ord[hsl], o);
+            mask |= 1ull << hsl;
+            done = true;
+          }
+          hsl = (hsl + 1) & (kTopoCap - 1);
         }
-        if (lane == 63) s_wave[wv] = sc;
-        __syncthreads();
-        int pos = sc - mine, nq = 0;
-        for (int w = 0; w < kHT / 64; ++w) {
-          if (w < wv) pos += s_wave[w];
-          nq += s_wave[w];
+        if (!done) atomicOr(err, kErrTopo);
+      }
+      // 2. junctions: the cell's list as a mask over the grain's table slots
+      int js = -1;
+      if (mask != 0) {
+        uint32_t hsl = (uint32_t)((mask * 0x9E3779B97F4A7C15ull) >> (64 - kJuncCapBits));
+        for (int pr = 0; pr < kJuncCap && js < 0; ++pr) {
+          unsigned long long old = s_t.jm[hsl];
+          if (old == 0ull) old = atomicCAS(&s_t.jm[hsl], 0ull, (unsigned long long)mask);
+          if (old == 0ull || old == mask) js = (int)hsl;
+          hsl = (hsl + 1) & (kJuncCap - 1);
         }
-        if (nq) any = 1;
-        // The triangles are listed cell by cell (entry = cell code | triangle
-        // index << 24) in windows of kChunk entries; every lane then takes one
-        // triangle at a time, so lanes do not wait on cells with more triangles.
-        for (int w0 = 0; w0 < nq; w0 += kChunk) {
-          int pp = pos;
+        if (js < 0) atomicOr(err, kErrTopo);
+        else if (cell < s_t.jo[js]) atomicMin(&s_t.jo[js], cell);
+      }
+      // 3. the triangles: volume, area, the element's barycenter and area sums
+      //    (src/grainHull.cpp:227-270, src/triangle.h:12-18), the record
+      const int nt = act ? s_tri.count[ci] : 0;
+      int incl = nt;
 #pragma unroll
-          for (int r = 0; r < kCPT; ++r) {
-            if (code[r] != 0u) {
-              const int t = s_ntri[code[r] & 0xFFu];
-              for (int j = 0; j < t; ++j, ++pp)
-                if (pp >= w0 && pp < w0 + kChunk) q[pp - w0] = code[r] | (uint32_t)j << 24;
-            }
-          }
-          __syncthreads();
-          const int nw = min(kChunk, nq - w0);
-          for (int w = tid; w < nw; w += kHT) {
-            const uint32_t cd = q[w];
-            const unsigned ci = cd & 0xFFu;
-            const int yl = (cd >> 8) & 0xFF, xl = (cd >> 16) & 0xFF;
-            const uint32_t row = (uint32_t)(s_tri[ci] >> (12 * (cd >> 24)));
-            const int x = x0 + xl, y = y0 + yl;
-            double p0x, p0y, p0z, p1x, p1y, p1z, p2x, p2y, p2z;
-            edge_vertex<T, NMAX>((int)(row & 15u), L, xl, yl, n, x, y, z, p0x, p0y, p0z);
-            edge_vertex<T, NMAX>((int)((row >> 4) & 15u), L, xl, yl, n, x, y, z, p1x, p1y, p1z);
-            edge_vertex<T, NMAX>((int)((row >> 8) & 15u), L, xl, yl, n, x, y, z, p2x, p2y, p2z);
-            const double v321 = p2x * p1y * p0z;
-            const double v231 = p1x * p2y * p0z;
-            const double v312 = p2x * p0y * p1z;
-            const double v132 = p0x * p2y * p1z;
-            const double v213 = p1x * p0y * p2z;
-            const double v123 = p0x * p1y * p2z;
-            vol.add((double)(1.0f / 6.0f) * (-v321 + v231 + v312 - v132 - v213 + v123));
-            const double abx = p0x - p1x, aby = p0y - p1y, abz = p0z - p1z;
-            const double acx = p0x - p2x, acy = p0y - p2y, acz = p0z - p2z;
-            const double cx = aby * acz - abz * acy;
-            const double cy = abz * acx - abx * acz;
-            const double cz = abx * acy - aby * acx;
-            area.add(sqrt(cx * cx + cy * cy + cz * cz) / 2.0);
-          }
-          __syncthreads();
+      for (int o = 1; o < 64; o <<= 1) {
+        const int u = __shfl_up(incl, o);
+        if (lane >= o) incl += u;
+      }
+      const int ntri = __builtin_amdgcn_readlane(incl, 63);
+      wave_fence();
+      uint64_t row = s_tri.row[ci];
+      double sx = 0.0, sy = 0.0, sz = 0.0, sa = 0.0;
+      TriRec* out = records ? topo.raw + rec + (incl - nt) : nullptr;
+      for (int j = 0; j < nt; ++j, row >>= 12) {
+        const Tri t = cell_triangle<T>((uint32_t)row, s_tri.edge, s.cv, lane, x0 + xl, y0 + yl, z0 + kl);
+        vol.add(t.volume());
+        const double ar = t.area();
+        area.add(ar);
+        sa += ar;
+        TriRec r;
+        r.x = (t.p0x + t.p1x + t.p2x) / 3;
+        r.y = (t.p0y + t.p1y + t.p2y) / 3;
+        r.z = (t.p0z + t.p1z + t.p2z) / 3;
+        sx += r.x;
+        sy += r.y;
+        sz += r.z;
+        if (records) {
+          r.g = js >= 0 ? g : 0;  // grain 0 has no elements: the record is passed over
+          r.slot = js >= 0 ? js : 0;
+          out[j] = r;
         }
-        __syncthreads();  // s_wave is read above before the next chunk writes it
+      }
+      if (js >= 0) {
+        atomicAdd(&s_t.jp[3 * js], fixpos(sx));
+        atomicAdd(&s_t.jp[3 * js + 1], fixpos(sy));
+        atomicAdd(&s_t.jp[3 * js + 2], fixpos(sz));
+        atomicAdd(&s_t.ja[js], sa);
+        atomicAdd(&s_t.jc[js], nt);
+      }
+      wave_fence();  // the queue and the corners are refilled
+      return ntri;
+    };
+    // room for cnt records, or none (the device error is set): -1
+    auto reserve = [&](int cnt) -> int64_t {
+      const unsigned long long rb = atomicAdd(topo.raw_n, (unsigned long long)cnt);
+      if (rb + (unsigned long long)cnt <= (unsigned long long)topo.raw_cap) return (int64_t)rb;
+      atomicOr(err, kErrTri);
+      for (unsigned long long r = rb; r < (unsigned long long)topo.raw_cap && r < rb + (unsigned long long)cnt; ++r)
+        topo.raw[r].g = topo.raw[r].slot = 0;
+      return -1;
+    };
+    auto triangles = [&](int base, int cnt) {  // of the queue's cells
+      int c = 0;
+      for (int i = lane; i < cnt; i += 64) c += s_tri.count[s.cells[base + i] >> 21];
+#pragma unroll
+      for (int o = 1; o < 64; o <<= 1) c += __shfl_xor(c, o);
+      return c;
+    };
+    // this wavefront's cut cells
+    int pend = 0;
+    bool cut = false;
+    {
+      const int k0 = m1 * wv / kTopoWaves, k1 = m1 * (wv + 1) / kTopoWaves;
+      for (int k = k0; k < k1;) {
+        const int nl = min(k1 - k, (TopoWave<T, NMAX>::kWords * 64 - 64) / nn2 - 1);
+        if (load_words<T>(s.w, box + (int64_t)k * nn2, (nl + 1) * nn2, lane)) {
+          wave_fence();
+          cut_cells<true>(s.w, n, k, nl, lane, [&](uint32_t e, bool has) {
+            const unsigned long long m = __ballot(has);
+            if (has) s.cells[pend + __popcll(m & below)] = e;
+            pend += __popcll(m);
+            cut = true;
+            if (pend > TopoWave<T, NMAX>::kCells) {
+              wave_fence();
+              pend -= 64;
+              int64_t rec = -1;
+              if (topo.corr) {
+                const int c = triangles(pend, 64);
+                if (lane == 0) rec = reserve(c);
+                rec = __shfl(rec, 0);
+              }
+              batch(pend, 64, rec, rec >= 0);
+            }
+          });
+          wave_fence();
+        }
+        k += nl;
       }
     }
-    // wavefront then workgroup reduction in a fixed order
-    double r4[4] = {vol.s, vol.c, area.s, area.c};
-    for (int off = 32; off > 0; off >>= 1) {
-      double s2 = __shfl_down(r4[0], off), c2 = __shfl_down(r4[1], off);
-      double a2 = __shfl_down(r4[2], off), d2 = __shfl_down(r4[3], off);
-      Acc va{r4[0], r4[1]}, aa{r4[2], r4[3]};
-      va.merge(s2, c2);
-      aa.merge(a2, d2);
-      r4[0] = va.s; r4[1] = va.c; r4[2] = aa.s; r4[3] = aa.c;
+    int64_t rec = -1;
+    if (topo.corr) {
+      const int c = triangles(0, pend);
+      if (lane == 0) s_cnt[wv] = c;
+      __syncthreads();
+      if (tid == 0) {
+        int tot = 0;
+        for (int w = 0; w < kTopoWaves; ++w) tot += s_cnt[w];
+        s_raw = tot ? (unsigned long long)reserve(tot) : 0ull;
+      }
+      __syncthreads();
+      rec = (int64_t)s_raw;
+      for (int w = 0; w < wv; ++w)
+        if (rec >= 0) rec += s_cnt[w];
     }
+    for (int base = 0; base < pend; base += 64) {
+      const int c = batch(base, min(64, pend - base), rec, rec >= 0);
+      if (rec >= 0) rec += c;
+    }
+    wave_reduce(vol, area);
     if (lane == 0) {
-      for (int qq = 0; qq < 4; ++qq) s_red[qq][wv] = r4[qq];
-      s_any[wv] = any;
+      s_red[wv][0] = vol.s;
+      s_red[wv][1] = vol.c;
+      s_red[wv][2] = area.s;
+      s_red[wv][3] = area.c;
+      if (cut) s_cut = 1;
     }
     __syncthreads();
+    const int cls = size_class(n);
+    const int64_t slot = P.layer_base[cls] + P.pre[kQLayers][p + cls];  // the grain's first layer (class c's prefixes start at cls_start[c] + c)
     if (tid == 0) {
-      Acc va{s_red[0][0], s_red[1][0]}, aa{s_red[2][0], s_red[3][0]};
-      int an = s_any[0];
-      for (int w = 1; w < kHT / 64; ++w) {
-        va.merge(s_red[0][w], s_red[1][w]);
-        aa.merge(s_red[2][w], s_red[3][w]);
-        an |= s_any[w];
+      Acc va{s_red[0][0], s_red[0][1]}, aa{s_red[0][2], s_red[0][3]};
+      for (int w = 1; w < kTopoWaves; ++w) {
+        va.merge(s_red[w][0], s_red[w][1]);
+        aa.merge(s_red[w][2], s_red[w][3]);
       }
       double* pp = partials + 4 * slot;
-      pp[0] = va.s; pp[1] = va.c; pp[2] = aa.s; pp[3] = aa.c;
-      if (an) atomicOr(&exflag[g], 1);
+      pp[0] = va.s;
+      pp[1] = va.c;
+      pp[2] = aa.s;
+      pp[3] = aa.c;
+      if (s_cut) atomicOr(&exflag[g], 1);
     }
-    __syncthreads();
+    for (int i = 4 + tid; i < 4 * n; i += 64 * kTopoWaves) partials[4 * slot + i] = 0.0;
+    if (tid < kTopoCap) {
+      topo.key[(int64_t)g * kTopoCap + tid] = s_t.key[tid];
+      topo.ord[(int64_t)g * kTopoCap + tid] = s_t.ord[tid];
+    }
+    const int64_t jb = (int64_t)g * kJuncCap;
+    for (int i = tid; i < kJuncCap; i += 64 * kTopoWaves) {
+      topo.jkey[jb + i] = s_t.jm[i];
+      topo.jcnt[jb + i] = s_t.jc[i];
+      topo.jarea[jb + i] = s_t.ja[i];
+      if (topo.corr) topo.jord[jb + i] = s_t.jo[i];
+    }
+    for (int i = tid; i < 3 * kJuncCap; i += 64 * kTopoWaves) topo.jpos[3 * jb + i] = s_t.jp[i];
+    __syncthreads();  // the tables are refilled for the next grain
   }
 }
 
@@ -669,57 +791,53 @@ void upload_mc_tables() {
   (void)hipMemcpyToSymbol(HIP_SYMBOL(c_tri), tri, sizeof(tri));
 }
 
-template <class T, bool TOPO>
-void hull_classes(const Launch& L, const SimParams& sp, const PlanDev& P, const DescDev& din, int32_t* exflag,
-                  double* partials, const IdlDev& il, const TopoDev& topo, int32_t* err, int c0, int c1) {
-  if (c0 <= 0 && 0 < c1)
-    hipLaunchKernelGGL((k_hull<T, 32, TOPO>), dim3(tile_grid(L, kGridPerCU, 0, sp.N, layers_of(0))), dim3(kHT), 0, L.stream, sp, P, 0,
-                       din, exflag, partials, il, topo, err);
-  if (c0 <= 1 && 1 < c1)
-    hipLaunchKernelGGL((k_hull<T, 48, TOPO>), dim3(tile_grid(L, kGridPerCU, 1, sp.N, layers_of(1))), dim3(kHT), 0, L.stream, sp, P, 1,
-                       din, exflag, partials, il, topo, err);
-  if (c0 <= 2 && 2 < c1)
-    hipLaunchKernelGGL((k_hull<T, 64, TOPO>), dim3(tile_grid(L, kGridPerCU, 2, sp.N, layers_of(2))), dim3(kHT), 0, L.stream, sp, P, 2,
-                       din, exflag, partials, il, topo, err);
-  if (c0 <= 3 && 3 < c1)
-    hipLaunchKernelGGL((k_hull<T, 96, TOPO>), dim3(tile_grid(L, kGridPerCU, 3, sp.N, layers_of(3))), dim3(kHT), 0, L.stream, sp, P, 3,
-                       din, exflag, partials, il, topo, err);
-}
-
-// Clears the grains' topology tables before a hull with topology on.
-__global__ __launch_bounds__(256) void k_topo_clear(SimParams sp, TopoDev topo) {
-  const int64_t n = (int64_t)(sp.N + 1) * kTopoCap, nj = (int64_t)(sp.N + 1) * kJuncCap;
-  for (int64_t i = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; i < nj; i += (int64_t)gridDim.x * blockDim.x) {
-    if (i < n) {
-      topo.key[i] = -1;
-      topo.ord[i] = INT_MAX;
+// Clears the topology tables of the grains the hull does not walk (it writes
+// whole tables), and the triangle records, before a hull with topology on.
+__global__ __launch_bounds__(256) void k_topo_clear(SimParams sp, PlanDev P, TopoDev topo) {
+  if (topo.corr && blockIdx.x == 0 && threadIdx.x == 0) *topo.raw_n = 0ull;
+  for (int g = blockIdx.x; g <= sp.N; g += gridDim.x) {
+    if (g > 0 && P.grain_pos[g] >= 0) continue;
+    const int64_t b = (int64_t)g * kTopoCap, jb = (int64_t)g * kJuncCap;
+    for (int i = threadIdx.x; i < kTopoCap; i += 256) {
+      topo.key[b + i] = -1;
+      topo.ord[b + i] = INT_MAX;
     }
-    topo.jkey[i] = 0ull;
-    topo.jcnt[i] = 0;
-    if (topo.corr) topo.jord[i] = INT_MAX;
-    if (topo.corr && i == 0) *topo.raw_n = 0ull;
-    topo.jpos[3 * i] = 0ull;
-    topo.jpos[3 * i + 1] = 0ull;
-    topo.jpos[3 * i + 2] = 0ull;
-    topo.jarea[i] = 0.0;
+    for (int i = threadIdx.x; i < kJuncCap; i += 256) {
+      topo.jkey[jb + i] = 0ull;
+      topo.jcnt[jb + i] = 0;
+      if (topo.corr) topo.jord[jb + i] = INT_MAX;
+      topo.jpos[3 * (jb + i)] = 0ull;
+      topo.jpos[3 * (jb + i) + 1] = 0ull;
+      topo.jpos[3 * (jb + i) + 2] = 0ull;
+      topo.jarea[jb + i] = 0.0;
+    }
   }
 }
 
-void launch_topo_clear(const Launch& L, const SimParams& sp, const TopoDev& topo) {
-  const int64_t n = (int64_t)(sp.N + 1) * kJuncCap;
-  const int blocks = (int)std::min<int64_t>((n + 255) / 256, 65536);
-  hipLaunchKernelGGL(k_topo_clear, dim3(blocks), dim3(256), 0, L.stream, sp, topo);
+void launch_topo_clear(const Launch& L, const SimParams& sp, const PlanDev& P, const TopoDev& topo) {
+  hipLaunchKernelGGL(k_topo_clear, dim3(std::min(sp.N + 1, L.grid)), dim3(256), 0, L.stream, sp, P, topo);
+}
+
+template <class T>
+void hull_all(const Launch& L, const SimParams& sp, const PlanDev& P, const DescDev& din, int32_t* exflag,
+              double* partials, const IdlDev& il, const TopoDev& topo, int32_t* err) {
+  if (!topo.on) {
+    const int64_t need = ((int64_t)sp.N * kMaxN / (4 * kHullRun) + kXcds) / kXcds * kXcds;
+    const int grid = (int)std::min<int64_t>((int64_t)L.cus * kGridPerCU, need);
+    hipLaunchKernelGGL(k_hull<T>, dim3(grid), dim3(256), 0, L.stream, P, din, exflag, partials);
+    return;
+  }
+  const int grid = std::min(sp.N, L.cus * kGridPerCU);
+  hipLaunchKernelGGL((k_hull_topo<T, 48>), dim3(grid), dim3(64 * kTopoWaves), 0, L.stream, P, 0, 2, din, exflag,
+                     partials, il, topo, err);
+  hipLaunchKernelGGL((k_hull_topo<T, 96>), dim3(grid), dim3(64 * kTopoWaves), 0, L.stream, P, 2, 4, din, exflag,
+                     partials, il, topo, err);
 }
 
 void launch_hull(const Launch& L, const SimParams& sp, const PlanDev& P, const DescDev& din, int32_t* exflag,
-                 double* partials, const IdlDev& il, const TopoDev& topo, int32_t* err, bool fp32, int c0, int c1) {
-  if (fp32) {
-    if (topo.on) hull_classes<float, true>(L, sp, P, din, exflag, partials, il, topo, err, c0, c1);
-    else hull_classes<float, false>(L, sp, P, din, exflag, partials, il, topo, err, c0, c1);
-  } else {
-    if (topo.on) hull_classes<double, true>(L, sp, P, din, exflag, partials, il, topo, err, c0, c1);
-    else hull_classes<double, false>(L, sp, P, din, exflag, partials, il, topo, err, c0, c1);
-  }
+                 double* partials, const IdlDev& il, const TopoDev& topo, int32_t* err, bool fp32) {
+  if (fp32) hull_all<float>(L, sp, P, din, exflag, partials, il, topo, err);
+  else hull_all<double>(L, sp, P, din, exflag, partials, il, topo, err);
 }
 
 void launch_finalize(const Launch& L, const SimParams& sp, const PlanDev& P, int32_t* state, const ListDev& ld,

@@ -252,16 +252,22 @@ __device__ inline void plan_tile(const PlanDev& P, int c, int q, int t, int& g, 
 // XCDs round-robin (workgroup b runs on XCD b % 8) and every XCD has its own
 // L2, so XCD x takes the contiguous tile range [x*T/8, (x+1)*T/8): the tiles of
 // neighbouring grains (the plan orders grains spatially) then share one L2.
+// A launch that takes several tile lists one after another passes on `skip`:
+// the workgroups of an XCD go on with the next list where the last one ended, so
+// a list that does not fill them leaves the rest to the next.
 struct TileRange {
   int first, end, step;
+  int skip;  // for the next list
 };
 constexpr int kXcds = 8;
-__device__ inline TileRange xcd_tiles(int total) {
+__device__ inline TileRange xcd_tiles(int total, int skip = 0) {
   const int G = gridDim.x, b = blockIdx.x;
-  if (G % kXcds) return TileRange{b, total, G};
-  const int x = b % kXcds, r = b / kXcds;
-  const int lo = (int)((int64_t)total * x / kXcds), hi = (int)((int64_t)total * (x + 1) / kXcds);
-  return TileRange{lo + r, hi, G / kXcds};
+  const int per = G % kXcds ? G : G / kXcds;  // workgroups that share a range
+  const int x = G % kXcds ? 0 : b % kXcds, r = G % kXcds ? b : b / kXcds;
+  const int lo = G % kXcds ? 0 : (int)((int64_t)total * x / kXcds);
+  const int hi = G % kXcds ? total : (int)((int64_t)total * (x + 1) / kXcds);
+  const int turn = r - skip < 0 ? r - skip + per : r - skip;
+  return TileRange{lo + turn, hi, per, (skip + hi - lo) % per};
 }
 
 // Flattened tile lookup over all classes for one quantity.
@@ -405,11 +411,10 @@ enum { kSpaceAll = 0, kSpaceBuild = 1, kSpaceRun = 2 };
 void launch_comparison_space(const Launch& L, int shape, const SimParams& sp, const PlanDev& P, const DescDev& din,
                              const DescDev& dout, const ListDev& ld, const IdlDev& il_old, const IdlDev& il_new,
                              int32_t* newb, const CmpSpaceDev& W, int32_t* err, bool fp32, int part = kSpaceAll);
-// Clears the grains' topology tables; before every hull with topology on.
-void launch_topo_clear(const Launch& L, const SimParams& sp, const TopoDev& topo);
+// Clears the topology tables of grains outside the plan; before every hull with topology on.
+void launch_topo_clear(const Launch& L, const SimParams& sp, const PlanDev& P, const TopoDev& topo);
 void launch_hull(const Launch& L, const SimParams& sp, const PlanDev& P, const DescDev& din, int32_t* exflag,
-                 double* partials, const IdlDev& il, const TopoDev& topo, int32_t* err, bool fp32, int c0 = 0,
-                 int c1 = kClasses);
+                 double* partials, const IdlDev& il, const TopoDev& topo, int32_t* err, bool fp32);
 // Parts of the level-set finalize (k_finalize).
 constexpr int kFinBounds = 1, kFinState = 2, kFinCoarsen = 4;
 void launch_finalize(const Launch& L, const SimParams& sp, const PlanDev& P, int32_t* state,
