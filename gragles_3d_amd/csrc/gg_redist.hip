@@ -282,38 +282,69 @@ __global__ __launch_bounds__(64) void k_redist_z(SimParams sp, PlanDev P, int cl
   }
 }
 
-// One forward step of a register-resident sweep at q -> q+1 (the loop bodies
-// above): `act` = q inside the loop range, `ip` = interpolate (in values a, b
-// at q, q+1).  FP64 keeps the reference's two divisions (bit-identical); FP32
-// uses d = -a*h/(b - a) with the hardware reciprocal and no branch, which
+// h with the sign of v, 0 for 0: (T)sgnv(v) * h without the conversion.
+__device__ inline float sgnh(float v, float h) { return v == 0.f ? 0.f : __builtin_copysignf(h, v); }
+__device__ inline double sgnh(double v, double h) { return v == 0.0 ? 0.0 : __builtin_copysign(h, v); }
+
+// One step of a register-resident sweep from cur to nxt (the loop bodies
+// above): `ip` = interpolate (in values a, b at the two points), `act` = the
+// step is in the loop's range (ip only where act).  FP64 keeps the reference's
+// two divisions (bit-identical), taken only where some lane has a sign change;
+// FP32 uses d = -a*h/(b - a) with the hardware reciprocal and no branch, which
 // rounds differently but is the same formula.
-__device__ inline void fwd_step(double& cur, double& nxt, double a, double b, bool act, bool ip, double h) {
+__device__ inline void sweep_step(double& cur, double& nxt, double a, double b, bool act, bool ip, double h) {
+  if (ip && a * b <= 0.0) {
+    const double slope = (b - a) / h;
+    const double d = -a / slope;
+    if (absv(cur) > absv(d)) cur = -d * (double)sgnv(slope);
+  }
+  const double cand = cur + sgnh(ip ? b : nxt, h);
+  if (act && absv(cand) < absv(nxt)) nxt = cand;
+}
+__device__ inline void sweep_step(float& cur, float& nxt, float a, float b, bool act, bool ip, float h) {
+  const float dba = b - a;
+  const float d = -a * h * __builtin_amdgcn_rcpf(dba);
+  // a taken d is finite, so dba is not 0: -d times the sign of dba
+  const float sd = __int_as_float(__float_as_int(-d) ^ (__float_as_int(dba) & (int)0x80000000));
+  cur = ip & (a * b <= 0.f) & (fabsf(cur) > fabsf(d)) ? sd : cur;
+  const float cand = cur + sgnh(ip ? b : nxt, h);
+  nxt = act & (fabsf(cand) < fabsf(nxt)) ? cand : nxt;
+}
+
+// The FP64 z step: the same, with branches around what no lane needs (1.37
+// against 1.53 ms at 8000 grains for the form above; in x/y, where each lane
+// has its own range, the form above is the faster one, 2.15 against 2.36).
+__device__ inline void branch_step(double& cur, double& nxt, double a, double b, bool act, bool ip, double h) {
   if (!act) return;
   double cand;
   if (ip) cand = step_interp(a, b, cur, h);
   else cand = cur + ((double)sgnv(nxt) * h);
   if (absv(cand) < absv(nxt)) nxt = cand;
 }
-__device__ inline float sgnh(float v, float h) { return v > 0.f ? h : (v < 0.f ? -h : 0.f); }
-__device__ inline void fwd_step(float& cur, float& nxt, float a, float b, bool act, bool ip, float h) {
-  const float dba = b - a;
-  const float d = -a * h * __builtin_amdgcn_rcpf(dba);
-  const bool moved = ip & (a * b <= 0.f) & (fabsf(cur) > fabsf(d));
-  const float c1 = moved ? -d * (dba > 0.f ? 1.f : (dba < 0.f ? -1.f : 0.f)) : cur;
-  const float cand = c1 + sgnh(ip ? b : nxt, h);
-  const bool take = act & (fabsf(cand) < fabsf(nxt));
-  cur = act ? c1 : cur;
-  nxt = take ? cand : nxt;
-}
 
-// Register-resident forms of the two kernels (boxes up to 32 in both types,
-// up to 48 in FP32): one wavefront per tile, a lane keeps its whole line (out
-// and in values) in registers, the sweeps are unrolled over the line with the
-// reference's loop ranges as predicates, and LDS is used once, to turn rows
-// into columns.  The update order along a line is the same as above, so FP64
-// results are identical; the FP32 steps are written without branches (vector
-// selects), which a sequential recurrence needs to avoid an exec-mask round
-// trip per step.
+// A lane's loop bound as a value the compiler knows nothing about: predicates
+// then compare in vector registers where they are used.  Known bounds (or one
+// copy for several sweeps) made it keep a scalar lane mask per position, up to
+// 670 of them spilled.
+__device__ inline int opaque(int v) {
+  __asm__ volatile("" : "+v"(v));
+  return v;
+}
+constexpr int kNever = 1 << 20;  // a position no line has
+
+// Register-resident forms of the two kernels (boxes up to 48): one wavefront
+// per tile, a lane keeps its whole line (out and in values) in registers, the
+// sweeps are unrolled over the line with the reference's loop ranges as
+// predicates, and LDS is used once, to turn rows into columns.  The update
+// order along a line is the same as above, so FP64 results are identical; the
+// FP32 steps are written without branches (vector selects), which a sequential
+// recurrence needs to avoid an exec-mask round trip per step.
+//
+// The x/y sweeps are bound by vector issue (85 % busy at 8000 FP32 grains),
+// the z sweeps by HBM (3.9 TB/s in FP32).  Per step, 8000 grains, FP64: x/y
+// 3.83 ms with the n <= 48 lines in LDS, 2.36 with them in registers, 2.15
+// with the sweeps' steps as below; z 2.60 and 1.37.  FP32: x/y 1.16 and 1.08,
+// z 0.76 and 0.73.
 
 // x/y sweeps of one output layer.  LDS B first holds the in/out intersection of
 // the input layer (read as rows), then the swept out rows (read as columns).
@@ -334,12 +365,16 @@ struct XYTile {
   bool do_xy, tv;
 };
 
+// A step before a line's first point (or past its last) needs no predicate
+// where it changes nothing: out is -1 before the first point, and -1 - h is no
+// candidate; past the box side only positions that are never stored change.
 template <class T, int NMAX, int NS, int LW>
-__device__ __forceinline__ void xy_sweeps(T* B, const XYTile& t, int xlo, int xim, int ylo, int yim, int nol, int ln,
-                                          T h) {
+__device__ __forceinline__ void xy_sweeps(T* B, const XYTile& t, int ln, T h) {
   constexpr int S = NMAX + 1;
   const T* src = (const T*)t.src;
   const int no = t.no, ni = t.ni;
+  // loop ranges in box coordinates; im: the last input point
+  const int xlo = t.ixmin - t.ox0, xim = t.ixmax - 1 - t.ox0, ylo = t.iymin - t.oy0, yim = t.iymax - 1 - t.oy0;
   T o[NS], in[NS];
 #pragma unroll
   for (int q = 0; q < NS; ++q) {
@@ -358,13 +393,18 @@ __device__ __forceinline__ void xy_sweeps(T* B, const XYTile& t, int xlo, int xi
     const bool inrow = r <= yim;
 #pragma unroll
     for (int q = 0; q < NS; ++q) in[q] = B[r * S + q];
+    {
+      const int lo = opaque(xlo);
+      const unsigned span = (unsigned)opaque(inrow ? xim - xlo : 0);
 #pragma unroll
-    for (int q = 0; q < NS - 1; ++q)
-      fwd_step(o[q], o[q + 1], in[q], in[q + 1], (q >= xlo) & (q < nol), (q < xim) & inrow, h);
+      for (int q = 0; q < NS - 1; ++q)
+        sweep_step(o[q], o[q + 1], in[q], in[q + 1], true, (unsigned)(q - lo) < span, h);
+    }
+    const int last = opaque(xim), first = opaque(inrow ? xlo : kNever);
 #pragma unroll
     for (int q = NS - 1; q >= 1; --q) {
-      const T cand = o[q] + ((T)sgnv(((q > xlo) & inrow) ? in[q - 1] : o[q - 1]) * h);
-      o[q - 1] = ((q <= xim) & (absv(cand) < absv(o[q - 1]))) ? cand : o[q - 1];
+      const T cand = o[q] + sgnh(q > first ? in[q - 1] : o[q - 1], h);
+      o[q - 1] = ((q <= last) & (absv(cand) < absv(o[q - 1]))) ? cand : o[q - 1];
     }
   }
   __syncthreads();
@@ -384,17 +424,23 @@ __device__ __forceinline__ void xy_sweeps(T* B, const XYTile& t, int xlo, int xi
       const bool incol = c <= xim;
       if (incol) {
         const T* scol = src + (t.ox0 + c - t.ib[0]) + (int64_t)(t.oy0 - t.ib[1]) * ni;  // scol[q * ni] = in(oy0 + q, j)
+        const int lo = opaque(ylo), last = opaque(yim);
 #pragma unroll
         for (int q = 0; q < NS; ++q)
-          if (q >= ylo && q <= yim) in[q] = scol[(int64_t)q * ni];
+          if (q >= lo && q <= last) in[q] = scol[(int64_t)q * ni];
       }
+      {
+        const int lo = opaque(ylo);
+        const unsigned span = (unsigned)opaque(incol ? yim - ylo : 0);
 #pragma unroll
-      for (int q = 0; q < NS - 1; ++q)
-        fwd_step(o[q], o[q + 1], in[q], in[q + 1], (q >= ylo) & (q < nol), incol & (q < yim), h);
+        for (int q = 0; q < NS - 1; ++q)
+          sweep_step(o[q], o[q + 1], in[q], in[q + 1], q >= lo, (unsigned)(q - lo) < span, h);
+      }
+      const int last = opaque(yim), first = opaque(incol ? ylo : kNever);
 #pragma unroll
       for (int q = NS - 1; q >= 1; --q) {
-        const T cand = o[q] + ((T)sgnv((incol & (q > ylo)) ? in[q - 1] : o[q - 1]) * h);
-        o[q - 1] = ((q <= yim) & (absv(cand) < absv(o[q - 1]))) ? cand : o[q - 1];
+        const T cand = o[q] + sgnh(q > first ? in[q - 1] : o[q - 1], h);
+        o[q - 1] = ((q <= last) & (absv(cand) < absv(o[q - 1]))) ? cand : o[q - 1];
       }
     }
   }
@@ -440,19 +486,14 @@ __global__ __launch_bounds__(64) void k_redist_xy_reg(SimParams sp, PlanDev P, i
     const bool do_xy = tv && !empty && k >= izmin && k < izmax - 1;
     const XYTile t{ib, ain + din.off[g] + (int64_t)(k - ib[2]) * ni * ni, aout + dout.off[g] + (int64_t)kl * no * no,
                    ni, ox0, oy0, no, iymin, iymax, ixmin, ixmax, do_xy, tv};
-    // local (box) coordinates of the loop ranges
-    // loop-range bounds as per-lane values: the predicates below then compare in
-    // vector registers instead of building a scalar lane mask for every step
-    int xlo = ixmin - ox0, xim = ixmax - 1 - ox0, ylo = iymin - oy0, yim = iymax - 1 - oy0, nol = no - 1;
-    __asm__ volatile("" : "+v"(xlo), "+v"(xim), "+v"(ylo), "+v"(yim), "+v"(nol));
     // the wavefront's largest box side picks the sweep length
     int nw = tv ? no : 0;
     if constexpr (PACK == 2) nw = max(nw, __shfl_xor(nw, 32));
     nw = __builtin_amdgcn_readfirstlane(nw);
-    if (nw <= NMAX - 12) xy_sweeps<T, NMAX, NMAX - 12, LW>(B, t, xlo, xim, ylo, yim, nol, ln, h);
-    else if (nw <= NMAX - 8) xy_sweeps<T, NMAX, NMAX - 8, LW>(B, t, xlo, xim, ylo, yim, nol, ln, h);
-    else if (nw <= NMAX - 4) xy_sweeps<T, NMAX, NMAX - 4, LW>(B, t, xlo, xim, ylo, yim, nol, ln, h);
-    else xy_sweeps<T, NMAX, NMAX, LW>(B, t, xlo, xim, ylo, yim, nol, ln, h);
+    if (nw <= NMAX - 12) xy_sweeps<T, NMAX, NMAX - 12, LW>(B, t, ln, h);
+    else if (nw <= NMAX - 8) xy_sweeps<T, NMAX, NMAX - 8, LW>(B, t, ln, h);
+    else if (nw <= NMAX - 4) xy_sweeps<T, NMAX, NMAX - 4, LW>(B, t, ln, h);
+    else xy_sweeps<T, NMAX, NMAX, LW>(B, t, ln, h);
   }
 }
 
@@ -464,6 +505,7 @@ __global__ __launch_bounds__(64) void k_redist_xy_reg(SimParams sp, PlanDev P, i
 template <class T, int NMAX>
 __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(sizeof(T) == 4 && NMAX == 48 ? 3 : 1)))
 void k_redist_z_reg(SimParams sp, PlanDev P, int cls, DescDev din, DescDev dout) {
+  constexpr bool FP32 = sizeof(T) == 4;
   const int total = P.totals[kQCols * kClasses + cls];
   const T* __restrict__ ain = (const T*)din.arena;
   T* __restrict__ aout = (T*)dout.arena;
@@ -493,22 +535,45 @@ void k_redist_z_reg(SimParams sp, PlanDev P, int cls, DescDev din, DescDev dout)
     if (!empty && i >= iymin && j >= ixmin) {
       const bool inside = i < iymax && j < ixmax;
       int zlo = izmin - oz0, zim = izmax - 1 - oz0, nol = no - 1;
-      __asm__ volatile("" : "+v"(zlo), "+v"(zim), "+v"(nol));  // per-lane predicates (see above)
+      // FP64: one opaque copy for all uses and branches around the steps out of
+      // range (the positions past the side, a third of them at side 33)
+      if constexpr (!FP32) zlo = opaque(zlo), zim = opaque(zim), nol = opaque(nol);
       if (inside) {
         const int64_t lsi = (int64_t)ni * ni;
         const T* ic = ain + din.off[g] + (int64_t)(i - ib[1]) * ni + (j - ib[0]) + (int64_t)(oz0 - ib[2]) * lsi;
+        const int lo = FP32 ? opaque(zlo) : zlo, last = FP32 ? opaque(zim) : zim;
 #pragma unroll
         for (int q = 0; q < NMAX; ++q)
-          if (q >= zlo && q <= zim) in[q] = ic[q * lsi];
+          if (q >= lo && q <= last) in[q] = ic[q * lsi];
       }
+      if constexpr (FP32) {
+        const int lo = opaque(zlo);
+        const unsigned span = (unsigned)opaque(inside ? zim - zlo : 0);
 #pragma unroll
-      for (int q = 0; q < NMAX - 1; ++q)
-        fwd_step(o[q], o[q + 1], in[q], in[q + 1], (q >= zlo) & (q < nol), (q < zim) & inside, h);
+        for (int q = 0; q < NMAX - 1; ++q)
+          sweep_step(o[q], o[q + 1], in[q], in[q + 1], q >= lo, (unsigned)(q - lo) < span, h);
+      } else {
+#pragma unroll
+        for (int q = 0; q < NMAX - 1; ++q)
+          branch_step(o[q], o[q + 1], in[q], in[q + 1], (q >= zlo) & (q < nol), (q < zim) & inside, h);
+      }
       // z-backward interpolates too: the same step towards q - 1
+      if constexpr (FP32) {
+        const int lo = opaque(zlo), last = opaque(zim);
+        const unsigned span = (unsigned)opaque(inside ? zim - zlo : 0);
 #pragma unroll
-      for (int q = NMAX - 1; q >= 1; --q)
-        fwd_step(o[q], o[q - 1], in[q], in[q - 1], q <= zim, (q > zlo) & inside, h);
+        for (int q = NMAX - 1; q >= 1; --q)
+          sweep_step(o[q], o[q - 1], in[q], in[q - 1], q <= last, (unsigned)(q - 1 - lo) < span, h);
+      } else {
+#pragma unroll
+        for (int q = NMAX - 1; q >= 1; --q)
+          branch_step(o[q], o[q - 1], in[q], in[q - 1], q <= zim, (q > zlo) & inside, h);
+      }
     }
+    // the layer offsets are made again for the stores (kept from the loads they
+    // would take two scalar registers each, and spill)
+    int64_t lso = ls;
+    if constexpr (FP32) __asm__ volatile("" : "+s"(lso));
     // clampValues(-delta, delta) (src/dimensionalBufferReal.h:44-57)
 #pragma unroll
     for (int q = 0; q < NMAX; ++q) {
@@ -516,7 +581,7 @@ void k_redist_z_reg(SimParams sp, PlanDev P, int cls, DescDev din, DescDev dout)
         T v = o[q];
         if (v < -dl) v = -dl;
         else if (v > dl) v = dl;
-        oc[q * ls] = v;
+        oc[q * lso] = v;
       }
     }
   }
@@ -532,34 +597,25 @@ void xy_class(const Launch& L, const SimParams& sp, const PlanDev& P, int cls, c
 template <class T>
 void redist_all(const Launch& L, int part, const SimParams& sp, const PlanDev& P, const DescDev& din,
                 const DescDev& dout, int32_t* err, int c0, int c1) {
-  // register-resident lines for boxes up to 32 (both types) and up to 48 (FP32)
-  constexpr bool reg48 = sizeof(T) == 4;
+  // register-resident lines for boxes up to 48; a line of 64 does not fit a
+  // lane's registers twice over
   auto in = [&](int c) { return c0 <= c && c < c1; };
   if (part == 0) {
     if (in(0))
       hipLaunchKernelGGL((k_redist_xy_reg<T, 32>), dim3(tile_grid(L, kGridPerCU, 0, sp.N, layers_of(0) / 2)), dim3(64), 0, L.stream, sp, P, 0,
                          din, dout, err);
-    if (in(1)) {
-      if constexpr (reg48)
-        hipLaunchKernelGGL((k_redist_xy_reg<T, 48>), dim3(tile_grid(L, kGridPerCU, 1, sp.N, layers_of(1))), dim3(64), 0, L.stream, sp, P,
-                           1, din, dout, err);
-      else
-        xy_class<T, 48>(L, sp, P, 1, din, dout, err);
-    }
+    if (in(1))
+      hipLaunchKernelGGL((k_redist_xy_reg<T, 48>), dim3(tile_grid(L, kGridPerCU, 1, sp.N, layers_of(1))), dim3(64), 0, L.stream, sp, P, 1,
+                         din, dout, err);
     if (in(2)) xy_class<T, 64>(L, sp, P, 2, din, dout, err);
     if (in(3)) xy_class<T, 96>(L, sp, P, 3, din, dout, err);
   } else {
     if (in(0))
       hipLaunchKernelGGL((k_redist_z_reg<T, 32>), dim3(tile_grid(L, kGridPerCU, 0, sp.N, cols_of(0))), dim3(64), 0, L.stream, sp, P, 0,
                          din, dout);
-    if (in(1)) {
-      if constexpr (reg48)
-        hipLaunchKernelGGL((k_redist_z_reg<T, 48>), dim3(tile_grid(L, kGridPerCU, 1, sp.N, cols_of(1))), dim3(64), 0, L.stream, sp, P, 1,
-                           din, dout);
-      else
-        hipLaunchKernelGGL((k_redist_z<T, 48>), dim3(tile_grid(L, kGridPerCU, 1, sp.N, cols_of(1))), dim3(64), 0, L.stream, sp, P, 1,
-                           din, dout);
-    }
+    if (in(1))
+      hipLaunchKernelGGL((k_redist_z_reg<T, 48>), dim3(tile_grid(L, kGridPerCU, 1, sp.N, cols_of(1))), dim3(64), 0, L.stream, sp, P, 1,
+                         din, dout);
     if (in(2))
       hipLaunchKernelGGL((k_redist_z<T, 64>), dim3(tile_grid(L, kGridPerCU, 2, sp.N, cols_of(2))), dim3(64), 0, L.stream, sp, P, 2, din,
                          dout);
