@@ -76,23 +76,29 @@ __device__ inline bool deep_inside(int j, int i, int k, int gb, int m) {
 // running maximum and its id for each of the run's layers in registers.  The
 // neighbour table is walked once per wavefront, in list order: an entry whose
 // box overlaps the run in z and whose rectangle covers some lane's column
-// gives each covered lane its offset in the neighbour's layer once, then its
-// values over the run's layers are gathered QB at a time (independent loads,
-// the layer index clamped into the entry's z range so every address is inside
-// the neighbour's box; lanes off the rectangle read its first voxel) and the
-// maxima are updated with a strict '>' (ties keep the earlier entry: the
-// reference's order).  The per-entry set-up is paid once per ZL layers, there
-// is no LDS and no barrier.  Then, per voxel, the wall distance, IDLocal (new
-// id or the stale one), the set-comparison and the bounding box, as above.
+// gives each covered lane its offset in the neighbour's layer once, then the
+// covered lanes alone gather its values over the run's layers QB at a time
+// (independent loads, the byte offset clamped in vector registers to the
+// entry's layers, so every address is inside the neighbour's box) and the
+// maxima of the layers it covers are updated with a strict '>' (ties keep the
+// earlier entry: the reference's order).  The per-entry set-up is paid once per
+// ZL layers, there is no LDS and no barrier.  Then, per voxel, the wall
+// distance, IDLocal (new id or the stale one), the set-comparison and the
+// bounding box, as above.
+// Bound: the latency of the gathers (69 % of a wavefront's cycles), at 8.9 TB/s
+// from L2.  Gathers by all 64 lanes, those off the rectangle reading a voxel
+// that no one needs, with the layer clamps and range masks in the scalar unit
+// took 12.7 instead of 4.9 L1 accesses and 15 scalar instructions per gather,
+// both units 80 % busy: 2.54 against 2.21 ms at 8000 FP32 grains, 3.91 against
+// 3.84 in FP64.  (A branch around each load as well, instead of the clamp,
+// spills 67 registers: 6.5 ms.)
 // One wavefront tile: column block cb (64 consecutive columns (y, x) of grain
 // g's box) over run zc of ZL z-layers.
 // B16: the winning ids of the run's layers are kept as 16-bit halves, two per
-// register (grain ids below 0xFFFF; 0xFFFF stands for "not covered").  With
-// the spatial kernel's request of eight wavefronts per SIMD (64 vector
-// registers) the FP32 body spills about ten registers, outside the gather
-// loop, and still runs faster than at seven wavefronts with unpacked ids
-// (3.33 against 3.65 ms at 8000 grains, measured with a grid-stride launch of
-// 64 workgroups per CU).
+// register (grain ids below 0xFFFF; 0xFFFF stands for "not covered").  The
+// FP32 spatial kernel then asks for seven wavefronts per SIMD, which need no
+// spill (eight spill 8 registers, and the same time); FP64 has five (six, with
+// 4 registers spilled: 3.83 against 3.76 ms at 8000 grains).
 template <bool B16>
 __device__ inline uint32_t bid_get(const uint32_t* bid, int q) {
   if constexpr (!B16) return bid[q];
@@ -135,6 +141,8 @@ __device__ inline void cmp_tile(const SimParams& sp, int g, int cb, int zc, cons
   const int4* tab = ld.tab + (int64_t)g * maxL;
   const int32_t* tid_of = ld.tab_id + (int64_t)g * maxL;
   const int len = ld.tab_len[g];
+  // rows of the wavefront's columns
+  const int ya = (cb * 64) / n, yb = min(cb * 64 + 63, nn2 - 1) / n;
   for (int pb = 0; pb < len; pb += 64) {
     const int idx = pb + lane;
     bool keep = false;
@@ -145,7 +153,8 @@ __device__ inline void cmp_tile(const SimParams& sp, int g, int cb, int zc, cons
       nb = tid_of[idx];
       q2 = e.w & 0xFFFF;
       q5 = (int)((uint32_t)e.w >> 16);
-      keep = q2 < zlo + qn && q5 > zlo;  // the neighbour's box meets the run's layers
+      // the neighbour's box meets the run's layers, its rectangle the wavefront's rows
+      keep = q2 < zlo + qn && q5 > zlo && (int)(((uint32_t)e.z >> 16) & 0xFF) <= yb && (int)((uint32_t)e.z >> 24) > ya;
     }
     uint64_t m = __ballot(keep);
     while (m) {
@@ -154,8 +163,7 @@ __device__ inline void cmp_tile(const SimParams& sp, int g, int cb, int zc, cons
       const uint32_t rc = (uint32_t)__builtin_amdgcn_readlane((int)(uint32_t)e.z, a);
       const int rx0 = rc & 0xFF, rx1 = (rc >> 8) & 0xFF, ry0 = (rc >> 16) & 0xFF, ry1 = rc >> 24;
       const bool cov = act & ((uint32_t)(xl - rx0) < (uint32_t)(rx1 - rx0)) & ((uint32_t)(yl - ry0) < (uint32_t)(ry1 - ry0));
-      const uint64_t cmask = __ballot(cov);
-      if (cmask == 0) continue;  // the rectangle misses this wavefront's columns
+      if (__ballot(cov) == 0) continue;  // the rectangle misses this wavefront's columns
       const uint32_t id = (uint32_t)__builtin_amdgcn_readlane(nb, a);
       const uint32_t elo = (uint32_t)__builtin_amdgcn_readlane(e.x, a);
       const uint32_t ehi = (uint32_t)__builtin_amdgcn_readlane(e.y, a);
@@ -164,31 +172,35 @@ __device__ inline void cmp_tile(const SimParams& sp, int g, int cb, int zc, cons
       const int eq2 = __builtin_amdgcn_readlane(q2, a), eq5 = __builtin_amdgcn_readlane(q5, a);
       const int qa = max(eq2, zlo) - zlo, qb = min(eq5, zlo + qn) - zlo;  // run layers the entry covers
       const int ls = nn * nn;
-      // layer zlo + qa of the neighbour; element q of the run is at (q - qa) * ls + off from it
-      const T* __restrict__ src = ain + B + (int64_t)(zlo + qa - eq2) * ls;
-      // lanes off the rectangle read the first covered lane's voxel: a line the
-      // gather fetches anyway (the rectangle's first voxel of every layer would
-      // be one more line per gather)
-      const uint32_t offc = (uint32_t)((yl - ry0) * nn + (xl - rx0));
-      const uint32_t off0 = (uint32_t)__builtin_amdgcn_readlane((int)offc, (int)__builtin_ctzll(cmask));
-      const uint32_t off = cov ? offc : off0;
+      // layer zlo + qa of the neighbour's rectangle
+      const char* __restrict__ src = (const char*)(ain + B + (int64_t)(zlo + qa - eq2) * ls);
+      const int lsb = ls * (int)sizeof(T);
+      const uint32_t in = (qb < 32 ? (1u << qb) - 1u : ~0u) & ~((1u << qa) - 1u);  // covered layers, one bit each
+      if (cov) {
+        const int vlo = ((yl - ry0) * nn + (xl - rx0)) * (int)sizeof(T);
+        const int vhi = vlo + (qb - 1 - qa) * lsb;
 #pragma unroll
-      for (int c0 = 0; c0 < ZL; c0 += QB) {
-        if (c0 >= qb || c0 + QB <= qa) continue;
-        T v[QB];
+        for (int c0 = 0; c0 < ZL; c0 += QB) {
+          constexpr uint32_t kAll = QB < 32 ? (1u << (QB & 31)) - 1u : ~0u;
+          const uint32_t bits = (in >> c0) & kAll;
+          if (bits == 0) continue;
+          int vo = vlo + (c0 - qa) * lsb;
+          T v[QB];
 #pragma unroll
-        for (int u = 0; u < QB; ++u) {
-          const int qc = min(max(c0 + u, qa), qb - 1) - qa;
-          // 32-bit byte offset from a wavefront-uniform base
-          v[u] = *(const T*)((const char*)src + (uint32_t)((qc * ls + (int)off) * (int)sizeof(T)));
-        }
+          for (int u = 0; u < QB; ++u) {
+            v[u] = *(const T*)(src + (uint32_t)min(max(vo, vlo), vhi));
+            vo += lsb;
+          }
 #pragma unroll
-        for (int u = 0; u < QB; ++u) {
-          const int q = c0 + u;
-          const bool up = cov & (q >= qa) & (q < qb) & (v[u] > best[q]);
-          best[q] = up ? v[u] : best[q];
-          const int w = B16 ? (q >> 1) : q;
-          bid[w] = up ? bid_with<B16>(bid[w], q, id) : bid[w];
+          for (int u = 0; u < QB; ++u) {
+            if ((bits >> u) & 1u) {
+              __asm__ volatile("" : "+v"(v[u]));  // a uniform branch, not masks (2.21 against 2.28 ms)
+              const int q = c0 + u, w = B16 ? (q >> 1) : q;
+              const bool up = v[u] > best[q];
+              best[q] = up ? v[u] : best[q];
+              bid[w] = up ? bid_with<B16>(bid[w], q, id) : bid[w];
+            }
+          }
         }
       }
     }
@@ -201,15 +213,15 @@ __device__ inline void cmp_tile(const SimParams& sp, int g, int cb, int zc, cons
   const int64_t oldsize = (int64_t)(olb[3] - olb[0]) * (olb[4] - olb[1]) * (olb[5] - olb[2]);
   const uint32_t* __restrict__ idl_old = ilo.arena + ilo.off[g];
   uint32_t* __restrict__ idl_new = iln.arena + iln.off[g];
-  const T* own = ain + din.off[g];
+  const T* __restrict__ own = ain + din.off[g];
   T* dst = aout + dout.off[g];
   const int i = y0 + yl, j = x0 + xl;
   int kmin = INT_MAX, kmax = -INT_MAX;
+  if (wall) {
 #pragma unroll
-  for (int q = 0; q < ZL; ++q) {
-    if (q >= qn || !act) continue;
-    const int k = zlo + q;
-    if (wall && !deep_inside(j, i, k, sp.gb, sp.ngp)) {
+    for (int q = 0; q < ZL; ++q) {
+      const int k = zlo + q;
+      if (q >= qn || !act || deep_inside(j, i, k, sp.gb, sp.ngp)) continue;
       const double dist = bc_dist(j, i, k, x0, y0, z0, x1, y1, sp.gb, sp.ngp);
       if (dist > -sp.gb) {
         const T dh = (T)(dist * sp.h);
@@ -220,16 +232,38 @@ __device__ inline void cmp_tile(const SimParams& sp, int g, int cb, int zc, cons
         }
       }
     }
-    const int64_t li = (int64_t)(qlo + q) * nn2 + col;
-    uint32_t idv = bid_get<B16>(bid, q);
-    if (idv == 0xFFFFFFFFu) idv = li < oldsize ? idl_old[li] : 0u;
-    idl_new[li] = idv;
-    const T a_in = own[li];
-    const T o = (a_in < T(0) ? -a_in : a_in) < lim ? (T)0.5 * (a_in - best[q]) : a_in;
-    dst[li] = o;
-    if (o >= T(0)) {
-      kmin = min(kmin, k);
-      kmax = max(kmax, k);
+  }
+  // TB layers at a time, their loads (own value; previous id where nothing
+  // covers the voxel) before their stores: one latency per TB layers instead of
+  // one per layer (FP32 2.20 -> 2.12 ms at 8000 grains, FP64 3.84 -> 3.76)
+  constexpr int TB = sizeof(T) == 4 ? 8 : 4;
+#pragma unroll
+  for (int c0 = 0; c0 < ZL; c0 += TB) {
+    if (c0 >= qn) continue;
+    T av[TB];
+    uint32_t idv[TB];
+    if (act) {
+#pragma unroll
+      for (int u = 0; u < TB; ++u) av[u] = own[(int64_t)(qlo + min(c0 + u, qn - 1)) * nn2 + col];
+#pragma unroll
+      for (int u = 0; u < TB; ++u) {
+        const int64_t li = (int64_t)(qlo + min(c0 + u, qn - 1)) * nn2 + col;
+        idv[u] = bid_get<B16>(bid, c0 + u);
+        if (idv[u] == 0xFFFFFFFFu) idv[u] = li < oldsize ? idl_old[li] : 0u;
+      }
+#pragma unroll
+      for (int u = 0; u < TB; ++u) {
+        const int q = c0 + u, k = zlo + q;
+        if (q >= qn) continue;
+        const int64_t li = (int64_t)(qlo + q) * nn2 + col;
+        idl_new[li] = idv[u];
+        const T o = (av[u] < T(0) ? -av[u] : av[u]) < lim ? (T)0.5 * (av[u] - best[q]) : av[u];
+        dst[li] = o;
+        if (o >= T(0)) {
+          kmin = min(kmin, k);
+          kmax = max(kmax, k);
+        }
+      }
     }
   }
   // bounding box of the voxels >= 0: the lane's column spans (j, i) x [kmin, kmax]
@@ -463,7 +497,7 @@ __global__ __launch_bounds__(kScanT) void k_scan_add(int32_t* a, int n, const in
 }
 
 template <class T, int ZL, int QB, bool B16>
-__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(B16 && sizeof(T) == 4 ? 8 : 1))) void k_cmp_space(SimParams sp, CmpSpaceDev W, DescDev din, DescDev dout,
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(B16 && sizeof(T) == 4 ? 7 : 1))) void k_cmp_space(SimParams sp, CmpSpaceDev W, DescDev din, DescDev dout,
                                                    ListDev ld, IdlDev ilo, IdlDev iln, int32_t* newb) {
   const int total = min(W.cnt[W.nkeys], W.cap);
   const int wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
