@@ -50,7 +50,10 @@ constexpr int kEW = 256;                           // threads of an element-buil
 constexpr int kRec = kJuncCap + kJuncCap / 2;      // lists + high-order junctions made by merging
 constexpr int kTopoCapBitsC = 6;
 static_assert((1 << kTopoCapBitsC) == kTopoCap, "grain topology table size");
-constexpr int kCorrGridPerCU = 512;  // workgroups per CU of a correction launch: about one per tile
+// workgroups per CU of a correction launch: 16 times what is resident, for
+// balance; each costs its start (correction per step at 20000 grains with 24:
+// 18.7, 64: 18.6, 512: 21.4, one per layer: 23.9 ms)
+constexpr int kCorrGridPerCU = 64;
 
 enum { kClsGB = 0, kClsTL = 1, kClsQJ = 2, kClsHJ = 3 };
 
@@ -180,98 +183,148 @@ __global__ __launch_bounds__(kEW) void k_elements(SimParams sp, const int32_t* _
       s_red[r] = -1;
     }
     __syncthreads();
-    if (tid == 0) {
-      int nh = 0, nq = 0, nrec = nl;
-      for (int r = 0; r < nl; ++r) {
-        if (s_cls[r] == kClsHJ) s_hj[nh++] = (short)r;
-        else if (s_cls[r] == kClsQJ) s_qj[nq++] = (short)r;
-      }
-      // junction position = mean barycenter (computePosition); distance of two
-      auto near = [&](int a, int b) {
-        const double na = (double)s_cnt[a], nb = (double)s_cnt[b];
-        const double dx = s_sx[a] / na - s_sx[b] / nb, dy = s_sy[a] / na - s_sy[b] / nb,
-                     dz = s_sz[a] / na - s_sz[b] / nb;
-        return sqrt(dx * dx + dy * dy + dz * dz) < 2;
+    // the merges and the order, by the first wavefront: every scan of a list for
+    // the first near junction takes 64 of its entries at a time (one lane
+    // testing one pair after the other: k_elements took 5.8 ms per step at 20000
+    // grains, 82 % of it waiting; 1.0 ms this way); a merged entry is marked, not closed up
+    if (tid < 64) {
+      const int lane = tid;
+      const unsigned long long below = (1ull << lane) - 1ull;
+      auto settle = [] {  // what one lane wrote, before any lane reads it
+        __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+        __builtin_amdgcn_wave_barrier();
       };
-      auto absorb = [&](int h, int b) {  // mergeWith: b's barycenters and ids join h
-        s_cnt[h] += s_cnt[b];
-        s_sx[h] += s_sx[b];
-        s_sy[h] += s_sy[b];
-        s_sz[h] += s_sz[b];
-        s_em[h] |= s_em[b];
-        s_en[h] = s_mo[h] = 1.0;
-        s_red[b] = (short)h;
+      int nh = 0, nq = 0, nrec = nl;
+      for (int r0 = 0; r0 < nl; r0 += 64) {
+        const int c = r0 + lane < nl ? (int)s_cls[r0 + lane] : -1;
+        const unsigned long long mh = __ballot(c == kClsHJ), mq = __ballot(c == kClsQJ);
+        if (c == kClsHJ) s_hj[nh + __popcll(mh & below)] = (short)(r0 + lane);
+        if (c == kClsQJ) s_qj[nq + __popcll(mq & below)] = (short)(r0 + lane);
+        nh += __popcll(mh);
+        nq += __popcll(mq);
+      }
+      settle();
+      // first entry of list[lo, n) whose junction lies within 2 of record a's
+      // (position = mean barycenter, computePosition), -1: none
+      auto first_near = [&](int a, const short* list, int lo, int n) {
+        const double na = (double)s_cnt[a];
+        const double ax = s_sx[a] / na, ay = s_sy[a] / na, az = s_sz[a] / na;
+        for (int j0 = lo; j0 < n; j0 += 64) {
+          const int b = j0 + lane < n ? (int)list[j0 + lane] : -1;
+          bool hit = false;
+          if (b >= 0) {
+            const double nb = (double)s_cnt[b];
+            const double dx = ax - s_sx[b] / nb, dy = ay - s_sy[b] / nb, dz = az - s_sz[b] / nb;
+            hit = sqrt(dx * dx + dy * dy + dz * dz) < 2;
+          }
+          const unsigned long long m = __ballot(hit);
+          if (m) return j0 + (int)__builtin_ctzll(m);
+        }
+        return -1;
+      };
+      auto absorb = [&](int h, short* list, int at) {  // mergeWith: the entry's barycenters and ids join h
+        if (lane == 0) {
+          const int b = list[at];
+          s_cnt[h] += s_cnt[b];
+          s_sx[h] += s_sx[b];
+          s_sy[h] += s_sy[b];
+          s_sz[h] += s_sz[b];
+          s_em[h] |= s_em[b];
+          s_en[h] = s_mo[h] = 1.0;
+          s_red[b] = (short)h;
+          list[at] = -1;
+        }
+        settle();
       };
       // mergeJunction (src/grainHull.cpp:483-531)
-      for (int i = 0; i < nq; i++) {
-        for (int j = i + 1; j < nq; j++) {
-          const int A = s_qj[i], B = s_qj[j];
-          if (near(A, B)) {
-            // HighOrderJunction(A, B): A's ids (B adds only ids A has), A's then
-            // B's barycenters
-            const int h = nrec++;
-            s_em[h] = s_em[A];
-            s_cnt[h] = s_cnt[A];
-            s_sx[h] = s_sx[A];
-            s_sy[h] = s_sy[A];
-            s_sz[h] = s_sz[A];
-            s_cls[h] = kClsHJ;
-            s_red[h] = -1;
-            absorb(h, B);
-            s_em[h] = s_em[A];
-            s_red[A] = (short)h;
-            for (int t = j; t + 1 < nq; ++t) s_qj[t] = s_qj[t + 1];
-            --nq;
-            for (int t = i; t + 1 < nq; ++t) s_qj[t] = s_qj[t + 1];
-            --nq;
-            i--;
-            s_hj[nh++] = (short)h;
-            break;
-          }
+      for (int i = 0; i < nq; ++i) {
+        const int A = s_qj[i];
+        if (A < 0) continue;
+        const int j = first_near(A, s_qj, i + 1, nq);
+        if (j < 0) continue;
+        // HighOrderJunction(A, B): A's ids (B adds only ids A has), A's then B's
+        // barycenters
+        const int h = nrec++;
+        if (lane == 0) {
+          const int B = s_qj[j];
+          s_em[h] = s_em[A];
+          s_cnt[h] = s_cnt[A] + s_cnt[B];
+          s_sx[h] = s_sx[A] + s_sx[B];
+          s_sy[h] = s_sy[A] + s_sy[B];
+          s_sz[h] = s_sz[A] + s_sz[B];
+          s_en[h] = s_mo[h] = 1.0;
+          s_cls[h] = kClsHJ;
+          s_red[h] = -1;
+          s_red[A] = s_red[B] = (short)h;
+          s_qj[i] = s_qj[j] = -1;
+          s_hj[nh] = (short)h;
         }
+        ++nh;
+        settle();
       }
-      for (int k = 0; k < nh; k++)
-        for (int i = 0; i < nq; i++)
-          if (near(s_qj[i], s_hj[k])) {
-            absorb(s_hj[k], s_qj[i]);
-            for (int t = i; t + 1 < nq; ++t) s_qj[t] = s_qj[t + 1];
-            --nq;
-            i--;
-          }
-      for (int i = 0; i < nh; i++)
-        for (int k = i + 1; k < nh; k++)
-          if (near(s_hj[i], s_hj[k])) {
-            absorb(s_hj[i], s_hj[k]);
-            for (int t = k; t + 1 < nh; ++t) s_hj[t] = s_hj[t + 1];
-            --nh;
-            k--;
-          }
+      for (int k = 0; k < nh; ++k) {
+        const int h = s_hj[k];
+        for (int i = 0; (i = first_near(h, s_qj, i, nq)) >= 0; ++i) absorb(h, s_qj, i);
+      }
+      for (int i = 0; i < nh; ++i) {
+        const int h = s_hj[i];
+        if (h < 0) continue;
+        for (int k = i + 1; (k = first_near(h, s_hj, k, nh)) >= 0; ++k) absorb(h, s_hj, k);
+      }
       // projection order: high-order junctions, quadruple junctions, triple
       // lines, boundaries
       int E = 0;
-      for (int t = 0; t < nh; ++t) s_ord[E++] = s_hj[t];
-      for (int t = 0; t < nq; ++t) s_ord[E++] = s_qj[t];
-      for (int r = 0; r < nl; ++r)
-        if (s_cls[r] == kClsTL) s_ord[E++] = (short)r;
-      const int ntl = E - nh - nq;
-      for (int r = 0; r < nl; ++r)
-        if (s_cls[r] == kClsGB) s_ord[E++] = (short)r;
-      int64_t acc = 0;
+      auto append = [&](bool take, int rec) {
+        const unsigned long long m = __ballot(take);
+        if (take) s_ord[E + __popcll(m & below)] = (short)rec;
+        E += __popcll(m);
+      };
+      auto append_list = [&](const short* list, int n) {
+        for (int t0 = 0; t0 < n; t0 += 64) {
+          const int rec = t0 + lane < n ? (int)list[t0 + lane] : -1;
+          append(rec >= 0, rec);
+        }
+      };
+      auto append_class = [&](int cls) {
+        for (int r0 = 0; r0 < nl; r0 += 64) append(r0 + lane < nl && s_cls[min(r0 + lane, nl - 1)] == cls, r0 + lane);
+      };
+      append_list(s_hj, nh);
+      const int eh = E;
+      append_list(s_qj, nq);
+      const int eq = E;
+      append_class(kClsTL);
+      const int et = E;
+      append_class(kClsGB);
+      settle();
+      long long acc = 0;
       int32_t* ef = cd.efirst + (int64_t)g * (kElemCap + 1);
-      for (int e = 0; e < E; ++e) {
-        s_elem[s_ord[e]] = (short)e;
-        ef[e] = (int32_t)acc;
-        acc += s_cnt[s_ord[e]];
+      for (int e0 = 0; e0 < E; e0 += 64) {
+        const int e = e0 + lane;
+        const int rec = e < E ? (int)s_ord[e] : 0;
+        const long long c = e < E ? (long long)s_cnt[rec] : 0ll;
+        long long incl = c;
+#pragma unroll
+        for (int d = 1; d < 64; d <<= 1) {
+          const long long u = __shfl_up(incl, d, 64);
+          if (lane >= d) incl += u;
+        }
+        if (e < E) {
+          s_elem[rec] = (short)e;
+          ef[e] = (int32_t)(acc + incl - c);
+        }
+        acc += __shfl(incl, 63, 64);
       }
-      ef[E] = (int32_t)acc;
-      const unsigned long long tb = atomicAdd(cd.tri_n, (unsigned long long)acc);
-      if (tb + (unsigned long long)acc > (unsigned long long)cd.tri_cap) atomicOr(err, kErrTri);
-      cd.tbase[g] = (int64_t)tb;
-      cd.ecount[g] = E;
-      cd.eclass[4 * g] = nh;
-      cd.eclass[4 * g + 1] = nq;
-      cd.eclass[4 * g + 2] = ntl;
-      s_E = E;
+      if (lane == 0) {
+        ef[E] = (int32_t)acc;
+        const unsigned long long tb = atomicAdd(cd.tri_n, (unsigned long long)acc);
+        if (tb + (unsigned long long)acc > (unsigned long long)cd.tri_cap) atomicOr(err, kErrTri);
+        cd.tbase[g] = (int64_t)tb;
+        cd.ecount[g] = E;
+        cd.eclass[4 * g] = eh;
+        cd.eclass[4 * g + 1] = eq - eh;
+        cd.eclass[4 * g + 2] = et - eq;
+        s_E = E;
+      }
     }
     __syncthreads();
     const int E = s_E;
@@ -379,7 +432,9 @@ __global__ __launch_bounds__(256) void k_tri_scatter(TopoDev topo, CorrDev cd) {
 // against 146 and, for chunk boxes, 3.4 of the FP64 search over boxed chunks
 // that it replaced; queueing and output are about 9 ms of it, the rest is the
 // minima (vector) behind the products, at four wavefronts per SIMD (128
-// registers; three: 28.9 ms).  128 voxels per search read each row once for
+// registers; three: 28.9 ms).  Tiles dealt to the XCDs and fewer workgroups
+// (below) have since brought k_correct to 18.6 ms, and runs of 8 layers instead
+// of 4 for n <= 32 (fuller searches) to 17.9.  128 voxels per search read each row once for
 // four products; 64 took 4 % longer.
 typedef __bf16 v8bf __attribute__((ext_vector_type(8)));
 typedef float v16f __attribute__((ext_vector_type(16)));
@@ -588,6 +643,16 @@ struct Near {
 };
 #pragma float_control(pop)
 
+// The XCD's l-th tile: tiles go to the XCDs in chunks of two or so grains (the
+// grain's rows and tables come from one L2), chunk by chunk in turn.  A search's
+// length depends on how far its grain is from the plane x = y, so ranges of
+// grains that lie together are uneven work (20000 grains: 24.6 ms per step with
+// one range per XCD, 21.4 dealt).
+constexpr int kDealt = 64;
+__device__ inline int dealt_tile(int l) {
+  return (l / kDealt * kXcds + (int)(blockIdx.x % kXcds)) * kDealt + l % kDealt;
+}
+
 // One workgroup per (grain, run of ZT z-layers) of the output box: its band
 // voxels are queued in LDS grouped by the slot of their IDLocal id in the
 // grain's hull-id table, and a wavefront takes up to kTake of one slot at a
@@ -609,10 +674,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4))) void k
   const T* __restrict__ ain = (const T*)din.arena;
   T* __restrict__ aout = (T*)dout.arena;
   const double delta = sp.delta;
-  // consecutive tiles (the layers of one grain) on one XCD: the grain's
-  // rows and tables come from that XCD's L2
-  const TileRange tr = xcd_tiles(total);
-  for (int tile = tr.first; tile < tr.end; tile += tr.step) {
+  for (int l = blockIdx.x / kXcds, tile; (tile = dealt_tile(l)) < total; l += gridDim.x / kXcds) {
     int g, kl;
     plan_tile(P, cls, kQLayers, tile, g, kl);
     if (kl % ZT) continue;  // the plan's tiles are single layers; the first of a run takes the run
@@ -925,7 +987,7 @@ template <class T>
 void correct_classes(const Launch& L, const SimParams& sp, const PlanDev& P, const int32_t* state, const DescDev& din,
                      const DescDev& dout, const IdlDev& il, const TopoDev& topo, const CorrDev& cd, int c0, int c1) {
   if (c0 <= 0 && 0 < c1)
-    hipLaunchKernelGGL((k_correct<T, 32, 4>), dim3(tile_grid(L, kCorrGridPerCU, 0, sp.N, layers_of(0))), dim3(256), 0, L.stream, sp, P, 0,
+    hipLaunchKernelGGL((k_correct<T, 32, 8>), dim3(tile_grid(L, kCorrGridPerCU, 0, sp.N, layers_of(0))), dim3(256), 0, L.stream, sp, P, 0,
                      state, din, dout, il, topo, cd);
   if (c0 <= 1 && 1 < c1)
     hipLaunchKernelGGL((k_correct<T, 48, 4>), dim3(tile_grid(L, kCorrGridPerCU, 1, sp.N, layers_of(1))), dim3(256), 0, L.stream, sp, P, 1,
