@@ -616,12 +616,12 @@ class LevelSetContext:
         return b
 
     def phi(self, gid, which):
+        b = self.bounds(gid, which)
         n = ctypes.c_int64(0)
-        self._chk(lib().gg_download_distance(self.h, int(gid), int(which), None, 0, ctypes.byref(n)))
-        buf = np.empty(max(n.value, 1), dtype=np.float64)
+        buf = np.empty(max(int(np.prod((b[3:] - b[:3]).astype(np.int64))), 1), dtype=np.float64)
         self._chk(lib().gg_download_distance(self.h, int(gid), int(which), _p(buf, ctypes.c_double), buf.size,
                                              ctypes.byref(n)))
-        return self.bounds(gid, which), buf[: n.value]
+        return b, buf[: n.value]
 
     def upload_phi(self, gid, which, values):
         """Overwrite grain gid's distance buffer (which: 0 input, 1 output) with
