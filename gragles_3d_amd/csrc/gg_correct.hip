@@ -376,23 +376,28 @@ __global__ __launch_bounds__(256) void k_tri_scatter(TopoDev topo, CorrDev cd) {
       valid = (unsigned)e < (unsigned)cd.ecount[t.g];  // false only after a table overflow (device error set)
       key = (unsigned)t.g * (unsigned)kElemCap + (unsigned)e;
     }
-    int64_t pos = 0;
+    // one round per distinct (grain, element) among the wavefront's records;
+    // then every leader reserves its run in the same instruction (1.5 ms per
+    // step at 20000 grains; an add in every round, one after the other: 1.75)
+    int lead = lane, at = 0, run = 0;
     bool done = !valid;
-    for (;;) {  // one round per distinct (grain, element) among the wavefront's records
+    for (;;) {
       const unsigned long long pend = __ballot(!done);
       if (pend == 0ull) break;
       const int leader = __ffsll((long long)pend) - 1;
       const unsigned k0 = __shfl(key, leader);
       const bool mine = !done && key == k0;
       const unsigned long long m = __ballot(mine);
-      int b0 = 0;
-      if (lane == leader) b0 = atomicAdd(&cd.ecur[k0], __popcll(m));
-      b0 = __shfl(b0, leader);
       if (mine) {
-        pos = b0 + __popcll(m & ((1ull << lane) - 1ull));
+        lead = leader;
+        at = __popcll(m & ((1ull << lane) - 1ull));
+        run = __popcll(m);
         done = true;
       }
     }
+    int b0 = 0;
+    if (valid && lane == lead) b0 = atomicAdd(&cd.ecur[key], run);
+    const int64_t pos = __shfl(b0, lead) + at;
     if (valid) {
       const int64_t q = cd.tbase[t.g] + cd.efirst[(int64_t)t.g * (kElemCap + 1) + e] + pos;
       if (q < cd.tri_cap) {
@@ -428,14 +433,15 @@ __global__ __launch_bounds__(256) void k_tri_scatter(TopoDev topo, CorrDev cd) {
 //
 // What bounds it: at 20000 grains (5.8e8 band voxels per step) the searches hold
 // 14 groups of 8 rows on average (75 before k_slots leaves out the ones that
-// cannot be nearest), and k_correct takes 24.5 ms per step and k_slots 5.0,
-// against 146 and, for chunk boxes, 3.4 of the FP64 search over boxed chunks
-// that it replaced; queueing and output are about 9 ms of it, the rest is the
-// minima (vector) behind the products, at four wavefronts per SIMD (128
-// registers; three: 28.9 ms).  Tiles dealt to the XCDs and fewer workgroups
-// (below) have since brought k_correct to 18.6 ms, and runs of 8 layers instead
-// of 4 for n <= 32 (fuller searches) to 17.9.  128 voxels per search read each row once for
-// four products; 64 took 4 % longer.
+// cannot be nearest).  The FP64 search over boxed chunks that this replaced took
+// 146 ms per step (and its chunk boxes 3.4); k_correct took 24.5 in this form,
+// with tiles dealt to the XCDs and fewer workgroups (below) 18.6, with runs of 8
+// layers instead of 4 for n <= 32 (fuller searches) 17.9, and with a grain's lists
+// next to each other 17.5; k_slots takes 2.5.
+// Queueing and output are about 9 ms of it, the rest is the minima (vector)
+// behind the products, at four wavefronts per SIMD (128 registers; three: 28.9
+// against 24.5).  128 voxels per search read each row once for four products; 64
+// took 4 % longer.
 typedef __bf16 v8bf __attribute__((ext_vector_type(8)));
 typedef float v16f __attribute__((ext_vector_type(16)));
 constexpr float kFilterEps = 1.0f / 1048576.0f;  // 2^-20
@@ -479,6 +485,9 @@ __global__ __launch_bounds__(256) void k_slots(SimParams sp, const int32_t* __re
   __shared__ unsigned long long s_em[kElemCap];
   __shared__ int s_ef[kElemCap + 1];
   __shared__ int s_rho;
+  __shared__ double s_q0[kTopoCap][4];  // per slot: its nearest barycenter to the box centre, and R
+  __shared__ int s_groups[kTopoCap], s_first[kTopoCap];
+  static_assert(kTopoCap == 64, "one lane per slot");
   const int tid = threadIdx.x, lane = tid & 63;
   const int wv = __builtin_amdgcn_readfirstlane(tid >> 6);
   for (int g = 1 + blockIdx.x; g <= sp.N; g += gridDim.x) {
@@ -497,36 +506,41 @@ __global__ __launch_bounds__(256) void k_slots(SimParams sp, const int32_t* __re
     const double dd2 = 2.0 * (double)(ox - oy), half2 = 2.0 * (double)(n / 2);
     const double* __restrict__ tri = cd.tri + 3 * tb;
     float rho2 = 0.f;
+    // f(r, valid): 64 barycenters (r relative to the grain's first) of the
+    // slot's elements per call, element by element; after(e): past the
+    // element's last call
+    auto over = [&](int slot, auto f, auto after) {
+      for (int e0 = 0; e0 < E; e0 += 64) {
+        const int el = e0 + lane;
+        unsigned long long m = __ballot(el < E && ((s_em[el < E ? el : 0] >> slot) & 1ull));
+        for (; m; m &= m - 1) {
+          const int e = e0 + (int)__builtin_ctzll(m);
+          const int r0 = s_ef[e], r1 = s_ef[e + 1];
+          for (int r = r0; r < r1; r += 64) f(r + lane, r + lane < r1);
+          after(e);
+        }
+      }
+    };
+    auto load = [&](int r, double& qx, double& qy, double& qz) {
+      const double* q = tri + 3 * (int64_t)r;
+      qx = q[0] - ox;
+      qy = q[1] - oy;
+      qz = q[2] - oz;
+      return qx * qx + qy * qy + qz * qz + dd2 * (qx - qy);
+    };
+    // 1e-3: far above the rounding of either side (and of the FP64 search)
+    auto keep = [&](const double* q0, double R, double qx, double qy, double qz) {
+      return (R - q0[3]) - half2 * (fabs(qx - q0[0]) + fabs(qy - q0[1]) + fabs(qz - q0[2])) <= 1e-3;
+    };
     for (int slot = wv; slot < kTopoCap; slot += 4) {
-      int2* out = cd.slist + (int64_t)g * kTopoCap + slot;
       if (s_key[slot] == -1 || s_key[slot] == g) {
-        if (lane == 0) *out = make_int2(0, 0);
+        if (lane == 0) s_groups[slot] = 0;
         continue;
       }
-      // f(e, r, valid): barycenter r (relative to the grain's first) of
-      // element e, 64 per call; after(e): past the element's last call
-      auto over = [&](auto f, auto after) {
-        for (int e0 = 0; e0 < E; e0 += 64) {
-          const int el = e0 + lane;
-          unsigned long long m = __ballot(el < E && ((s_em[el < E ? el : 0] >> slot) & 1ull));
-          for (; m; m &= m - 1) {
-            const int e = e0 + (int)__builtin_ctzll(m);
-            const int r0 = s_ef[e], r1 = s_ef[e + 1];
-            for (int r = r0; r < r1; r += 64) f(e, r + lane, r + lane < r1);
-            after(e);
-          }
-        }
-      };
-      auto load = [&](int r, double& qx, double& qy, double& qz) {
-        const double* q = tri + 3 * (int64_t)r;
-        qx = q[0] - ox;
-        qy = q[1] - oy;
-        qz = q[2] - oz;
-        return qx * qx + qy * qy + qz * qz + dd2 * (qx - qy);
-      };
       double R0 = 1e300, x0 = 0, y0 = 0, z0 = 0;
       over(
-          [&](int, int r, bool valid) {
+          slot,
+          [&](int r, bool valid) {
             if (!valid) return;
             double qx, qy, qz;
             const double R = load(r, qx, qy, qz);
@@ -542,38 +556,54 @@ __global__ __launch_bounds__(256) void k_slots(SimParams sp, const int32_t* __re
 #pragma unroll
       for (int o = 1; o < 64; o <<= 1) best = fmin(best, __shfl_xor(best, o));
       const int src = (int)__builtin_ctzll(__ballot(R0 == best));
-      R0 = best;
-      x0 = __shfl(x0, src);
-      y0 = __shfl(y0, src);
-      z0 = __shfl(z0, src);
-      // 1e-3: far above the rounding of either side (and of the FP64 search)
-      auto keep = [&](double R, double qx, double qy, double qz) {
-        return (R - R0) - half2 * (fabs(qx - x0) + fabs(qy - y0) + fabs(qz - z0)) <= 1e-3;
-      };
+      const double q0[4] = {__shfl(x0, src), __shfl(y0, src), __shfl(z0, src), best};
+      if (lane < 4) s_q0[slot][lane] = lane == 0 ? q0[0] : lane == 1 ? q0[1] : lane == 2 ? q0[2] : q0[3];
       int groups = 0, cnt = 0;
       over(
-          [&](int, int r, bool valid) {
+          slot,
+          [&](int r, bool valid) {
             double qx, qy, qz;
             const double R = load(valid ? r : 0, qx, qy, qz);
-            cnt += __popcll(__ballot(valid && keep(R, qx, qy, qz)));
+            cnt += __popcll(__ballot(valid && keep(q0, R, qx, qy, qz)));
           },
           [&](int) {
             groups += (cnt + kChunk - 1) / kChunk;
             cnt = 0;
           });
-      int first = 0;
-      if (lane == 0 && groups > 0) first = atomicAdd(cd.row_n, groups);
-      first = __builtin_amdgcn_readfirstlane(first);
-      if (first > cd.row_groups - groups) {
-        if (lane == 0) *out = make_int2(0, -1);  // no room: the slot is searched without a list
-        continue;
+      if (lane == 0) s_groups[slot] = groups;
+    }
+    __syncthreads();
+    // the grain's groups are reserved with one add (2.5 ms per step at 20000
+    // grains; one per slot, 2.8e5 on one counter: 3.7)
+    if (wv == 0) {
+      const int groups = s_groups[lane];
+      int incl = groups;
+#pragma unroll
+      for (int d = 1; d < 64; d <<= 1) {
+        const int u = __shfl_up(incl, d, 64);
+        if (lane >= d) incl += u;
       }
-      int cur = first;
+      const int all = __builtin_amdgcn_readlane(incl, 63);
+      int first = 0;
+      if (lane == 0 && all > 0) first = atomicAdd(cd.row_n, all);
+      first = __builtin_amdgcn_readfirstlane(first) + incl - groups;
+      // no room: the slot is searched without a list
+      const int2 sl = groups == 0 ? make_int2(0, 0)
+                      : first > cd.row_groups - groups ? make_int2(0, -1) : make_int2(first, groups);
+      cd.slist[(int64_t)g * kTopoCap + lane] = sl;
+      s_first[lane] = sl.y > 0 ? sl.x : -1;
+    }
+    __syncthreads();
+    for (int slot = wv; slot < kTopoCap; slot += 4) {
+      int cur = s_first[slot], cnt = 0;
+      if (cur < 0) continue;
+      const double q0[4] = {s_q0[slot][0], s_q0[slot][1], s_q0[slot][2], s_q0[slot][3]};
       over(
-          [&](int, int r, bool valid) {
+          slot,
+          [&](int r, bool valid) {
             double qx, qy, qz;
             const double R = load(valid ? r : 0, qx, qy, qz);
-            const bool k = valid && keep(R, qx, qy, qz);
+            const bool k = valid && keep(q0, R, qx, qy, qz);
             const unsigned long long m = __ballot(k);
             if (k) {
               const int pos = cnt + __popcll(m & ((1ull << lane) - 1ull));
@@ -595,7 +625,6 @@ __global__ __launch_bounds__(256) void k_slots(SimParams sp, const int32_t* __re
             cur += ng;
             cnt = 0;
           });
-      if (lane == 0) *out = make_int2(first, groups);
     }
 #pragma unroll
     for (int o = 1; o < 64; o <<= 1) rho2 = fmaxf(rho2, __shfl_xor(rho2, o));
