@@ -435,9 +435,9 @@ __global__ __launch_bounds__(256) void k_tri_scatter(TopoDev topo, CorrDev cd) {
 // 14 groups of 8 rows on average (75 before k_slots leaves out the ones that
 // cannot be nearest).  The FP64 search over boxed chunks that this replaced took
 // 146 ms per step (and its chunk boxes 3.4); k_correct took 24.5 in this form,
-// with tiles dealt to the XCDs and fewer workgroups (below) 18.6, with runs of 8
-// layers instead of 4 for n <= 32 (fuller searches) 17.9, and with a grain's lists
-// next to each other 17.5; k_slots takes 2.5.
+// with fewer workgroups and runs of 8 layers instead of 4 for n <= 32 (fuller
+// searches) 17.9, and with single tiles in turn over the XCDs (below) 16.0;
+// k_slots takes 2.5.
 // Queueing and output are about 9 ms of it, the rest is the minima (vector)
 // behind the products, at four wavefronts per SIMD (128 registers; three: 28.9
 // against 24.5).  128 voxels per search read each row once for four products; 64
@@ -672,16 +672,6 @@ struct Near {
 };
 #pragma float_control(pop)
 
-// The XCD's l-th tile: tiles go to the XCDs in chunks of two or so grains (the
-// grain's rows and tables come from one L2), chunk by chunk in turn.  A search's
-// length depends on how far its grain is from the plane x = y, so ranges of
-// grains that lie together are uneven work (20000 grains: 24.6 ms per step with
-// one range per XCD, 21.4 dealt).
-constexpr int kDealt = 64;
-__device__ inline int dealt_tile(int l) {
-  return (l / kDealt * kXcds + (int)(blockIdx.x % kXcds)) * kDealt + l % kDealt;
-}
-
 // One workgroup per (grain, run of ZT z-layers) of the output box: its band
 // voxels are queued in LDS grouped by the slot of their IDLocal id in the
 // grain's hull-id table, and a wavefront takes up to kTake of one slot at a
@@ -703,7 +693,13 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4))) void k
   const T* __restrict__ ain = (const T*)din.arena;
   T* __restrict__ aout = (T*)dout.arena;
   const double delta = sp.delta;
-  for (int l = blockIdx.x / kXcds, tile; (tile = dealt_tile(l)) < total; l += gridDim.x / kXcds) {
+  // Tile by tile over the XCDs: a search's length depends on how far its grain is
+  // from the plane x = y, so tiles that lie together are uneven work.  20000
+  // grains, correction per step: one range per XCD 24.6 ms, chunks of 64 tiles in
+  // turn 21.4, and, with 64 workgroups per CU, 256: 18.2, 64: 17.5, 16: 16.9,
+  // 4: 16.4, single ones 16.0 (a grain's rows then come from every L2, but the
+  // last-level cache holds them).
+  for (int tile = blockIdx.x; tile < total; tile += gridDim.x) {
     int g, kl;
     plan_tile(P, cls, kQLayers, tile, g, kl);
     if (kl % ZT) continue;  // the plan's tiles are single layers; the first of a run takes the run

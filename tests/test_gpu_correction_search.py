@@ -1,5 +1,5 @@
 """The correction's nearest-element search against the oracle, FP64 bit for bit, where its layout can go
-wrong: every box-size class (runs of 4, 2 and 1 layers, sides that are no multiple of the run), grains
+wrong: every box-size class (runs of 8, 4, 2 and 1 layers, sides that are no multiple of the run), grains
 whose few barycenters fill partial groups, and a row pool too small for every slot's list (those slots
 are searched without one).
 
