@@ -359,9 +359,9 @@ int conv_mode(const gg_ctx* c) {
 // launch leaves much of the chip idle, and a launch of a class without grains
 // still takes about 4 us, so the classes run side by side; the correction has
 // long tails at any size.  Per step, classes one after another and as branches:
-// 77 grains of side 45 to 80, FP64: 1.95 and 1.72 ms; 343 grains, FP64,
-// correction: 2.52 and 2.24; 512 grains, FP64: 0.98 and 0.88; 4000 grains, FP32,
-// correction: 14.8 and 14.1.  Elsewhere only the list build, the n <= 32
+// 77 grains of side 45 to 80, FP64: 1.88 and 1.60 ms; 343 grains, FP64,
+// correction: 1.69 and 1.46; 512 grains, FP64: 0.92 and 0.81; 4000 grains, FP32,
+// correction: 8.11 and 7.58; 20000: 41.4 and 40.8.  Elsewhere only the list build, the n <= 32
 // comparison and the hull leave the main stream: more voxels fill the GPU launch
 // by launch (8000 grains, FP32: 8.11 and 8.24), and where a step is short the
 // forks cost more than they overlap, on the device and, eager, on the host (27
