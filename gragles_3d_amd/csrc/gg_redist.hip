@@ -282,9 +282,10 @@ __global__ __launch_bounds__(64) void k_redist_z(SimParams sp, PlanDev P, int cl
   }
 }
 
-// h with the sign of v, 0 for 0: (T)sgnv(v) * h without the conversion.
-__device__ inline float sgnh(float v, float h) { return v == 0.f ? 0.f : __builtin_copysignf(h, v); }
-__device__ inline double sgnh(double v, double h) { return v == 0.0 ? 0.0 : __builtin_copysign(h, v); }
+// h with the sign of v, 0 for 0 and for NaN: (T)sgnv(v) * h without the
+// conversion (one ordered compare; v == 0 would give a NaN a sign).
+__device__ inline float sgnh(float v, float h) { return __builtin_islessgreater(v, 0.f) ? __builtin_copysignf(h, v) : 0.f; }
+__device__ inline double sgnh(double v, double h) { return __builtin_islessgreater(v, 0.0) ? __builtin_copysign(h, v) : 0.0; }
 
 // One step of a register-resident sweep from cur to nxt (the loop bodies
 // above): `ip` = interpolate (in values a, b at the two points), `act` = the
