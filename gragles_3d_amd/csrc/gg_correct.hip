@@ -42,6 +42,7 @@
 // positions (used only for the merge test) are the hull's barycenter sums
 // (fixed point, summed in any order to the same value) over their count.
 #include "gg_internal.h"
+#include "gg_runs.h"
 
 namespace gg {
 namespace {
@@ -50,9 +51,9 @@ constexpr int kEW = 256;                           // threads of an element-buil
 constexpr int kRec = kJuncCap + kJuncCap / 2;      // lists + high-order junctions made by merging
 constexpr int kTopoCapBitsC = 6;
 static_assert((1 << kTopoCapBitsC) == kTopoCap, "grain topology table size");
-// workgroups per CU of a correction launch: 16 times what is resident, for
+// most workgroups per CU of a correction launch: 16 times what is resident, for
 // balance; each costs its start (correction per step at 20000 grains with 24:
-// 18.7, 64: 18.6, 512: 21.4, one per layer: 23.9 ms)
+// 16.1, 32: 16.3, 64: 15.8, 128: 15.9, 256: 16.1 ms)
 constexpr int kCorrGridPerCU = 64;
 
 enum { kClsGB = 0, kClsTL = 1, kClsQJ = 2, kClsHJ = 3 };
@@ -436,8 +437,8 @@ __global__ __launch_bounds__(256) void k_tri_scatter(TopoDev topo, CorrDev cd) {
 // cannot be nearest).  The FP64 search over boxed chunks that this replaced took
 // 146 ms per step (and its chunk boxes 3.4); k_correct took 24.5 in this form,
 // with fewer workgroups and runs of 8 layers instead of 4 for n <= 32 (fuller
-// searches) 17.9, and with single tiles in turn over the XCDs (below) 16.0;
-// k_slots takes 2.5.
+// searches) 17.9, and with runs in turn over the XCDs (below) 15.8; k_slots
+// takes 2.5.
 // Queueing and output are about 9 ms of it, the rest is the minima (vector)
 // behind the products, at four wavefronts per SIMD (128 registers; three: 28.9
 // against 24.5).  128 voxels per search read each row once for four products; 64
@@ -688,21 +689,37 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4))) void k
   __shared__ uint16_t s_q[ZT * NMAX * NMAX];  // band voxels grouped by slot
   __shared__ int s_cnt[kBuckets];
   __shared__ int s_next;
-  const int total = P.totals[kQLayers * kClasses + cls];
+  __shared__ int s_at[4][2];
   const int tid = threadIdx.x, lane = tid & 63;
   const T* __restrict__ ain = (const T*)din.arena;
   T* __restrict__ aout = (T*)dout.arena;
   const double delta = sp.delta;
-  // Tile by tile over the XCDs: a search's length depends on how far its grain is
-  // from the plane x = y, so tiles that lie together are uneven work.  20000
-  // grains, correction per step: one range per XCD 24.6 ms, chunks of 64 tiles in
-  // turn 21.4, and, with 64 workgroups per CU, 256: 18.2, 64: 17.5, 16: 16.9,
-  // 4: 16.4, single ones 16.0 (a grain's rows then come from every L2, but the
-  // last-level cache holds them).
-  for (int tile = blockIdx.x; tile < total; tile += gridDim.x) {
-    int g, kl;
-    plan_tile(P, cls, kQLayers, tile, g, kl);
-    if (kl % ZT) continue;  // the plan's tiles are single layers; the first of a run takes the run
+  // The plan's tiles are single layers: a window of ZT consecutive ones holds the
+  // first layers of the runs a workgroup takes next (about one), found with one
+  // load.  A search's length depends on how far its grain is from the plane x =
+  // y, so windows that lie together are uneven work; they go to the XCDs in turn
+  // (run_window; a grain's rows then come from every L2, but the last-level
+  // cache holds them).  Correction per step, 20000 grains: one range per XCD
+  // 24.6 ms, chunks of 64 tiles in turn 17.5, of 4 16.4, windows 15.8.  Single
+  // tiles in turn, each first layer taking its run, gave 16.1 there, but boxes of
+  // equal sides have their first layers on one or two XCDs: 3375 of side 24,
+  // 7.2 ms against 1.9; 1331 of 32, 10.4 and 2.7; 1000 of 48 and more, 13.9 and
+  // 7.8.
+  int* at = s_at[tid >> 6];  // the loop's state during a run, off the registers
+  for (int u = blockIdx.x, starts = 0;;) {
+    const uint32_t* __restrict__ map = P.tmap[kQLayers] + P.tile_base[kQLayers * kClasses + cls];
+    while (starts == 0) {
+      const int total = P.totals[kQLayers * kClasses + cls];
+      if (u >= ((total + ZT - 1) / ZT + kXcds - 1) / kXcds * kXcds) return;
+      const int t = run_window(u) * ZT + lane;
+      const bool mine = lane < ZT && t < total;
+      starts = (int)__ballot(mine && (map[mine ? t : 0] & 0xFFu) % ZT == 0);
+      u += gridDim.x;
+    }
+    const uint32_t tile = map[run_window(u - gridDim.x) * ZT + __builtin_ctz(starts)];
+    const int g = (int)(tile >> 8), kl = (int)(tile & 0xFFu);
+    at[0] = u;
+    at[1] = starts & (starts - 1);
     const int32_t* b = dout.bounds + 6 * g;
     const int x0 = b[0], y0 = b[1], z0 = b[2], n = b[3] - b[0], nn2 = n * n;
     const int nv = min(ZT, n - kl) * nn2;  // voxels of the run
@@ -1004,7 +1021,9 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4))) void k
         }
       }
     }
-    __syncthreads();  // the queue is refilled for the next tile
+    __syncthreads();  // the queue is refilled for the next run
+    u = __builtin_amdgcn_readfirstlane(at[0]);
+    starts = __builtin_amdgcn_readfirstlane(at[1]);
   }
 }
 
@@ -1012,16 +1031,16 @@ template <class T>
 void correct_classes(const Launch& L, const SimParams& sp, const PlanDev& P, const int32_t* state, const DescDev& din,
                      const DescDev& dout, const IdlDev& il, const TopoDev& topo, const CorrDev& cd, int c0, int c1) {
   if (c0 <= 0 && 0 < c1)
-    hipLaunchKernelGGL((k_correct<T, 32, 8>), dim3(tile_grid(L, kCorrGridPerCU, 0, sp.N, layers_of(0))), dim3(256), 0, L.stream, sp, P, 0,
+    hipLaunchKernelGGL((k_correct<T, 32, 8>), dim3(tile_grid(L, kCorrGridPerCU, 0, sp.N, layers_of(0) / 8 + 1)), dim3(256), 0, L.stream, sp, P, 0,
                      state, din, dout, il, topo, cd);
   if (c0 <= 1 && 1 < c1)
-    hipLaunchKernelGGL((k_correct<T, 48, 4>), dim3(tile_grid(L, kCorrGridPerCU, 1, sp.N, layers_of(1))), dim3(256), 0, L.stream, sp, P, 1,
+    hipLaunchKernelGGL((k_correct<T, 48, 4>), dim3(tile_grid(L, kCorrGridPerCU, 1, sp.N, layers_of(1) / 4 + 1)), dim3(256), 0, L.stream, sp, P, 1,
                      state, din, dout, il, topo, cd);
   if (c0 <= 2 && 2 < c1)
-    hipLaunchKernelGGL((k_correct<T, 64, 2>), dim3(tile_grid(L, kCorrGridPerCU, 2, sp.N, layers_of(2))), dim3(256), 0, L.stream, sp, P, 2,
+    hipLaunchKernelGGL((k_correct<T, 64, 2>), dim3(tile_grid(L, kCorrGridPerCU, 2, sp.N, layers_of(2) / 2 + 1)), dim3(256), 0, L.stream, sp, P, 2,
                      state, din, dout, il, topo, cd);
   if (c0 <= 3 && 3 < c1)
-    hipLaunchKernelGGL((k_correct<T, 96, 1>), dim3(tile_grid(L, kCorrGridPerCU, 3, sp.N, layers_of(3))), dim3(256), 0, L.stream, sp, P, 3,
+    hipLaunchKernelGGL((k_correct<T, 96, 1>), dim3(tile_grid(L, kCorrGridPerCU, 3, sp.N, layers_of(3) / 1 + 1)), dim3(256), 0, L.stream, sp, P, 3,
                      state, din, dout, il, topo, cd);
 }
 
