@@ -1556,6 +1556,19 @@ int gg_download_elements(gg_ctx* c, int32_t id, int32_t* cls, int32_t* nnb, int3
   return GG_OK;
 }
 
+int gg_get_correction_lists(gg_ctx* c, int64_t* asked, int64_t* room) {
+  if (!c) return GG_ERR_ARG;
+  if (!c->cd.ready) return fail(c, GG_ERR_STATE, "the convolution correction was never enabled");
+  int rc = gg_synchronize(c);
+  if (rc) return rc;
+  int32_t ready = 0, n = 0;
+  HIPCHK(c, hipMemcpy(&ready, c->cd.ready, 4, hipMemcpyDeviceToHost));
+  if (ready) HIPCHK(c, hipMemcpy(&n, c->cd.row_n, 4, hipMemcpyDeviceToHost));
+  if (asked) *asked = n;
+  if (room) *room = c->cd.row_groups;
+  return GG_OK;
+}
+
 // The grain's topology table, sorted by first appearance.
 static int topo_ids(gg_ctx* c, int32_t id, std::vector<std::pair<int32_t, int32_t>>& out) {
   out.clear();

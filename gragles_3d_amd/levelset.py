@@ -106,6 +106,7 @@ SIGNATURES = {
     "gg_download_hull_neighbours": (ctypes.c_int, [_vp, _i32, _i32p, _i32, _i32p]),
     "gg_get_hull_junction_counts": (ctypes.c_int, [_vp, _i32p]),
     "gg_get_faces": (ctypes.c_int, [_vp, _i32p, _i32p, _f64p, ctypes.c_int64, _i64p]),
+    "gg_get_correction_lists": (ctypes.c_int, [_vp, _i64p, _i64p]),
     "gg_get_element_counts": (ctypes.c_int, [_vp, _i32p]),
     "gg_download_all_lists": (ctypes.c_int, [_vp, _i32, _i32p, _i32p, ctypes.c_int64, ctypes.POINTER(ctypes.c_int64)]),
     "gg_get_new_bounds": (ctypes.c_int, [_vp, _i32p]),
@@ -479,6 +480,13 @@ class LevelSetContext:
         m = n.value
         return {"cls": cls[:m], "nb": [tuple(nb8[8 * e:8 * e + min(8, nnb[e])].tolist()) for e in range(m)],
                 "nbary": nbary[:m], "pos": pos[:3 * m].reshape(m, 3), "energy": en[:m], "mobility": mo[:m]}
+
+    def correction_lists(self):
+        """(asked, room): groups of 8 barycenters in the correction's lists after the last hull, and what
+        their pool holds; lists past it are left out (the same results, more slowly)."""
+        asked, room = ctypes.c_int64(0), ctypes.c_int64(0)
+        self._chk(lib().gg_get_correction_lists(self.h, ctypes.byref(asked), ctypes.byref(room)))
+        return asked.value, room.value
 
     def voxel_container(self):
         """saveNetworkAsVoxelContainer's id container (Container_size_*.raw

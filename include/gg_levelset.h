@@ -227,6 +227,13 @@ int gg_set_physics(gg_ctx* ctx, const gg_physics* phys, const double* quat, cons
 int gg_download_elements(gg_ctx* ctx, int32_t id, int32_t* cls, int32_t* nnb, int32_t* nb8, int32_t* nbary,
                          double* pos, double* energy, double* mobility, int32_t cap, int32_t* n);
 
+/* The correction's barycenter lists after the last hull, in groups of 8: how
+ * many all grains asked for, and how many there is room for.  A list past the
+ * room is left out and its voxels are searched over every barycenter of the
+ * elements they border: the same result, several times slower; a larger
+ * arena_voxels gives more room.  Either pointer may be NULL. */
+int gg_get_correction_lists(gg_ctx* ctx, int64_t* asked, int64_t* room);
+
 /* countGrains: synchronises and returns the number of grains not deleted. */
 int gg_count_grains(gg_ctx* ctx, int32_t* count);
 
