@@ -1467,25 +1467,24 @@ int gg_set_physics(gg_ctx* c, const gg_physics* ph, const double* quat, const do
   if (!d.ready) {
     const size_t ne = n1 * kElemCap;
     const int64_t cap = c->arena_cap / 8 + 65536;  // triangles of one hull pass (about 3 per surface voxel)
-    const int64_t tcap = cap + cap / 4;
-    // groups of the slot lists: the lists leave most barycenters out (k_slots),
-    // and a slot that finds no room is searched without a list
-    const size_t rgroups = (size_t)std::min<int64_t>(tcap / kChunk, INT32_MAX / 2);
+    // groups of the slot lists, in the memory of the records (12 to 77 % of it in
+    // arenas of the default size); a slot that finds no room is searched without
+    // a list
+    const size_t rgroups = (size_t)std::min<int64_t>(cap / kChunk - kRowSpare, INT32_MAX / 2);
     if ((rc = dalloc(c, &c->topo.jord, n1 * kJuncCap)) || (rc = dalloc(c, &c->topo.raw, (size_t)cap)) ||
         (rc = dalloc(c, &c->topo.raw_n, 1)) || (rc = dalloc(c, &d.ready, 1)) || (rc = dalloc(c, &d.ecount, n1)) ||
         (rc = dalloc(c, &d.eclass, 4 * n1)) || (rc = dalloc(c, &d.epos, 3 * ne)) || (rc = dalloc(c, &d.emask, ne)) ||
         (rc = dalloc(c, &d.energy, ne)) || (rc = dalloc(c, &d.mobility, ne)) ||
         (rc = dalloc(c, &d.efirst, n1 * (kElemCap + 1))) || (rc = dalloc(c, &d.ecur, ne)) ||
         (rc = dalloc(c, &d.slot_elem, n1 * kJuncCap)) || (rc = dalloc(c, &d.tbase, n1)) ||
-        (rc = dalloc(c, &d.tri, 3 * (size_t)tcap)) || (rc = dalloc(c, &d.slist, n1 * kTopoCap)) ||
+        (rc = dalloc(c, &d.tri, 3 * (size_t)cap)) || (rc = dalloc(c, &d.slist, n1 * kTopoCap)) ||
         (rc = dalloc(c, &d.sbox, n1)) || (rc = dalloc(c, &d.org, n1)) ||
-        (rc = dalloc(c, &d.rows, kRowLen * kChunk * (rgroups + kRowSpare))) ||
         (rc = dalloc(c, &d.rsrc, kChunk * rgroups)) || (rc = dalloc(c, &d.tags, rgroups + kRowSpare)) ||
-        (rc = dalloc(c, &d.row_n, 1)) ||
-        (rc = dalloc(c, &d.tri_n, 1)) || (rc = dalloc(c, (double**)&d.see, n1)))
+        (rc = dalloc(c, &d.row_n, 1)) || (rc = dalloc(c, &d.tri_n, 1)) || (rc = dalloc(c, (double**)&d.see, n1)))
       return rc;
     c->topo.raw_cap = cap;
-    d.tri_cap = tcap;
+    d.tri_cap = cap;
+    d.rows = (uint16_t*)c->topo.raw;
     d.row_groups = (int)rgroups;
     HIPCHK(c, hipMemset(d.ecount, 0, 4 * n1));
     HIPCHK(c, hipMemset(d.slot_elem, 0xFF, 4 * n1 * kJuncCap));

@@ -81,7 +81,7 @@ struct TopoDev {
   double* jarea;               // [(N+1) * kJuncCap] summed triangle areas of each list (grid units)
   int corr;                    // also the triangle records and first appearances below
   int32_t* jord;               // [(N+1) * kJuncCap] first appearance of each list
-  TriRec* raw;                 // [raw_cap] triangle records of the last hull
+  TriRec* raw;                 // [raw_cap] triangle records of the last hull, until its elements are built (CorrDev::rows)
   unsigned long long* raw_n;   // records written (may exceed raw_cap: then the topology error bit is set)
   int64_t raw_cap;
 };
@@ -95,7 +95,8 @@ struct TopoDev {
 constexpr int kElemCap = kJuncCap;
 constexpr int kChunk = 8;          // rows of one element come in groups of kChunk
 constexpr double kFarPoint = 1e30;  // squared distance that a group's padding rows stand for
-constexpr int kRowLen = 16;        // BF16 values of a barycenter's row in the nearest-element filter
+constexpr int kRowLen = 16;        // 16-bit values of a barycenter's row in the nearest-element filter
+static_assert(sizeof(TriRec) == 2 * kRowLen, "rows take the place of records");
 constexpr int kRowSpare = 64;      // groups past the pool's end, read ahead and never used
 constexpr int kTagEnd = 0x8000;
 struct CorrDev {
@@ -125,7 +126,10 @@ struct CorrDev {
   int4* sbox;                  // [N+1] the box the lists hold for: x0, y0, z0, side
   int4* org;                   // [N+1] grid point the rows are relative to (x, y, z), and the largest distance of
                                // a listed barycenter from it (the bits of a float)
-  uint16_t* rows;              // [kRowLen * kChunk * (row_groups + kRowSpare)] rows of the filter's matrix
+  uint16_t* rows;              // [kRowLen * kChunk * (row_groups + kRowSpare)] rows of the filter's matrix, in the
+                               // memory of TopoDev::raw: a record is as long as a row, k_tri_scatter has read all
+                               // records before k_slots writes rows, and every hull that writes new records is
+                               // followed by the build of its elements and rows
   int32_t* rsrc;               // [kChunk * row_groups] the row's barycenter, relative to tbase (-1: padding)
   uint16_t* tags;              // [row_groups + kRowSpare] element of each group, kTagEnd on its last one
   int* row_n;                  // groups placed (may exceed row_groups: then slots have no list)

@@ -214,7 +214,9 @@ typedef struct gg_physics {
  * needed when energies or mobilities depend on the misorientation; see:
  * n_grains+1 doubles (see[0] for the wall), needed with stored_energy.  The
  * pair tables are computed on the host (gg_gb_pair_tables).  Drops a
- * captured step graph; enables the hull topology. */
+ * captured step graph; enables the hull topology.  The first call takes about
+ * 7.5 bytes of device memory per voxel of the distance arena and 55 KiB per
+ * grain, plus 16 bytes per pair of ids for misorientation-dependent tables. */
 int gg_set_physics(gg_ctx* ctx, const gg_physics* phys, const double* quat, const double* see);
 
 /* The interfacial elements of grain id's last hull, in the order the
