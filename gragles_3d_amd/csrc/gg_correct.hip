@@ -38,8 +38,9 @@
 //                  them over: w_energy = the element's mobility, w_mobility =
 //                  its energy (src/InterfacialElement.h:22-31, 70-72).
 //
-// FP64 arithmetic throughout, in the reference's operation order; the junction
-// positions (used only for the merge test) are the hull's barycenter sums
+// FP64 arithmetic in the reference's operation order; only which barycenters need
+// comparing in FP64 is found by a BF16-piece product with an error bound (below),
+// so every result is FP64's.  The junction positions (used only for the merge test) are the hull's barycenter sums
 // (fixed point, summed in any order to the same value) over their count.
 #include "gg_internal.h"
 #include "gg_runs.h"
@@ -424,13 +425,20 @@ __global__ __launch_bounds__(256) void k_tri_scatter(TopoDev topo, CorrDev cd) {
 // element.  Where the two are closer than the error bound, and only there, the
 // wavefront searches the bordering elements' barycenters in FP64 for the first
 // nearest one in projection order, so the chosen element is always the
-// reference's (about 1.5 % of the searches of 64 voxels hold such a voxel).
+// reference's.
 //
 // Bound: with rho >= |q'| over the grain's rows, the terms of W sum to at most
-// S = rho^2 + 2 rho (|D| + |p'|) in magnitude; 12 terms are added, each
-// addition rounds to at most 2^-24 S, and the pieces' remainders are 2^-26 of a
-// term, so 16 x 2^-24 S covers the error (measured on random rows and columns
-// of every box size: at most 2.2 x 2^-24 S).
+// S = rho^2 + 2 rho (|D| + |p'|) in magnitude, their pieces to 1.01 S.  Of the
+// instruction's adder nothing is assumed but that each rounding is within one
+// unit of the last place, 2^-23 of a value that the pieces' sum bounds, so
+// truncation is allowed and any order of the adds.  12 products are added: 12
+// roundings, 24 x 2^-24 of 1.01 S, and the pieces' remainders are 2^-26 of a
+// term.  kFilterEps, 32 x 2^-24, covers these and three roundings more
+// (measured on random rows and columns of every box size: at most 2.2 x 2^-24
+// S).  FP64 rounds a squared distance below 1e7 to 6e-9, so a gap also has to
+// pass kDecided: the reference's rounded comparison then agrees with the exact
+// one.  (Half this bound, enough for an adder that rounds to nearest, saves 0.2
+// of 15.9 ms per step at 20000 grains.)
 //
 // What bounds it: at 20000 grains (5.8e8 band voxels per step) the searches hold
 // 14 groups of 8 rows on average (75 before k_slots leaves out the ones that
@@ -445,9 +453,13 @@ __global__ __launch_bounds__(256) void k_tri_scatter(TopoDev topo, CorrDev cd) {
 // took 4 % longer.
 typedef __bf16 v8bf __attribute__((ext_vector_type(8)));
 typedef float v16f __attribute__((ext_vector_type(16)));
-constexpr float kFilterEps = 1.0f / 1048576.0f;  // 2^-20
-constexpr float kNone = 3e38f;                   // above every filter value
-constexpr int kManyExact = 12;  // voxels of 64 to decide from which on each lane searches for its own
+constexpr float kFilterEps = 1.0f / 524288.0f;  // 2^-19
+constexpr float kDecided = 1e-6f;               // a gap that FP64 rounding cannot turn round
+constexpr float kNone = 3e38f;                  // above every filter value
+// Voxels of 64 to decide from which on each lane searches for its own.  Correction
+// per step at 4000 grains, 20000, 343 in FP64: with 12 2.00, 15.9, 0.47 ms; 20
+// 1.94, 15.7, 0.43; 32 1.98, 15.8, 0.40; 4 2.23, 16.4, 0.60.
+constexpr int kManyExact = 24;
 constexpr int kTake = 128;  // voxels of a wavefront's search: each row is read once for four products
 
 // A barycenter as a row of the filter: -2q' (three BF16 pieces per axis) and R
@@ -932,7 +944,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4))) void k
             // a squared distance of 1e7 or more is no neighbour (the reference's
             // initial minimum): the FP64 search decides where one could be that far
             const float reach = dd + pp + rho;
-            exact = act && emin >= 0 && (me.m2 - me.m1 <= 2.0f * kFilterEps * S || reach * reach > 9.9e6f);
+            exact = act && emin >= 0 && (me.m2 - me.m1 <= 2.0f * kFilterEps * S + kDecided || reach * reach > 9.9e6f);
           }
           // f(e, r0, r1): the slot's elements, barycenters [r0, r1)
           auto over_elements = [&](auto f) {
