@@ -27,7 +27,9 @@ static std::mutex g_scratch_mu[kScratchDevices];          // one call at a time 
 static int32_t* g_scratch_ptr[kScratchDevices] = {};      // device address of scratch, per GPU
 
 constexpr int kSides = 3;  // with the main stream, the four hardware queues a process gets
-// bytes of a distance arena (twice the first boxes') between which every size class gets a branch
+// voxels of a distance arena of the default size
+constexpr int64_t arena_for(int64_t box_voxels) { return 2 * box_voxels + 65536; }
+// bytes of such an arena between which every size class gets a branch
 constexpr int64_t kBranchMin = 100000000, kBranchMax = 400000000;
 
 struct gg_ctx {
@@ -61,6 +63,7 @@ struct gg_ctx {
   int sel = 0;  // D[sel] is the input role
   void* arena[2] = {nullptr, nullptr};
   int64_t arena_cap = 0;
+  int64_t set_voxels = 0;  // voxels of the boxes last set
   // IDLocal
   IdlDev IL[2]{};
   int il_cur = 0;  // IL[il_cur] holds the latest IDLocal content
@@ -358,21 +361,26 @@ int conv_mode(const gg_ctx* c) {
 // A branch per size class where that pays: below a full GPU's worth of voxels a
 // launch leaves much of the chip idle, and a launch of a class without grains
 // still takes about 4 us, so the classes run side by side; the correction has
-// long tails at any size.  Per step, classes one after another and as branches:
-// 77 grains of side 45 to 80, FP64: 1.88 and 1.60 ms; 343 grains, FP64,
-// correction: 1.69 and 1.46; 512 grains, FP64: 0.92 and 0.81; 4000 grains, FP32,
-// correction: 8.11 and 7.58; 20000: 41.4 and 40.8.  Elsewhere only the list build, the n <= 32
-// comparison and the hull leave the main stream: more voxels fill the GPU launch
-// by launch (8000 grains, FP32: 8.11 and 8.24), and where a step is short the
-// forks cost more than they overlap, on the device and, eager, on the host (27
-// grains: 0.35 and 0.38; 2000 grains, FP32, eager: 4 % slower).
+// long tails at any size.  The rule goes by the voxels of the boxes that were
+// set (whatever arena_voxels is) and not by whether a step is captured, so it
+// holds where neither form loses.  ms per step, classes one after another and as
+// branches, captured unless said.  Inside, FP64: 343 grains 0.77 and 0.68, 77 of
+// side 45 to 80 1.84 and 1.58, 512 0.92 and 0.82 (eager 0.95 and 0.91), 1000 of
+// 16 points 1.50 and 1.41; with the correction: 343 in FP64 1.66 and 1.45 (eager
+// 1.66 and 1.55), 2000 in FP64 8.47 and 7.93, 1000 in FP32 2.38 and 2.08, 4000
+// 8.45 and 7.86, 20000 44.0 and 43.0.  Outside, the forks cost an eager step
+// more than they overlap: FP64 64 grains 0.28 and 0.33, 216 0.58 and 0.63; FP32
+// 216 0.38 and 0.49, 2000 2.01 and 2.11, 8000 7.17 and 7.40; captured FP32 steps
+// lose up to 512 grains (216: 0.35 and 0.38).  What the line leaves: captured
+// FP64 steps of fewer voxels (27 grains 0.33 and 0.26, 216 0.56 and 0.48) and FP64
+// above it (1000 of 20 points 2.63 and 2.44, 2000 4.80 and 4.65, 8000 17.3 and 17.1).
 int sides_of(const gg_ctx* c) {
-  const int64_t bytes = c->arena_cap * (int64_t)c->esz;
+  const int64_t bytes = arena_for(c->set_voxels) * (int64_t)c->esz;
   const bool many = bytes >= kBranchMin && (c->corr_on || (!c->fp32 && bytes <= kBranchMax));
   return many ? kSides : 1;
 }
 // The side streams that sides_of() asks for: each takes about 0.3 ms to make,
-// so they are made where what it depends on (the arena, the correction) is set.
+// so they are made where what it depends on (the boxes, the correction) is set.
 int make_sides(gg_ctx* c) {
   for (int i = 0; i < sides_of(c); ++i) {
     if (!c->side[i]) HIPCHK(c, hipStreamCreateWithFlags(&c->side[i], hipStreamNonBlocking));
@@ -569,7 +577,7 @@ void stage_redistancing(gg_ctx* c) {
 // redistancing: the hull reads the input role and IDLocal, the redistancing
 // reads the input role and writes the output role, and the existence, volume
 // and area finish after both.  The post-redistancing resize follows the
-// deletion marks, as in the stage-by-stage order. 
+// deletion marks, as in the stage-by-stage order.
 void stage_level_set_and_redistancing(gg_ctx* c) {
   if (c->timing) {
     stage_level_set(c);
@@ -780,15 +788,20 @@ int gg_set_boxes(gg_ctx* c, const int32_t* bounds, const uint8_t* exists) {
     total += (int64_t)n * n * n;
   }
   if (c->arena[0] == nullptr) {
-    c->arena_cap = c->p.arena_voxels > 0 ? c->p.arena_voxels : 2 * total + 65536;
+    c->arena_cap = c->p.arena_voxels > 0 ? c->p.arena_voxels : arena_for(total);
     c->spec_cap = c->arena_cap;
-    const int rc = make_sides(c);
-    if (rc) return rc;
   } else if (total > c->arena_cap) {
     // the arenas, the spectral scratch and the work lists keep the size of the
     // first call
     return fail(c, GG_ERR_CAPACITY, "boxes exceed the arena sized by the first gg_set_boxes");
   }
+  const int sides = sides_of(c);
+  c->set_voxels = total;
+  if (sides_of(c) != sides) {  // a captured step has the branches of the boxes before
+    HIPCHK(c, hipStreamSynchronize(c->stream));
+    drop_graph(c);
+  }
+  if (const int rc = make_sides(c)) return rc;
   for (int r = 0; r < 2; ++r) {
     if (c->arena[r] == nullptr) {
       int rc;

@@ -1,7 +1,7 @@
-"""The correction where every size class is a branch of its own (distance arenas from 100 MB, here asked for with
-arena_voxels), on a case with boxes of all four size classes: the convolution and correction of the classes run
-beside each other and beside the list build and the IDLocal resize.  FP64, eager and captured steps, against the
-oracle bit for bit; FP32 against the same run on one side stream, bit for bit.  And what the FP32 correction does
+"""The correction where every size class is a branch of its own (boxes of 50 MB and more: 1.6e7 voxels here), on a
+case with boxes of all four size classes: the convolution and correction of the classes run beside each other and
+beside the list build and the IDLocal resize.  FP64, eager and captured steps, against the oracle bit for bit; FP32
+against the same run on one stream (as stage timing has it), bit for bit.  And what the FP32 correction does
 to boxes above 32, from a second context without it: every band voxel moves by the weights of one of the elements
 that border its id.
 
@@ -17,7 +17,7 @@ from parity import compare_all
 
 pytestmark = pytest.mark.gpu
 
-N, PPG, BORDER, SEED = 27, 26, 3, 1
+N, PPG, BORDER, SEED = 216, 26, 3, 1
 
 
 @pytest.fixture(scope="module")
@@ -25,6 +25,7 @@ def case():
     c = PC.voronoi_case(N, PPG, BORDER, SEED)
     side = np.max(c[2][1:, 3:] - c[2][1:, :3], axis=1)
     assert all(((side > a) & (side <= b)).any() for a, b in ((0, 32), (32, 48), (48, 64), (64, 96))), side
+    assert np.sum(side.astype(np.int64) ** 3) * 4 > 50_000_000  # FP32 too
     return c
 
 
@@ -33,9 +34,9 @@ def _physics():
                 quat=PC.low_angle_orientations(N, 11), see=G.lognormal_energies(N, 3, median=0.1, sigma=1.0))
 
 
-def _context(case, precision, arena=0, correction=True):
+def _context(case, precision, correction=True):
     p, idf, bounds, exists, offs, ids = case
-    ctx = G.LevelSetContext(p, precision=precision, arena_voxels=arena)
+    ctx = G.LevelSetContext(p, precision=precision)
     ctx.set_boxes(bounds, exists)
     ctx.init_distance(idf)
     ctx.set_neighbour_lists(offs, ids)
@@ -46,7 +47,7 @@ def _context(case, precision, arena=0, correction=True):
 
 def test_branches_fp64_equal_oracle(case):
     print("correction branches: FP64, n=%d ppg=%d border=%d seed=%d" % (N, PPG, BORDER, SEED), flush=True)
-    ctx = _context(case, G.FP64_PLAIN, arena=13_000_000)
+    ctx = _context(case, G.FP64_PLAIN)
     orc = PC.oracle_sim(O, case)
     orc.set_physics(tl_drag=1e6, **_physics())
     for step in range(2):
@@ -62,12 +63,36 @@ def test_branches_fp64_equal_oracle(case):
     orc.close()
 
 
+def test_branches_follow_the_boxes_set(case):
+    """One context: first few of the grains (no branches), captured steps, then all of them (branches)."""
+    print("correction branches: boxes set twice, n=%d ppg=%d" % (N, PPG), flush=True)
+    p, idf, bounds, exists, offs, ids = case
+    ctx = G.LevelSetContext(p, precision=G.FP64_PLAIN, arena_voxels=2 * int(np.sum(
+        np.max(bounds[1:, 3:] - bounds[1:, :3], axis=1).astype(np.int64) ** 3)))
+    few = exists.copy()
+    few[40:] = 0
+    for some in (few, exists):
+        o, i = G.initial_neighbour_lists(p, bounds, some)
+        ctx.set_boxes(bounds, some)
+        ctx.set_physics(triple_line_drag=1e6, **_physics())
+        orc = PC.oracle_sim(O, (p, idf, bounds, some, o, i))
+        orc.set_physics(tl_drag=1e6, **_physics())
+        ctx.init_distance(idf)
+        ctx.set_neighbour_lists(o, i)
+        ctx.timestep(3, use_graph=True)
+        orc.timestep(3)
+        compare_all(ctx, orc, "%d grains" % int(some.sum()))
+        orc.close()
+    ctx.close()
+
+
 @pytest.mark.parametrize("graph", [False, True])
 def test_branches_fp32_equal_one_stream(case, graph):
     print("correction branches: FP32, %s, n=%d ppg=%d" % ("captured" if graph else "eager", N, PPG), flush=True)
     out = []
-    for arena in (26_000_000, 0):
-        ctx = _context(case, G.FP32_BATCHED, arena=arena)
+    for one_stream in (False, True):
+        ctx = _context(case, G.FP32_BATCHED)
+        ctx.enable_stage_timing(one_stream)
         ctx.timestep(6, use_graph=graph)
         state = ctx.stats()[0]
         out.append((state, [ctx.phi(g, 1) for g in np.nonzero(state == G.ALIVE)[0]]))
