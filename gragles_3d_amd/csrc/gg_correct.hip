@@ -360,8 +360,10 @@ __global__ void k_clear_counters(unsigned long long* tri_n, int* row_n) {
 }
 
 // Every triangle record of the last hull into its element's barycenter range.
-// The records of one hull tile are consecutive in the pool and in cell order;
-// a wavefront reserves one run per (grain, element) among its 64 records.
+// A grain's records are consecutive in the pool, one wavefront of its hull
+// workgroup after the other (those a full cell queue forced out lie apart), so a
+// wavefront's 64 records here name few elements: it reserves one run per (grain,
+// element) among them.
 __global__ __launch_bounds__(256) void k_tri_scatter(TopoDev topo, CorrDev cd) {
   unsigned long long n = *topo.raw_n;
   if (n > (unsigned long long)topo.raw_cap) n = (unsigned long long)topo.raw_cap;
@@ -447,10 +449,11 @@ __global__ __launch_bounds__(256) void k_tri_scatter(TopoDev topo, CorrDev cd) {
 // with fewer workgroups and runs of 8 layers instead of 4 for n <= 32 (fuller
 // searches) 17.9, and with runs in turn over the XCDs (below) 15.8; k_slots
 // takes 2.5.
-// Queueing and output are about 9 ms of it, the rest is the minima (vector)
-// behind the products, at four wavefronts per SIMD (128 registers; three: 28.9
-// against 24.5).  128 voxels per search read each row once for four products; 64
-// took 4 % longer.
+// Of the 15.8 ms, queueing and output are 8.1, the products and the minima behind
+// them (vector) 6.2, the FP64 decisions 1.5 (4000 grains: 0.6, 0.8, 0.5 of 1.9;
+// 343 in FP64: 0.08, 0.18, 0.15 of 0.42), at four wavefronts per SIMD (128
+// registers; three, when it took 24.5: 28.9).  128 voxels per search read each
+// row once for four products; 64 took 4 % longer.
 typedef __bf16 v8bf __attribute__((ext_vector_type(8)));
 typedef float v16f __attribute__((ext_vector_type(16)));
 constexpr float kFilterEps = 1.0f / 524288.0f;  // 2^-19
