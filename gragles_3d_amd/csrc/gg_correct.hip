@@ -435,12 +435,11 @@ __global__ __launch_bounds__(256) void k_tri_scatter(TopoDev topo, CorrDev cd) {
 // unit of the last place, 2^-23 of a value that the pieces' sum bounds, so
 // truncation is allowed and any order of the adds.  12 products are added: 12
 // roundings, 24 x 2^-24 of 1.01 S, and the pieces' remainders are 2^-26 of a
-// term.  kFilterEps, 32 x 2^-24, covers these and three roundings more
-// (measured on random rows and columns of every box size: at most 2.2 x 2^-24
-// S).  FP64 rounds a squared distance below 1e7 to 6e-9, so a gap also has to
+// term: 24.5 x 2^-24, and kFilterEps is 26 x 2^-24 (measured on random rows and
+// columns of every box size: at most 2.2 x 2^-24 S).  FP64 rounds a squared distance below 1e7 to 6e-9, so a gap also has to
 // pass kDecided: the reference's rounded comparison then agrees with the exact
-// one.  (Half this bound, enough for an adder that rounds to nearest, saves 0.2
-// of 15.9 ms per step at 20000 grains.)
+// one.  (Correction per step with 16, enough for an adder that rounds to nearest,
+// 25 and 32 x 2^-24: 1000 grains 1.07, 1.09, 1.12 ms; 20000 15.5, 15.7, 15.8.)
 //
 // What bounds it: at 20000 grains (5.8e8 band voxels per step) the searches hold
 // 14 groups of 8 rows on average (75 before k_slots leaves out the ones that
@@ -456,9 +455,9 @@ __global__ __launch_bounds__(256) void k_tri_scatter(TopoDev topo, CorrDev cd) {
 // row once for four products; 64 took 4 % longer.
 typedef __bf16 v8bf __attribute__((ext_vector_type(8)));
 typedef float v16f __attribute__((ext_vector_type(16)));
-constexpr float kFilterEps = 1.0f / 524288.0f;  // 2^-19
-constexpr float kDecided = 1e-6f;               // a gap that FP64 rounding cannot turn round
-constexpr float kNone = 3e38f;                  // above every filter value
+constexpr float kFilterEps = 26.0f / 16777216.0f;
+constexpr float kDecided = 1e-6f;                 // a gap that FP64 rounding cannot turn round
+constexpr float kNone = 3e38f;                    // above every filter value
 // Voxels of 64 to decide from which on each lane searches for its own.  Correction
 // per step at 4000 grains, 20000, 343 in FP64: with 12 2.00, 15.9, 0.47 ms; 20
 // 1.94, 15.7, 0.43; 32 1.98, 15.8, 0.40; 4 2.23, 16.4, 0.60.

@@ -17,8 +17,8 @@ SRC = os.path.join(os.path.dirname(os.path.dirname(os.path.abspath(__file__))), 
 
 
 def filter_eps():
-    m = re.search(r"constexpr float kFilterEps = 1\.0f / (\d+)\.0f;", open(SRC).read())
-    return 1.0 / int(m.group(1))
+    m = re.search(r"constexpr float kFilterEps = (\d+)\.0f / (\d+)\.0f;", open(SRC).read())
+    return int(m.group(1)) / int(m.group(2))
 
 
 def bf16(x):
