@@ -441,7 +441,7 @@ void enqueue_convolution(gg_ctx* c, const Launch& L, int c0, int c1) {
 // and writes distance values only.  The work list needs the plan and the input
 // bounds, which the convolution leaves alone.
 void stage_convolution(gg_ctx* c, bool lists = false) {
-  if (c->timing) {
+  if (c->timing || (!lists && sides_of(c) == 1)) {  // nothing to run beside it
     enqueue_convolution(c, launch_of(c), 0, kClasses);
     SegTimer t(c, kSegIdl);
     launch_idl_resize(launch_of(c), c->sp, c->d_state, dout(c), c->IL[c->il_cur ^ 1]);
@@ -502,10 +502,11 @@ void stage_comparison(gg_ctx* c) {
   c->il_cur ^= 1;
 }
 
-// Runs launch(L, c0, c1) over the size classes, outside stage timing as branches.
+// Runs launch(L, c0, c1) over the size classes, outside stage timing as branches
+// where every class has its own.
 template <class F>
 void over_classes(gg_ctx* c, F launch) {
-  if (c->timing) {
+  if (c->timing || sides_of(c) == 1) {
     launch(launch_of(c), 0, kClasses);
     return;
   }
