@@ -446,9 +446,9 @@ __global__ __launch_bounds__(256) void k_tri_scatter(TopoDev topo, CorrDev cd) {
 // cannot be nearest).  The FP64 search over boxed chunks that this replaced took
 // 146 ms per step (and its chunk boxes 3.4); k_correct took 24.5 in this form,
 // with fewer workgroups and runs of 8 layers instead of 4 for n <= 32 (fuller
-// searches) 17.9, and with runs in turn over the XCDs (below) 15.8; k_slots
-// takes 2.5.
-// Of the 15.8 ms, queueing and output are 8.1, the products and the minima behind
+// searches) 17.9, and with the runs dealt to the XCDs (below) 15.5; k_slots takes
+// 2.5.
+// Of the 15.5 ms (15.8 when this was taken), queueing and output are 8.1, the products and the minima behind
 // them (vector) 6.2, the FP64 decisions 1.5 (4000 grains: 0.6, 0.8, 0.5 of 1.9;
 // 343 in FP64: 0.08, 0.18, 0.15 of 0.42), at four wavefronts per SIMD (128
 // registers; three, when it took 24.5: 28.9).  128 voxels per search read each
@@ -696,6 +696,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4))) void k
                                                  DescDev din, DescDev dout, IdlDev il, TopoDev topo, CorrDev cd) {
   if (*cd.ready == 0) return;  // no hull yet (run_sim's first step)
   constexpr int kBuckets = kTopoCap + 1;  // a slot, or the last bucket: an id the hull does not name
+  constexpr int kRow = run_chunk(NMAX, ZT);
   static_assert(kTopoCap == 64, "one lane per slot");
   constexpr int VPT = (ZT * NMAX * NMAX + 255) / 256;  // voxels per thread
   static_assert(ZT * NMAX * NMAX <= 0xFFFF, "cell indexes are 16-bit");
@@ -711,26 +712,32 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4))) void k
   // The plan's tiles are single layers: a window of ZT consecutive ones holds the
   // first layers of the runs a workgroup takes next (about one), found with one
   // load.  A search's length depends on how far its grain is from the plane x =
-  // y, so windows that lie together are uneven work; they go to the XCDs in turn
-  // (run_window; a grain's rows then come from every L2, but the last-level
-  // cache holds them).  Correction per step, 20000 grains: one range per XCD
-  // 24.6 ms, chunks of 64 tiles in turn 17.5, of 4 16.4, windows 15.8.  Single
-  // tiles in turn, each first layer taking its run, gave 16.1 there, but boxes of
-  // equal sides have their first layers on one or two XCDs: 3375 of side 24,
-  // 7.2 ms against 1.9; 1331 of 32, 10.4 and 2.7; 1000 of 48 and more, 13.9 and
-  // 7.8.
+  // y, so one range of tiles per XCD is uneven work; about a box's windows at a
+  // time go to each XCD in turn (run_window), so a grain's runs still share an
+  // L2.  Correction per step at 20000 grains, 4000, 1000: one range per XCD 24.6
+  // ms at 20000; single windows in turn 15.7, 1.92, 1.10; a box's at a time 15.5,
+  // 1.85, 1.08.  Single tiles in turn, each first layer taking its run, gave 16.3,
+  // 1.97, 1.05, but boxes of equal sides have their first layers on one or two
+  // XCDs: 3375 cubes of side 24, 7.2 ms against 1.8; 1331 of 32, 10.4 and 2.5; 1000 of
+  // 48 and more, 14.0 and 7.0.
   int* at = s_at[tid >> 6];  // the loop's state during a run, off the registers
-  for (int u = blockIdx.x, starts = 0;;) {
-    const uint32_t* __restrict__ map = P.tmap[kQLayers] + P.tile_base[kQLayers * kClasses + cls];
-    while (starts == 0) {
-      const int total = P.totals[kQLayers * kClasses + cls];
-      if (u >= ((total + ZT - 1) / ZT + kXcds - 1) / kXcds * kXcds) return;
-      const int t = run_window(u) * ZT + lane;
-      const bool mine = lane < ZT && t < total;
-      starts = (int)__ballot(mine && (map[mine ? t : 0] & 0xFFu) % ZT == 0);
-      u += gridDim.x;
+  for (int u = blockIdx.x, starts = 0;; u += starts ? 0 : gridDim.x) {
+    const int total = P.totals[kQLayers * kClasses + cls];
+    const int windows = ((total + ZT - 1) / ZT + kXcds * kRow - 1) / (kXcds * kRow) * (kXcds * kRow);
+    // a grid with room for it takes the windows twice, the second time for what
+    // begins in them after their first run: two runs of a window one after the
+    // other are twice the latency of a small launch
+    const bool twice = 2 * windows <= (int)gridDim.x, again = twice && u >= windows;
+    if (u >= (twice ? 2 * windows : windows)) return;
+    const int t = run_window(again ? u - windows : u, kRow) * ZT + lane;
+    const bool mine = lane < ZT && t < total;
+    const uint32_t v = P.tmap[kQLayers][P.tile_base[kQLayers * kClasses + cls] + (mine ? t : 0)];
+    if (starts == 0) {
+      starts = (int)__ballot(mine && (v & 0xFFu) % ZT == 0);
+      if (twice) starts = again ? starts & (starts - 1) : starts & -starts;
+      if (starts == 0) continue;
     }
-    const uint32_t tile = map[run_window(u - gridDim.x) * ZT + __builtin_ctz(starts)];
+    const uint32_t tile = (uint32_t)__builtin_amdgcn_readlane((int)v, __builtin_ctz(starts));
     const int g = (int)(tile >> 8), kl = (int)(tile & 0xFFu);
     at[0] = u;
     at[1] = starts & (starts - 1);
@@ -1064,16 +1071,16 @@ template <class T>
 void correct_classes(const Launch& L, const SimParams& sp, const PlanDev& P, const int32_t* state, const DescDev& din,
                      const DescDev& dout, const IdlDev& il, const TopoDev& topo, const CorrDev& cd, int c0, int c1) {
   if (c0 <= 0 && 0 < c1)
-    hipLaunchKernelGGL((k_correct<T, 32, 8>), dim3(tile_grid(L, kCorrGridPerCU, 0, sp.N, layers_of(0) / 8 + 1)), dim3(256), 0, L.stream, sp, P, 0,
+    hipLaunchKernelGGL((k_correct<T, 32, 8>), dim3(tile_grid(L, kCorrGridPerCU, 0, sp.N, 2 * (layers_of(0) / 8 + 1))), dim3(256), 0, L.stream, sp, P, 0,
                      state, din, dout, il, topo, cd);
   if (c0 <= 1 && 1 < c1)
-    hipLaunchKernelGGL((k_correct<T, 48, 4>), dim3(tile_grid(L, kCorrGridPerCU, 1, sp.N, layers_of(1) / 4 + 1)), dim3(256), 0, L.stream, sp, P, 1,
+    hipLaunchKernelGGL((k_correct<T, 48, 4>), dim3(tile_grid(L, kCorrGridPerCU, 1, sp.N, 2 * (layers_of(1) / 4 + 1))), dim3(256), 0, L.stream, sp, P, 1,
                      state, din, dout, il, topo, cd);
   if (c0 <= 2 && 2 < c1)
-    hipLaunchKernelGGL((k_correct<T, 64, 2>), dim3(tile_grid(L, kCorrGridPerCU, 2, sp.N, layers_of(2) / 2 + 1)), dim3(256), 0, L.stream, sp, P, 2,
+    hipLaunchKernelGGL((k_correct<T, 64, 2>), dim3(tile_grid(L, kCorrGridPerCU, 2, sp.N, 2 * (layers_of(2) / 2 + 1))), dim3(256), 0, L.stream, sp, P, 2,
                      state, din, dout, il, topo, cd);
   if (c0 <= 3 && 3 < c1)
-    hipLaunchKernelGGL((k_correct<T, 96, 1>), dim3(tile_grid(L, kCorrGridPerCU, 3, sp.N, layers_of(3) / 1 + 1)), dim3(256), 0, L.stream, sp, P, 3,
+    hipLaunchKernelGGL((k_correct<T, 96, 1>), dim3(tile_grid(L, kCorrGridPerCU, 3, sp.N, layers_of(3) + 1)), dim3(256), 0, L.stream, sp, P, 3,
                      state, din, dout, il, topo, cd);
 }
 

@@ -10,22 +10,33 @@ import pytest
 
 CSRC = os.path.join(os.path.dirname(os.path.dirname(os.path.abspath(__file__))), "gragles_3d_amd", "csrc")
 XCDS = 8
+NMAX = {8: 32, 4: 48, 2: 64, 1: 96}  # largest side of the class with runs of so many layers
 
 
 @pytest.fixture(scope="module")
 def run_window(tmp_path_factory):
     d = tmp_path_factory.mktemp("runs")
     src = d / "runs.cpp"
-    src.write_text('#include "gg_runs.h"\nextern "C" int w(int u) { return gg::run_window(u); }\n')
+    src.write_text('#include "gg_runs.h"\nextern "C" int w(int u, int chunk) { return gg::run_window(u, chunk); }\n'
+                   'extern "C" int chunk(int nmax, int zt) { return gg::run_chunk(nmax, zt); }\n')
     so = str(d / "runs.so")
     subprocess.run(["g++", "-std=c++17", "-shared", "-fPIC", "-I", CSRC, str(src), "-o", so], check=True)
-    f = ctypes.CDLL(so).w
-    return np.vectorize(lambda u: f(int(u)))
+    lib = ctypes.CDLL(so)
+
+    def order(n, zt):
+        """The windows of positions 0 .. m - 1, m the next multiple of the rule's period from n on."""
+        chunk = lib.chunk(NMAX[zt], zt)
+        m = -(-n // (XCDS * chunk)) * XCDS * chunk
+        return np.array([lib.w(u, chunk) for u in range(m)])
+
+    return order
 
 
-@pytest.mark.parametrize("n", [8, 64, 4096, 80000])
-def test_every_window_once(run_window, n):
-    assert np.array_equal(np.sort(run_window(np.arange(n))), np.arange(n))
+@pytest.mark.parametrize("zt", [8, 4, 2, 1])
+@pytest.mark.parametrize("n", [1, 8, 64, 4096, 80000])
+def test_every_window_once(run_window, n, zt):
+    w = run_window(n, zt)
+    assert w.size >= n and np.array_equal(np.sort(w), np.arange(w.size))
 
 
 @pytest.mark.parametrize("side,zt", [(9, 8), (17, 8), (24, 8), (28, 8), (31, 8), (32, 8), (33, 4), (36, 4), (40, 4),
@@ -37,9 +48,8 @@ def test_equal_sides_spread_evenly(run_window, side, zt):
     cost = 0.2 + np.sqrt(np.maximum(0.0, 1.0 - z * z))  # of a layer
     run_cost = np.array([cost[k:k + zt].sum() for k in range(0, side, zt)])
     at = np.nonzero(layer % zt == 0)[0]  # first tiles of the runs, in plan order
-    windows = -(-layer.size // zt)
-    positions = -(-windows // XCDS) * XCDS
-    xcd = np.empty(positions, dtype=np.int64)
-    xcd[run_window(np.arange(positions))] = np.arange(positions) % XCDS
+    w = run_window(-(-layer.size // zt), zt)
+    xcd = np.empty(w.size, dtype=np.int64)
+    xcd[w] = np.arange(w.size) % XCDS
     work = np.bincount(xcd[at // zt], weights=np.tile(run_cost, grains), minlength=XCDS)
     assert work.max() <= 1.05 * work.mean(), work / work.mean()
